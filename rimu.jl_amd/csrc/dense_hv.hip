@@ -4,9 +4,9 @@
 // Row r of a vector is the address of colex rank r: the N one-bits of the address at
 // positions p_0 < p_1 < ... give rank = sum_j C(p_j, j+1), and colex order equals
 // ascending numeric order of the bit strings.  A hop moves one boson by one bit, so the
-// rank of a neighbour follows from the row's own rank with one binomial: a one moving
-// from bit q to q+1 (the j-th one) adds C(q, j); from p to p-1 it subtracts C(p-1, j).
-// Hops across the periodic boundary rotate the string and are ranked from scratch.
+// rank of a neighbour follows from the row's own rank with one binomial, which depends only on
+// the bond and on the bosons below it (a small table in LDS).  Hops across the periodic
+// boundary rotate the string; their ranks are laid out with the basis.
 //
 // Vectors are row-major [dim][R] (R right-hand sides, one per Hamiltonian): a neighbour's
 // R amplitudes are one contiguous 8R-byte load.  Every reduction is a fixed-order tree,
@@ -31,7 +31,7 @@ constexpr int BINOM_N = 65;      // C(n, k) for 0 <= n, k <= 64
 
 struct DenseParams {
     double a[MAXR], b[MAXR], u[MAXR], t[MAXR];
-    int M, B;
+    int M, N;
 };
 
 // Colex rank from scratch.
@@ -47,133 +47,228 @@ __device__ inline int64_t colex_rank(uint64_t bits, const int64_t* __restrict__ 
     return r;
 }
 
-// The hops of row r (address `bits`, rank `rank`) in the order of hopnextneighbour's
-// `chosen` (bosefs.jl:297-345): for the s-th occupied mode, right hop then left hop.
-// f(neighbour_rank, sqrt_prod) is called for each; the matrix element is -t*sqrt_prod.
-template <class F>
-__device__ inline void for_each_hop(uint64_t bits, int64_t rank, int M, int B,
-                                    const int64_t* __restrict__ binom, F&& f) {
-    const uint64_t maskB = low_mask(B);
-    uint64_t st = run_starts(bits);
-    while (st) {
-        const int p = __builtin_ctzll(st);
-        st &= st - 1;
-        const int n = ones_from(bits, p);
-        const int m = p - popc64(bits & low_mask(p)) + 1;
-        // right hop
-        if (m == M) {
-            const uint64_t nb = ((bits << 1) | 1ull) & maskB;
-            f(colex_rank(nb, binom), sqrt((double)((int64_t)n * (ones_from(bits, 0) + 1))));
-        } else {
-            const int q = p + n - 1;  // the last one of the run moves to q+1
-            const int j = popc64(bits & low_mask(q));
-            f(rank + binom[q * BINOM_N + j], sqrt((double)((int64_t)n * (ones_from(bits, q + 2) + 1))));
-        }
-        // left hop
-        if (m == 1) {
-            const uint64_t nb = (bits >> 1) | (1ull << (B - 1));
-            const int hz = 63 - clz64(~bits & maskB);
-            f(colex_rank(nb, binom), sqrt((double)((int64_t)n * ((B - 1 - hz) + 1))));
-        } else {
-            const int j = popc64(bits & low_mask(p));  // the first one of the run moves to p-1
-            int nprev = 0;
-            if (p >= 2) {
-                const uint64_t z = ~bits & low_mask(p - 1);
-                nprev = z ? (p - 2 - (63 - clz64(z))) : (p - 1);
-            }
-            f(rank - binom[(p - 1) * BINOM_N + j], sqrt((double)((int64_t)n * (nprev + 1))));
-        }
-    }
+// Tables of one (M, N), built on the host and copied to LDS by every workgroup of a product:
+//   delta[i * (N + 2) + s] = C(s + i - 2, s - 1): the rank change of a hop from mode i to mode
+//     i + 1 (1 <= i < M) when modes 1 .. i hold s bosons before it (0 for s = 0); the hop back
+//     from mode i + 1 when they hold s - 1 changes the rank by the same amount down;
+//   root[x] = sqrt(x), x <= (N + 1)^2 / 4 >= n (n' + 1), the hop amplitudes.
+struct HopTables {
+    const uint32_t* delta;
+    const double* root;
+    int n_delta, n_root;
+};
+
+__device__ inline void stage_hop_tables(const HopTables& t, double* s_root, uint32_t* s_delta) {
+    for (int j = threadIdx.x; j < t.n_root; j += DT) s_root[j] = t.root[j];
+    for (int j = threadIdx.x; j < t.n_delta; j += DT) s_delta[j] = t.delta[j];
+    __syncthreads();
 }
 
-// w = (a + b H) v, one thread per row.
-template <int R>
-__global__ __launch_bounds__(DT) void dense_apply_kernel(const uint64_t* __restrict__ basis, int64_t D,
-                                                         DenseParams p, const int64_t* __restrict__ binom,
-                                                         const double* __restrict__ v,
-                                                         double* __restrict__ w) {
+// Rank of the neighbour across the periodic boundary: rot[r].x after a hop from mode M to
+// mode 1 (the string rotates up), rot[r].y after one from mode 1 to mode M; r where that mode
+// is empty.  Every bit moves, so these are ranked once, when the basis is laid out.
+__global__ __launch_bounds__(DT) void dense_rotations_kernel(const uint64_t* __restrict__ basis, int64_t D, int B,
+                                                             const int64_t* __restrict__ binom,
+                                                             uint2* __restrict__ rot) {
     const int64_t r = (int64_t)blockIdx.x * DT + threadIdx.x;
     if (r >= D) return;
     const uint64_t bits = basis[r];
-    const double dr = (double)bose_hubbard_interaction(bits) / 2;
-    double acc[R];
+    const uint64_t top = 1ull << (B - 1);
+    uint2 o = {(uint32_t)r, (uint32_t)r};
+    if (bits & top) o.x = (uint32_t)colex_rank(((bits << 1) | 1ull) & low_mask(B), binom);
+    if (bits & 1ull) o.y = (uint32_t)colex_rank((bits >> 1) | top, binom);
+    rot[r] = o;
+}
+
+// Workgroup -> tile of rows.  Workgroups go to the eight XCDs in turn; giving each XCD a
+// contiguous eighth of the rows keeps the near neighbours of its rows in its own L2.
+__device__ inline int64_t dense_tile(int64_t b, int64_t n) {
+    const int64_t per = n >> 3;
+    return b < per * 8 ? (b & 7) * per + (b >> 3) : b;
+}
+
+// K v at row r (K: the hopping with unit amplitude, elements -sqrt(n (n' + 1))): acc[i] =
+// sum over hops of -sqrt * v[neighbour][i]; returns sum n(n - 1) / 2 of the address.
+// One pass over the M - 1 bonds and the boundary, both directions of a bond from the same
+// occupations, the same instructions in every lane: a hop that the address does not have loads
+// the row itself and adds zero.  Bound by instruction issue: per bond two table reads, two
+// gathers of 8R bytes and 2R fused multiply-adds.  (Walking each lane's own occupied modes
+// with popcounts, clz and an f64 sqrt per hop took 106 us per product at dimension 1,352,078,
+// R = 4; see the figures at dense_apply_kernel.)
+template <int R>
+__device__ inline int hop_sum(uint64_t bits, int64_t r, int M, int row_len, uint2 rot,
+                              const double* s_root, const uint32_t* s_delta,
+                              const double* __restrict__ v, double (&acc)[R]) {
 #pragma unroll
     for (int i = 0; i < R; ++i) acc[i] = 0.0;
-    for_each_hop(bits, r, p.M, p.B, binom, [&](int64_t k, double sp) {
-        const double* vk = v + k * R;
+    auto add = [&](bool has, int64_t k, int x) {
+        const double* vk = v + (has ? k : r) * R;
+        const double amp = -s_root[has ? x : 0];
 #pragma unroll
-        for (int i = 0; i < R; ++i) acc[i] += -sp * vk[i];
-    });
+        for (int i = 0; i < R; ++i) {
+            const double y = vk[i];
+            acc[i] = fma(amp, has ? y : 0.0, acc[i]);
+        }
+    };
+    uint64_t x = bits;
+    const int n1 = __builtin_ctzll(~x);  // B < 64 or a full lowest mode: ~x has a bit (see below)
+    x = shr(x, n1 + 1);
+    int nc = n1, s = n1;
+    int pairs = n1 * (n1 - 1) / 2;
+    const uint32_t* dl = s_delta + row_len;  // mode 1
+#pragma unroll 2
+    for (int m = 1; m < M; ++m, dl += row_len) {
+        const int nn = ctz64(~x);
+        x = shr(x, nn + 1);
+        add(nc > 0, r + dl[s], nc * (nn + 1));
+        add(nn > 0, r - (int64_t)dl[s + 1], nn * (nc + 1));
+        s += nn;
+        nc = nn;
+        pairs += nn * (nn - 1) / 2;
+    }
+    add(nc > 0, rot.x, nc * (n1 + 1));
+    add(n1 > 0, rot.y, n1 * (nc + 1));
+    return pairs;
+}
+
+// Sum over the workgroup, the same in every run: a shuffle tree per wavefront, then the
+// wavefronts in order (two barriers; result in thread 0).
+template <int N>
+__device__ inline void dense_block_sums(double (&v)[N], double (*s)[DT / WAVE]) {
+    const int lane = threadIdx.x & (WAVE - 1), wid = threadIdx.x / WAVE;
 #pragma unroll
-    for (int i = 0; i < R; ++i)
-        w[r * R + i] = (p.a[i] + p.b[i] * (p.u[i] * dr)) * v[r * R + i] + p.b[i] * (p.t[i] * acc[i]);
+    for (int j = 0; j < N; ++j) {
+#pragma unroll
+        for (int off = WAVE / 2; off > 0; off >>= 1) v[j] += __shfl_xor(v[j], off, WAVE);
+        if (lane == 0) s[j][wid] = v[j];
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            double t = s[j][0];
+            for (int w = 1; w < DT / WAVE; ++w) t += s[j][w];
+            v[j] = t;
+        }
+    }
+    __syncthreads();
+}
+
+// w = (a + b H) v, one thread per row.  DOT: also per-block partials[i][block] of <v|w>.
+template <int R, bool DOT>
+__global__ __launch_bounds__(DT) void dense_apply_kernel(const uint64_t* __restrict__ basis,
+                                                         const uint2* __restrict__ rot, int64_t D,
+                                                         DenseParams p, HopTables t,
+                                                         const double* __restrict__ v,
+                                                         double* __restrict__ w, double* __restrict__ partials) {
+    extern __shared__ double s_tab[];
+    uint32_t* s_delta = (uint32_t*)(s_tab + t.n_root);
+    stage_hop_tables(t, s_tab, s_delta);
+    const int64_t tile = dense_tile(blockIdx.x, gridDim.x);
+    const int64_t r = tile * DT + threadIdx.x;
+    double dt[R];
+#pragma unroll
+    for (int i = 0; i < R; ++i) dt[i] = 0.0;
+    if (r < D) {
+        double acc[R];
+        const double dr = (double)hop_sum<R>(basis[r], r, p.M, p.N + 2, rot[r], s_tab, s_delta, v, acc);
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+            const double vr = v[r * R + i];
+            const double x = (p.a[i] + p.b[i] * (p.u[i] * dr)) * vr + p.b[i] * (p.t[i] * acc[i]);
+            w[r * R + i] = x;
+            dt[i] = vr * x;
+        }
+    }
+    if constexpr (DOT) {
+        __shared__ double s_sum[R][DT / WAVE];
+        dense_block_sums<R>(dt, s_sum);
+        if (threadIdx.x == 0)
+#pragma unroll
+            for (int i = 0; i < R; ++i) partials[(int64_t)i * gridDim.x + tile] = dt[i];
+    }
 }
 
 // Pullback: vbar = (a + b H) ybar; per-block partial sums of b <ybar|D|v> and b <ybar|K|v>
-// written to partials[blockIdx][2R].  K is real symmetric, so <ybar|K|v> = sum_r v_r (K ybar)_r
+// written to partials[2R][blocks].  K is real symmetric, so <ybar|K|v> = sum_r v_r (K ybar)_r
 // and only ybar is gathered at the neighbours.
 template <int R>
-__global__ __launch_bounds__(DT) void dense_pullback_kernel(const uint64_t* __restrict__ basis, int64_t D,
-                                                            DenseParams p, const int64_t* __restrict__ binom,
+__global__ __launch_bounds__(DT) void dense_pullback_kernel(const uint64_t* __restrict__ basis,
+                                                            const uint2* __restrict__ rot, int64_t D,
+                                                            DenseParams p, HopTables t,
                                                             const double* __restrict__ v,
                                                             const double* __restrict__ ybar,
                                                             double* __restrict__ vbar,
                                                             double* __restrict__ partials) {
-    const int64_t r = (int64_t)blockIdx.x * DT + threadIdx.x;
-    double pu[R], pt[R];
+    extern __shared__ double s_tab[];
+    __shared__ double s_sum[2 * R][DT / WAVE];
+    uint32_t* s_delta = (uint32_t*)(s_tab + t.n_root);
+    stage_hop_tables(t, s_tab, s_delta);
+    const int64_t tile = dense_tile(blockIdx.x, gridDim.x);
+    const int64_t r = tile * DT + threadIdx.x;
+    double ps[2 * R];
 #pragma unroll
-    for (int i = 0; i < R; ++i) { pu[i] = 0.0; pt[i] = 0.0; }
+    for (int i = 0; i < 2 * R; ++i) ps[i] = 0.0;
     if (r < D) {
-        const uint64_t bits = basis[r];
-        const double dr = (double)bose_hubbard_interaction(bits) / 2;
         double ky[R];
-#pragma unroll
-        for (int i = 0; i < R; ++i) ky[i] = 0.0;
-        for_each_hop(bits, r, p.M, p.B, binom, [&](int64_t k, double sp) {
-            const double* yk = ybar + k * R;
-#pragma unroll
-            for (int i = 0; i < R; ++i) ky[i] += -sp * yk[i];
-        });
+        const double dr = (double)hop_sum<R>(basis[r], r, p.M, p.N + 2, rot[r], s_tab, s_delta, ybar, ky);
 #pragma unroll
         for (int i = 0; i < R; ++i) {
             const double yr = ybar[r * R + i];
             const double vr = v[r * R + i];
             vbar[r * R + i] = (p.a[i] + p.b[i] * (p.u[i] * dr)) * yr + p.b[i] * (p.t[i] * ky[i]);
-            pu[i] = p.b[i] * (yr * (dr * vr));
-            pt[i] = p.b[i] * (vr * ky[i]);
+            ps[i] = p.b[i] * (yr * (dr * vr));
+            ps[R + i] = p.b[i] * (vr * ky[i]);
         }
     }
+    dense_block_sums<2 * R>(ps, s_sum);
+    if (threadIdx.x == 0)
 #pragma unroll
-    for (int i = 0; i < R; ++i) {
-        const double su = block_sum<DT>(pu[i]);
-        const double stt = block_sum<DT>(pt[i]);
-        if (threadIdx.x == 0) {
-            partials[(int64_t)blockIdx.x * 2 * R + i] = su;
-            partials[(int64_t)blockIdx.x * 2 * R + R + i] = stt;
-        }
-    }
+        for (int i = 0; i < 2 * R; ++i) partials[(int64_t)i * gridDim.x + tile] = ps[i];
 }
 
-// out[i] = sum_r x[r][i] * y[r][i] as per-block partials[blockIdx][R].
+// out[i] = sum_r x[r][i] * y[r][i] as per-block partials[R][blocks].
 template <int R>
 __global__ __launch_bounds__(DT) void dense_dot_kernel(const double* __restrict__ x, const double* __restrict__ y,
                                                        int64_t D, double* __restrict__ partials) {
+    __shared__ double s_sum[R][DT / WAVE];
     const int64_t r = (int64_t)blockIdx.x * DT + threadIdx.x;
+    double ps[R];
 #pragma unroll
-    for (int i = 0; i < R; ++i) {
-        const double s = block_sum<DT>(r < D ? x[r * R + i] * y[r * R + i] : 0.0);
-        if (threadIdx.x == 0) partials[(int64_t)blockIdx.x * R + i] = s;
-    }
+    for (int i = 0; i < R; ++i) ps[i] = r < D ? x[r * R + i] * y[r * R + i] : 0.0;
+    dense_block_sums<R>(ps, s_sum);
+    if (threadIdx.x == 0)
+#pragma unroll
+        for (int i = 0; i < R; ++i) partials[(int64_t)i * gridDim.x + blockIdx.x] = ps[i];
 }
 
-// Sum `rows` rows of width `width` in order: out[c] (+)= sum_b partials[b][c].
-__global__ __launch_bounds__(DT) void reduce_rows_kernel(const double* __restrict__ partials, int64_t rows,
-                                                         int width, double* __restrict__ out, int accumulate) {
-    const int c = blockIdx.x;
+// out[c] (+)= sum over blocks of partials[c][block], one workgroup per c; every thread's loads
+// are in flight together (with one load at a time 9.1 us at 5282 blocks).
+constexpr int RED_NT = 1024;
+__global__ __launch_bounds__(RED_NT) void reduce_rows_kernel(const double* __restrict__ partials, int64_t blocks,
+                                                             double* __restrict__ out, int accumulate) {
+    __shared__ double s[RED_NT / WAVE];
+    const double* p = partials + (int64_t)blockIdx.x * blocks;
     double acc = 0;
-    for (int64_t b = threadIdx.x; b < rows; b += DT) acc += partials[b * width + c];
-    const double s = block_sum<DT>(acc);
-    if (threadIdx.x == 0) out[c] = accumulate ? out[c] + s : s;
+    for (int64_t b0 = 0; b0 < blocks; b0 += 8 * RED_NT) {
+        double x[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int64_t b = b0 + j * RED_NT + threadIdx.x;
+            x[j] = b < blocks ? p[b] : 0.0;
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc += x[j];
+    }
+#pragma unroll
+    for (int off = WAVE / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, WAVE);
+    if ((threadIdx.x & (WAVE - 1)) == 0) s[threadIdx.x / WAVE] = acc;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double t = s[0];
+        for (int w = 1; w < RED_NT / WAVE; ++w) t += s[w];
+        out[blockIdx.x] = accumulate ? out[blockIdx.x] + t : t;
+    }
 }
 
 // lambda = 2 (Hv - E v) / <v|v>, per right-hand side (gradient of the Rayleigh quotient).
@@ -192,14 +287,16 @@ __global__ __launch_bounds__(DT) void rq_gradient_kernel(const double* __restric
 
 // One three-term Lanczos update per right-hand side: w -= alpha_j v_j + beta_j v_{j-1},
 // with alpha_j and beta_j^2 read from device memory, and the partial sums of |w|^2 of each
-// block written to partials[blockIdx][R] (reduced in order afterwards).
+// block written to partials[R][blocks] (reduced in order afterwards).
 template <int R>
 __global__ __launch_bounds__(DT) void lanczos_orth_kernel(double* __restrict__ w, const double* __restrict__ v,
                                                           const double* __restrict__ vprev,
                                                           const double* __restrict__ alpha,
                                                           const double* __restrict__ beta2, int64_t D,
                                                           double* __restrict__ partials) {
+    __shared__ double s_sum[R][DT / WAVE];
     const int64_t r = (int64_t)blockIdx.x * DT + threadIdx.x;
+    double ps[R];
 #pragma unroll
     for (int i = 0; i < R; ++i) {
         double x = 0;
@@ -207,9 +304,12 @@ __global__ __launch_bounds__(DT) void lanczos_orth_kernel(double* __restrict__ w
             x = w[r * R + i] - alpha[i] * v[r * R + i] - sqrt(beta2[i]) * vprev[r * R + i];
             w[r * R + i] = x;
         }
-        const double s = block_sum<DT>(x * x);
-        if (threadIdx.x == 0) partials[(int64_t)blockIdx.x * R + i] = s;
+        ps[i] = x * x;
     }
+    dense_block_sums<R>(ps, s_sum);
+    if (threadIdx.x == 0)
+#pragma unroll
+        for (int i = 0; i < R; ++i) partials[(int64_t)i * gridDim.x + blockIdx.x] = ps[i];
 }
 
 // out = w / sqrt(norm2) per right-hand side; a right-hand side whose norm fell to
@@ -236,7 +336,9 @@ struct rimu_dense {
     rimu_model models[MAXR];
     hipStream_t stream = nullptr;
     DevBuf<uint64_t> basis;
-    DevBuf<int64_t> binom;
+    DevBuf<uint2> rot;
+    DevBuf<uint32_t> delta;
+    DevBuf<double> root;
     DevBuf<double> x, y, z, partials, scal;
     double* h_scal = nullptr;  // pinned, 8 * MAXR
 };
@@ -252,27 +354,43 @@ DenseParams params(const rimu_dense* d, const double* a, const double* b) {
         p.t[i] = d->models[i].t;
     }
     p.M = d->M;
-    p.B = d->B;
+    p.N = d->N;
     return p;
 }
 
+HopTables tables(const rimu_dense* d) {
+    return HopTables{d->delta.p, d->root.p, d->M * (d->N + 2), (d->N + 1) * (d->N + 1) / 4 + 1};
+}
+size_t table_bytes(const HopTables& t) { return sizeof(double) * t.n_root + sizeof(uint32_t) * t.n_delta; }
+
+// w = (a + b H) v; with out also out[i] = <v_i|w_i>
 template <int R>
-int launch_apply(rimu_dense* d, const DenseParams& p, const double* v, double* w) {
-    dense_apply_kernel<R><<<ceil_div(d->D, DT), DT, 0, d->stream>>>(d->basis.p, d->D, p, d->binom.p, v, w);
+int launch_apply(rimu_dense* d, const DenseParams& p, const double* v, double* w, double* out) {
+    const HopTables t = tables(d);
+    const int64_t blocks = ceil_div(d->D, DT);
+    if (out) {
+        HIP_TRY(d->partials.alloc((size_t)blocks * R));
+        dense_apply_kernel<R, true><<<blocks, DT, table_bytes(t), d->stream>>>(d->basis.p, d->rot.p, d->D, p, t, v, w,
+                                                                               d->partials.p);
+        reduce_rows_kernel<<<R, RED_NT, 0, d->stream>>>(d->partials.p, blocks, out, 0);
+    } else {
+        dense_apply_kernel<R, false><<<blocks, DT, table_bytes(t), d->stream>>>(d->basis.p, d->rot.p, d->D, p, t, v, w,
+                                                                                nullptr);
+    }
     HIP_TRY(hipGetLastError());
     return RIMU_OK;
 }
 
-int apply(rimu_dense* d, const DenseParams& p, const double* v, double* w) {
+int apply(rimu_dense* d, const DenseParams& p, const double* v, double* w, double* out = nullptr) {
     switch (d->R) {
-        case 1: return launch_apply<1>(d, p, v, w);
-        case 2: return launch_apply<2>(d, p, v, w);
-        case 3: return launch_apply<3>(d, p, v, w);
-        case 4: return launch_apply<4>(d, p, v, w);
-        case 5: return launch_apply<5>(d, p, v, w);
-        case 6: return launch_apply<6>(d, p, v, w);
-        case 7: return launch_apply<7>(d, p, v, w);
-        default: return launch_apply<8>(d, p, v, w);
+        case 1: return launch_apply<1>(d, p, v, w, out);
+        case 2: return launch_apply<2>(d, p, v, w, out);
+        case 3: return launch_apply<3>(d, p, v, w, out);
+        case 4: return launch_apply<4>(d, p, v, w, out);
+        case 5: return launch_apply<5>(d, p, v, w, out);
+        case 6: return launch_apply<6>(d, p, v, w, out);
+        case 7: return launch_apply<7>(d, p, v, w, out);
+        default: return launch_apply<8>(d, p, v, w, out);
     }
 }
 
@@ -280,11 +398,12 @@ int apply(rimu_dense* d, const DenseParams& p, const double* v, double* w) {
 template <int R>
 int launch_pullback(rimu_dense* d, const DenseParams& p, const double* v, const double* ybar,
                     double* vbar, double* cot, int accumulate) {
+    const HopTables t = tables(d);
     const int64_t blocks = ceil_div(d->D, DT);
     HIP_TRY(d->partials.alloc((size_t)blocks * 2 * R));
-    dense_pullback_kernel<R><<<blocks, DT, 0, d->stream>>>(d->basis.p, d->D, p, d->binom.p, v, ybar,
-                                                            vbar, d->partials.p);
-    reduce_rows_kernel<<<2 * R, DT, 0, d->stream>>>(d->partials.p, blocks, 2 * R, cot, accumulate);
+    dense_pullback_kernel<R><<<blocks, DT, table_bytes(t), d->stream>>>(d->basis.p, d->rot.p, d->D, p, t, v, ybar,
+                                                                        vbar, d->partials.p);
+    reduce_rows_kernel<<<2 * R, RED_NT, 0, d->stream>>>(d->partials.p, blocks, cot, accumulate);
     HIP_TRY(hipGetLastError());
     return RIMU_OK;
 }
@@ -308,7 +427,7 @@ int launch_dot(rimu_dense* d, const double* x, const double* y, double* out) {
     const int64_t blocks = ceil_div(d->D, DT);
     HIP_TRY(d->partials.alloc((size_t)blocks * R));
     dense_dot_kernel<R><<<blocks, DT, 0, d->stream>>>(x, y, d->D, d->partials.p);
-    reduce_rows_kernel<<<R, DT, 0, d->stream>>>(d->partials.p, blocks, R, out, 0);
+    reduce_rows_kernel<<<R, RED_NT, 0, d->stream>>>(d->partials.p, blocks, out, 0);
     HIP_TRY(hipGetLastError());
     return RIMU_OK;
 }
@@ -348,7 +467,7 @@ int launch_lanczos(rimu_dense* d, double* w, const double* v, const double* vpre
     const int64_t blocks = ceil_div(d->D, DT);
     HIP_TRY(d->partials.alloc((size_t)blocks * R));
     lanczos_orth_kernel<R><<<blocks, DT, 0, d->stream>>>(w, v, vprev, alpha, beta2, d->D, d->partials.p);
-    reduce_rows_kernel<<<R, DT, 0, d->stream>>>(d->partials.p, blocks, R, norm2_out, 0);
+    reduce_rows_kernel<<<R, RED_NT, 0, d->stream>>>(d->partials.p, blocks, norm2_out, 0);
     lanczos_scale_kernel<R><<<blocks, DT, 0, d->stream>>>(w, norm2_out, floor2, d->D, vnext);
     HIP_TRY(hipGetLastError());
     return RIMU_OK;
@@ -448,13 +567,19 @@ int rimu_dense_create(const rimu_model* models, int32_t nrhs, rimu_dense** out) 
     };
     hipError_t e;
     if ((e = hipStreamCreateWithFlags(&d->stream, hipStreamNonBlocking)) != hipSuccess) return bad("stream", e);
-    // binomial table and the sorted basis (next bit pattern with the same popcount)
+    // binomial and hop tables, and the sorted basis (next bit pattern with the same popcount)
     std::vector<int64_t> binom(BINOM_N * BINOM_N, 0);
     for (int n = 0; n < BINOM_N; ++n)
         for (int k = 0; k < BINOM_N; ++k) {
             int64_t c;
             binom[n * BINOM_N + k] = binomial64(n, k, &c) ? c : INT64_MAX;
         }
+    const int row_len = d->N + 2;  // s = 0 .. N, and N + 1 for the row's last reader
+    std::vector<uint32_t> delta((size_t)d->M * row_len, 0);
+    for (int i = 1; i < d->M; ++i)
+        for (int s = 1; s <= d->N; ++s) delta[(size_t)i * row_len + s] = (uint32_t)binom[(s + i - 2) * BINOM_N + s - 1];
+    std::vector<double> root((size_t)(d->N + 1) * (d->N + 1) / 4 + 1);
+    for (size_t k = 0; k < root.size(); ++k) root[k] = std::sqrt((double)k);
     std::vector<uint64_t> keys((size_t)D);
     uint64_t x = (d->N >= 64) ? ~0ull : ((1ull << d->N) - 1);
     for (int64_t r = 0; r < D; ++r) {
@@ -463,13 +588,24 @@ int rimu_dense_create(const rimu_model* models, int32_t nrhs, rimu_dense** out) 
         x = c ? (((rr ^ x) >> 2) / c) | rr : 0;
     }
     if ((e = d->basis.alloc(D)) != hipSuccess) return bad("basis", e);
-    if ((e = d->binom.alloc(binom.size())) != hipSuccess) return bad("binomials", e);
+    DevBuf<int64_t> dbinom;
+    if ((e = dbinom.alloc(binom.size())) != hipSuccess) return bad("binomials", e);
+    if ((e = d->rot.alloc(D)) != hipSuccess) return bad("rotations", e);
+    if ((e = d->delta.alloc(delta.size())) != hipSuccess) return bad("hop table", e);
+    if ((e = d->root.alloc(root.size())) != hipSuccess) return bad("root table", e);
     if ((e = d->scal.alloc(8 * MAXR)) != hipSuccess) return bad("scalars", e);
     if ((e = hipHostMalloc((void**)&d->h_scal, 8 * MAXR * sizeof(double), hipHostMallocDefault)) != hipSuccess)
         return bad("pinned scalars", e);
     if ((e = hipMemcpy(d->basis.p, keys.data(), D * 8, hipMemcpyHostToDevice)) != hipSuccess) return bad("basis upload", e);
-    if ((e = hipMemcpy(d->binom.p, binom.data(), binom.size() * 8, hipMemcpyHostToDevice)) != hipSuccess)
+    if ((e = hipMemcpy(dbinom.p, binom.data(), binom.size() * 8, hipMemcpyHostToDevice)) != hipSuccess)
         return bad("binomial upload", e);
+    if ((e = hipMemcpy(d->delta.p, delta.data(), delta.size() * 4, hipMemcpyHostToDevice)) != hipSuccess)
+        return bad("hop table upload", e);
+    if ((e = hipMemcpy(d->root.p, root.data(), root.size() * 8, hipMemcpyHostToDevice)) != hipSuccess)
+        return bad("root table upload", e);
+    dense_rotations_kernel<<<ceil_div(D, DT), DT, 0, d->stream>>>(d->basis.p, D, d->B, dbinom.p, d->rot.p);
+    if ((e = hipGetLastError()) != hipSuccess) return bad("rotations", e);
+    if ((e = hipStreamSynchronize(d->stream)) != hipSuccess) return bad("rotations", e);
     *out = d;
     return RIMU_OK;
 }
@@ -477,7 +613,7 @@ int rimu_dense_create(const rimu_model* models, int32_t nrhs, rimu_dense** out) 
 int rimu_dense_destroy(rimu_dense* d) {
     if (!d) return RIMU_OK;
     if (d->stream) (void)hipStreamSynchronize(d->stream);
-    d->basis.release(); d->binom.release(); d->x.release(); d->y.release(); d->z.release();
+    d->basis.release(); d->rot.release(); d->delta.release(); d->root.release(); d->x.release(); d->y.release(); d->z.release();
     d->partials.release(); d->scal.release();
     if (d->h_scal) (void)hipHostFree(d->h_scal);
     if (d->stream) (void)hipStreamDestroy(d->stream);
@@ -564,9 +700,8 @@ int rimu_dense_projector(rimu_dense* d, int64_t K, double dtau, const double* sh
             std::swap(cur.p, nxt.p);
         }
         // energy: scal[0:R] = <v|v>, scal[R:2R] = <v|Hv>; HF: scal[2R:4R] = <v|D|v>, <v|K|v>
-        if (int rc = apply(d, pH, cur.p, hv.p)) return rc;
+        if (int rc = apply(d, pH, cur.p, hv.p, d->scal.p + R)) return rc;
         if (int rc = dot(d, cur.p, cur.p, d->scal.p)) return rc;
-        if (int rc = dot(d, cur.p, hv.p, d->scal.p + R)) return rc;
         {
             double one[MAXR], unit_b[MAXR];
             for (int i = 0; i < R; ++i) { one[i] = 0; unit_b[i] = 1; }
@@ -642,8 +777,7 @@ int rimu_dense_ground_state(rimu_dense* d, const double* v0, int64_t max_iters, 
         std::vector<int64_t> m_eff(R, -1);
         int64_t j = 0;
         for (; j < cap; ++j) {
-            if (int rc = apply(d, pH, v.p, w.p)) return rc;
-            if (int rc = dot(d, v.p, w.p, alpha + j * R)) return rc;
+            if (int rc = apply(d, pH, v.p, w.p, alpha + j * R)) return rc;
             if (int rc = lanczos_update(d, w.p, v.p, vprev.p, alpha + j * R, beta2 + j * R,
                                         beta2 + (j + 1) * R, vprev.p, FLOOR2)) return rc;
             std::swap(v.p, vprev.p);
