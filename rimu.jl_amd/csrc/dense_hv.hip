@@ -337,9 +337,8 @@ struct rimu_dense {
     hipStream_t stream = nullptr;
     DevBuf<uint64_t> basis;
     DevBuf<uint2> rot;
-    DevBuf<uint32_t> delta;
-    DevBuf<double> root;
-    DevBuf<double> x, y, z, partials, scal;
+    DevBuf<double> tab;  // root table, then the hop table (uint32), then the binomials (int64)
+    DevBuf<double> x, y, z, hist, partials, scal;
     double* h_scal = nullptr;  // pinned, 8 * MAXR
 };
 
@@ -359,7 +358,8 @@ DenseParams params(const rimu_dense* d, const double* a, const double* b) {
 }
 
 HopTables tables(const rimu_dense* d) {
-    return HopTables{d->delta.p, d->root.p, d->M * (d->N + 2), (d->N + 1) * (d->N + 1) / 4 + 1};
+    const int n_root = (d->N + 1) * (d->N + 1) / 4 + 1;
+    return HopTables{(const uint32_t*)(d->tab.p + n_root), d->tab.p, d->M * (d->N + 2), n_root};
 }
 size_t table_bytes(const HopTables& t) { return sizeof(double) * t.n_root + sizeof(uint32_t) * t.n_delta; }
 
@@ -575,11 +575,14 @@ int rimu_dense_create(const rimu_model* models, int32_t nrhs, rimu_dense** out) 
             binom[n * BINOM_N + k] = binomial64(n, k, &c) ? c : INT64_MAX;
         }
     const int row_len = d->N + 2;  // s = 0 .. N, and N + 1 for the row's last reader
-    std::vector<uint32_t> delta((size_t)d->M * row_len, 0);
+    const int n_root = (d->N + 1) * (d->N + 1) / 4 + 1, n_delta = d->M * row_len;
+    const int at_binom = n_root + (n_delta + 1) / 2;  // in 8-byte words
+    std::vector<double> tab((size_t)at_binom + binom.size(), 0.0);
+    uint32_t* delta = (uint32_t*)(tab.data() + n_root);
     for (int i = 1; i < d->M; ++i)
         for (int s = 1; s <= d->N; ++s) delta[(size_t)i * row_len + s] = (uint32_t)binom[(s + i - 2) * BINOM_N + s - 1];
-    std::vector<double> root((size_t)(d->N + 1) * (d->N + 1) / 4 + 1);
-    for (size_t k = 0; k < root.size(); ++k) root[k] = std::sqrt((double)k);
+    for (int k = 0; k < n_root; ++k) tab[k] = std::sqrt((double)k);
+    std::memcpy(tab.data() + at_binom, binom.data(), binom.size() * 8);
     std::vector<uint64_t> keys((size_t)D);
     uint64_t x = (d->N >= 64) ? ~0ull : ((1ull << d->N) - 1);
     for (int64_t r = 0; r < D; ++r) {
@@ -588,22 +591,16 @@ int rimu_dense_create(const rimu_model* models, int32_t nrhs, rimu_dense** out) 
         x = c ? (((rr ^ x) >> 2) / c) | rr : 0;
     }
     if ((e = d->basis.alloc(D)) != hipSuccess) return bad("basis", e);
-    DevBuf<int64_t> dbinom;
-    if ((e = dbinom.alloc(binom.size())) != hipSuccess) return bad("binomials", e);
     if ((e = d->rot.alloc(D)) != hipSuccess) return bad("rotations", e);
-    if ((e = d->delta.alloc(delta.size())) != hipSuccess) return bad("hop table", e);
-    if ((e = d->root.alloc(root.size())) != hipSuccess) return bad("root table", e);
+    if ((e = d->tab.alloc(tab.size())) != hipSuccess) return bad("tables", e);
     if ((e = d->scal.alloc(8 * MAXR)) != hipSuccess) return bad("scalars", e);
     if ((e = hipHostMalloc((void**)&d->h_scal, 8 * MAXR * sizeof(double), hipHostMallocDefault)) != hipSuccess)
         return bad("pinned scalars", e);
     if ((e = hipMemcpy(d->basis.p, keys.data(), D * 8, hipMemcpyHostToDevice)) != hipSuccess) return bad("basis upload", e);
-    if ((e = hipMemcpy(dbinom.p, binom.data(), binom.size() * 8, hipMemcpyHostToDevice)) != hipSuccess)
-        return bad("binomial upload", e);
-    if ((e = hipMemcpy(d->delta.p, delta.data(), delta.size() * 4, hipMemcpyHostToDevice)) != hipSuccess)
-        return bad("hop table upload", e);
-    if ((e = hipMemcpy(d->root.p, root.data(), root.size() * 8, hipMemcpyHostToDevice)) != hipSuccess)
-        return bad("root table upload", e);
-    dense_rotations_kernel<<<ceil_div(D, DT), DT, 0, d->stream>>>(d->basis.p, D, d->B, dbinom.p, d->rot.p);
+    if ((e = hipMemcpy(d->tab.p, tab.data(), tab.size() * 8, hipMemcpyHostToDevice)) != hipSuccess)
+        return bad("table upload", e);
+    dense_rotations_kernel<<<ceil_div(D, DT), DT, 0, d->stream>>>(d->basis.p, D, d->B,
+                                                                  (const int64_t*)(d->tab.p + at_binom), d->rot.p);
     if ((e = hipGetLastError()) != hipSuccess) return bad("rotations", e);
     if ((e = hipStreamSynchronize(d->stream)) != hipSuccess) return bad("rotations", e);
     *out = d;
@@ -613,7 +610,7 @@ int rimu_dense_create(const rimu_model* models, int32_t nrhs, rimu_dense** out) 
 int rimu_dense_destroy(rimu_dense* d) {
     if (!d) return RIMU_OK;
     if (d->stream) (void)hipStreamSynchronize(d->stream);
-    d->basis.release(); d->rot.release(); d->delta.release(); d->root.release(); d->x.release(); d->y.release(); d->z.release();
+    d->basis.release(); d->rot.release(); d->tab.release(); d->x.release(); d->y.release(); d->z.release(); d->hist.release();
     d->partials.release(); d->scal.release();
     if (d->h_scal) (void)hipHostFree(d->h_scal);
     if (d->stream) (void)hipStreamDestroy(d->stream);
@@ -681,49 +678,61 @@ int rimu_dense_projector(rimu_dense* d, int64_t K, double dtau, const double* sh
         b_h[i] = 1;
     }
     const DenseParams pT = params(d, a_t, b_t), pH = params(d, a_h, b_h);
-    DevBuf<double> ck, seg, cur, nxt, hv, lam, lam2;
-    auto cleanup = [&]() { ck.release(); seg.release(); cur.release(); nxt.release(); hv.release(); lam.release(); lam2.release(); };
+    // the vectors between checkpoints and the two that every call needs stay with the handle
+    // (d->x, d->y, d->z); the checkpoints, which grow with K, are given back
+    DevBuf<double> ck, seg, lam, lam2;
+    auto cleanup = [&]() { ck.release(); seg.release(); lam.release(); lam2.release(); };
     auto run = [&]() -> int {
+        const int64_t last0 = nseg > 0 ? (nseg - 1) * ckpt : 0;  // first step of the last segment
         HIP_TRY(ck.alloc(std::max<int64_t>(nseg, 1) * n));
         HIP_TRY(seg.alloc((size_t)std::min<int64_t>(ckpt, std::max<int64_t>(K, 1)) * n));
-        HIP_TRY(cur.alloc(n));
-        HIP_TRY(nxt.alloc(n));
-        HIP_TRY(hv.alloc(n));
+        HIP_TRY(d->x.alloc(n));
+        HIP_TRY(d->y.alloc(n));
+        HIP_TRY(d->z.alloc(n));
         HIP_TRY(lam.alloc(n));
         HIP_TRY(lam2.alloc(n));
-        HIP_TRY(hipMemcpyAsync(cur.p, v0, n * 8, hipMemcpyHostToDevice, d->stream));
-        // forward sweep, checkpoint every ckpt steps
+        double* cur = d->x.p;  // the final vector
+        double* hv = d->y.p;
+        HIP_TRY(hipMemcpyAsync(K > 0 ? ck.p : cur, v0, n * 8, hipMemcpyHostToDevice, d->stream));
+        // vector j of the segment that starts at step s * ckpt: its checkpoint, then seg
+        auto in_segment = [&](int64_t s, int64_t j) { return j == 0 ? ck.p + s * n : seg.p + j * n; };
+        // forward sweep: every product writes where its result stays (checkpoints, and the last
+        // segment, which the reverse sweep takes first) or alternates between two vectors
+        const double* src = ck.p;
         for (int64_t k = 0; k < K; ++k) {
-            if (k % ckpt == 0)
-                HIP_TRY(hipMemcpyAsync(ck.p + (k / ckpt) * n, cur.p, n * 8, hipMemcpyDeviceToDevice, d->stream));
-            if (int rc = apply(d, pT, cur.p, nxt.p)) return rc;
-            std::swap(cur.p, nxt.p);
+            const int64_t k1 = k + 1;
+            double* dst = k1 == K             ? cur
+                          : k1 % ckpt == 0    ? ck.p + (k1 / ckpt) * n
+                          : k1 > last0        ? in_segment(nseg - 1, k1 - last0)
+                          : (k & 1)           ? d->y.p
+                                              : d->z.p;
+            if (int rc = apply(d, pT, src, dst)) return rc;
+            src = dst;
         }
         // energy: scal[0:R] = <v|v>, scal[R:2R] = <v|Hv>; HF: scal[2R:4R] = <v|D|v>, <v|K|v>
-        if (int rc = apply(d, pH, cur.p, hv.p, d->scal.p + R)) return rc;
-        if (int rc = dot(d, cur.p, cur.p, d->scal.p)) return rc;
+        if (int rc = apply(d, pH, cur, hv, d->scal.p + R)) return rc;
+        if (int rc = dot(d, cur, cur, d->scal.p)) return rc;
         {
             double one[MAXR], unit_b[MAXR];
             for (int i = 0; i < R; ++i) { one[i] = 0; unit_b[i] = 1; }
             // pullback with ybar = v, b = 1 gives <v|D|v> and <v|K|v>; vbar is discarded
-            if (int rc = pullback(d, params(d, one, unit_b), cur.p, cur.p, lam2.p, d->scal.p + 2 * R, 0)) return rc;
+            if (int rc = pullback(d, params(d, one, unit_b), cur, cur, lam2.p, d->scal.p + 2 * R, 0)) return rc;
         }
         // cotangent of the Rayleigh quotient, and the (u, t) accumulators start at zero
-        if (int rc = rq_gradient(d, cur.p, hv.p, d->scal.p, lam.p)) return rc;
+        if (int rc = rq_gradient(d, cur, hv, d->scal.p, lam.p)) return rc;
         HIP_TRY(hipMemsetAsync(d->scal.p + 4 * R, 0, 2 * R * 8, d->stream));
-        // reverse sweep: recompute each segment from its checkpoint, then pull back
+        // reverse sweep: recompute each segment but the last from its checkpoint, then pull back
         for (int64_t s = nseg - 1; s >= 0; --s) {
-            const int64_t k0 = s * ckpt, k1 = std::min(K, k0 + ckpt);
-            HIP_TRY(hipMemcpyAsync(seg.p, ck.p + s * n, n * 8, hipMemcpyDeviceToDevice, d->stream));
-            for (int64_t k = k0; k < k1 - 1; ++k)
-                if (int rc = apply(d, pT, seg.p + (k - k0) * n, seg.p + (k - k0 + 1) * n)) return rc;
-            for (int64_t k = k1 - 1; k >= k0; --k) {
-                if (int rc = pullback(d, pT, seg.p + (k - k0) * n, lam.p, lam2.p, d->scal.p + 4 * R, 1)) return rc;
+            const int64_t len = std::min(K, (s + 1) * ckpt) - s * ckpt;
+            for (int64_t j = 1; s < nseg - 1 && j < len; ++j)
+                if (int rc = apply(d, pT, in_segment(s, j - 1), in_segment(s, j))) return rc;
+            for (int64_t j = len - 1; j >= 0; --j) {
+                if (int rc = pullback(d, pT, in_segment(s, j), lam.p, lam2.p, d->scal.p + 4 * R, 1)) return rc;
                 std::swap(lam.p, lam2.p);
             }
         }
         HIP_TRY(hipMemcpyAsync(d->h_scal, d->scal.p, 6 * R * 8, hipMemcpyDeviceToHost, d->stream));
-        if (v_final) HIP_TRY(hipMemcpyAsync(v_final, cur.p, n * 8, hipMemcpyDeviceToHost, d->stream));
+        if (v_final) HIP_TRY(hipMemcpyAsync(v_final, cur, n * 8, hipMemcpyDeviceToHost, d->stream));
         HIP_TRY(hipStreamSynchronize(d->stream));
         const double* h = d->h_scal;
         for (int i = 0; i < R; ++i) {
@@ -757,9 +766,8 @@ int rimu_dense_ground_state(rimu_dense* d, const double* v0, int64_t max_iters, 
     double a_h[MAXR], b_h[MAXR];
     for (int i = 0; i < R; ++i) { a_h[i] = 0; b_h[i] = 1; }
     const DenseParams pH = params(d, a_h, b_h);
-    DevBuf<double> v, vprev, w, hist;
+    DevBuf<double>&v = d->x, &vprev = d->y, &w = d->z, &hist = d->hist;  // kept with the handle
     // hist: alpha [cap][R], then beta^2 [cap + 1][R] (beta^2[0] = 0), then |v0|^2 [R]
-    auto cleanup = [&]() { v.release(); vprev.release(); w.release(); hist.release(); };
     auto run = [&]() -> int {
         HIP_TRY(v.alloc(n));
         HIP_TRY(vprev.alloc(n));
@@ -780,7 +788,7 @@ int rimu_dense_ground_state(rimu_dense* d, const double* v0, int64_t max_iters, 
             if (int rc = apply(d, pH, v.p, w.p, alpha + j * R)) return rc;
             if (int rc = lanczos_update(d, w.p, v.p, vprev.p, alpha + j * R, beta2 + j * R,
                                         beta2 + (j + 1) * R, vprev.p, FLOOR2)) return rc;
-            std::swap(v.p, vprev.p);
+            std::swap(v, vprev);
             const bool last_iter = j + 1 == cap;
             if ((j + 1) % CHECK != 0 && !last_iter) continue;
             const int64_t m = j + 1;
@@ -814,9 +822,7 @@ int rimu_dense_ground_state(rimu_dense* d, const double* v0, int64_t max_iters, 
         if (iters) *iters = j;
         return RIMU_OK;
     };
-    const int rc = run();
-    cleanup();
-    return rc;
+    return run();
 }
 
 }  // extern "C"
