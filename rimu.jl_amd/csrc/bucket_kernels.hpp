@@ -34,17 +34,24 @@
 namespace rimu {
 
 constexpr int BK_NT = 512;                    // threads of a bucket workgroup
-constexpr int BK_CAP = 2560;                  // records + vector entries per bucket in LDS
-constexpr int BK_IPT = BK_CAP / BK_NT;        // items per thread
+constexpr int BK_IPT_MIN = 3, BK_IPT_MAX = 5;  // items per thread of the smallest and largest shape
 constexpr int BK_IDX_BITS = 12;               // item index below the key bits of a packed word
-constexpr int BK_SUB_BITS = 11;               // sub-buckets of the LDS sort
-constexpr int BK_NSUB = 1 << BK_SUB_BITS;
-constexpr int BK_WG_PER_CU = 2;               // resident bucket workgroups per CU (LDS-bound)
 constexpr int BK_SORT_WIN = 2;                // sub-bucket words read at once by the ranking
 constexpr int BK_FOLD_EXTRA = 4;              // positions read past a thread's own for its runs
-static_assert(BK_CAP <= (1 << BK_IDX_BITS), "item indices fit their bits");
-static_assert(BK_CAP % BK_NT == 0 && BK_NSUB % BK_NT == 0, "whole rounds per thread");
-static_assert(BK_IPT < 8, "survivor masks are 32-bit; per-thread counts fit three bits");
+
+// A bucket kernel is built for buckets of up to IPT * BK_NT items (records + vector entries).
+// A bucket's LDS and the registers of its threads grow with IPT, so the smallest that holds
+// the step's buckets keeps the most workgroups on a CU and the fewest idle item slots:
+// BkShape::WG_PER_CU workgroups of 512 threads.
+template <int IPT> struct BkShape {
+    static constexpr int CAP = BK_NT * IPT;
+    static constexpr int SUB_BITS = 11;  // sub-buckets of the LDS sort
+    static constexpr int NSUB = 1 << SUB_BITS;
+    static constexpr int WG_PER_CU = IPT == 3 ? 3 : 2;
+    static_assert(CAP <= (1 << BK_IDX_BITS), "item indices fit their bits");
+    static_assert(NSUB % BK_NT == 0, "whole rounds per thread");
+    static_assert(IPT < 8, "survivor masks are 32-bit; per-thread counts fit three bits");
+};
 constexpr int FLAG_BUCKET_OVERFLOW = 16;
 
 // First record and first vector entry of every bucket: rstart[b] = lower bound of b among
@@ -112,13 +119,14 @@ __device__ inline T bk_block_exclusive_scan(T v, int lane, int wid, T* s_wave, T
 // LDS of one bucket workgroup.  `vin` holds the items' values by item index and `place`
 // their packed words sub-bucket by sub-bucket; `sk` receives the words in order.  After the
 // fold `place` and `vin` stage the values that ThresholdCompression draws for.
-template <class V, bool INIT>
+template <class V, bool INIT, int IPT>
 struct BucketLds {
-    uint64_t place[BK_CAP];
-    uint64_t sk[BK_CAP];
-    V vin[BK_CAP];
-    uint8_t cls[INIT ? BK_CAP : 1];  // initiator runs: the class of every item (see below)
-    uint32_t sub[BK_NSUB + 1];      // sub-bucket counts, then their starts
+    static constexpr int CAP = BkShape<IPT>::CAP;
+    uint64_t place[CAP];
+    uint64_t sk[CAP];
+    V vin[CAP];
+    uint8_t cls[INIT ? CAP : 1];  // initiator runs: the class of every item (see below)
+    uint32_t sub[BkShape<IPT>::NSUB + 1];  // sub-bucket counts, then their starts
     double red[2][BK_NT / WAVE];
     uint32_t scan_u[BK_NT / WAVE];
     int scan_i[BK_NT / WAVE];
@@ -133,15 +141,17 @@ struct BucketLds {
 // each address folds three components in list order -- safe (entries with the class, records
 // without), unsafe (records with the class), initiator (entries without) -- exists when one
 // is nonzero and takes the rule's value (initiator_value), as merge_kernel<K, V, true> does.
-template <class V, bool INIT>
-__global__ __launch_bounds__(BK_NT, 2 * BK_WG_PER_CU) void bucket_merge_kernel(
+template <class V, bool INIT, int IPT>
+__global__ __launch_bounds__(BK_NT, 2 * BkShape<IPT>::WG_PER_CU) void bucket_merge_kernel(
     StepArgs a, const uint64_t* __restrict__ ak, const V* __restrict__ av, const uint64_t* __restrict__ bk,
     const V* __restrict__ bv, const V* __restrict__ bo, const int64_t* __restrict__ rstart, const int64_t* __restrict__ vstart, int64_t nbk,
     int lowbits, uint64_t* __restrict__ slot_k, V* __restrict__ slot_v, int64_t* __restrict__ bucket_cnt,
     double* __restrict__ partials, int* flags) {
     constexpr int NW = BK_NT / WAVE;
     constexpr uint64_t IDX_MASK = (1ull << BK_IDX_BITS) - 1ull;
-    __shared__ BucketLds<V, INIT> sm;
+    constexpr int BK_IPT = IPT, BK_CAP = BkShape<IPT>::CAP;
+    constexpr int BK_SUB_BITS = BkShape<IPT>::SUB_BITS, BK_NSUB = BkShape<IPT>::NSUB;
+    __shared__ BucketLds<V, INIT, IPT> sm;
     // no sorted list to merge (raised by earlier kernels only: every wave reads the same bits)
     if (*flags & (FLAG_LOOKBACK | FLAG_SPEC)) {
         for (int64_t b = blockIdx.x; b < nbk; b += gridDim.x) {
@@ -514,7 +524,7 @@ __global__ __launch_bounds__(BK_NT, 2 * BK_WG_PER_CU) void bucket_merge_kernel(
 // Survivors of bucket b move from its slot range [rstart[b] + vstart[b], ...) to
 // [offs[b], offs[b + 1]) (offs: exclusive scan of the bucket counts; offs[nbuckets] is the new
 // length).  A new length above cap writes nothing and raises FLAG_VECTOR_OVERFLOW.
-template <class V>
+template <class V, int IPT>
 __global__ __launch_bounds__(NT) void bucket_compact_kernel(const uint64_t* __restrict__ slot_k,
                                                             const V* __restrict__ slot_v,
                                                             const int64_t* __restrict__ rstart,
@@ -535,7 +545,7 @@ __global__ __launch_bounds__(NT) void bucket_compact_kernel(const uint64_t* __re
     const int64_t off = offs[b];
     const int n = (int)(offs[b + 1] - off);
     const int64_t src = rstart[b] + vstart[b];
-    constexpr int CPT = (BK_CAP + NT - 1) / NT;
+    constexpr int CPT = BkShape<IPT>::CAP / NT;
     uint64_t k[CPT];
     V v[CPT];
 #pragma unroll

@@ -124,6 +124,7 @@ struct rimu_engine {
     DevBuf<uint64_t> lb_status;     // look-back radix: status words [pass][tile][digit]
     uint32_t lb_epoch = 0;          // sort calls since lb_status was last cleared
     int bucket_cooldown = 0;        // steps left on the merge path after a bucket overflow
+    int bucket_ipt_min = BK_IPT_MIN;  // smallest bucket shape (items per thread) the steps may take
     bool spec_ok = false;           // the grids of the next step may be sized from W_prev, S_prev
     int64_t W_prev = 0, S_prev = 0; // spawn attempts and records of the last step
     uint32_t lb_spin_limit = LB_SPIN_LIMIT;  // bound of every look-back wait
@@ -314,16 +315,27 @@ int scan_u32(rimu_engine* e, const uint32_t* in, uint32_t* out, int64_t n) {
 // whose digit is the same for every key.  Bits at and above nbits are carried, not sorted
 // (the initiator class bit).  Input in buffer `in`; returns the buffer index holding the
 // result.
-template <class K, class V>
+template <class K, class V, int RB>
 int radix_sort_lb(rimu_engine* e, int64_t n, int nbits, u128 varying, int in, int* result, int lo,
                   const int64_t* n_dev);
+
+// Nine-bit digits where they save a pass over the records (17 or 18 key bits in two passes
+// instead of three); else eight, whose passes are a little cheaper.  Past 36 bits the counts
+// of a sort with 512 digits would outgrow the arrays laid out for 256 (rimu_annihilate_noalloc).
+bool nine_bit_digits(int nbits, int lo) {
+    return nbits - lo <= 36 && ceil_div(nbits - lo, 9) < ceil_div(nbits - lo, RADIX_BITS);
+}
 
 template <class K, class V>
 int radix_sort(rimu_engine* e, int64_t n, int nbits, u128 varying, int in, int* result, int lo = 0,
                const int64_t* n_dev = nullptr) {
     int src = in;
     if (n <= 1 && !n_dev) { *result = src; return RIMU_OK; }
-    if (e->radix_mode != 0 || n_dev) return radix_sort_lb<K, V>(e, n, nbits, varying, in, result, lo, n_dev);
+    if (e->radix_mode != 0 || n_dev) {
+        if constexpr (sizeof(K) == 8)
+            if (nine_bit_digits(nbits, lo)) return radix_sort_lb<K, V, 9>(e, n, nbits, varying, in, result, lo, n_dev);
+        return radix_sort_lb<K, V, 8>(e, n, nbits, varying, in, result, lo, n_dev);
+    }
     const int64_t tiles = ceil_div(n, sort_tile<K>::value);
     const int64_t nchunks = ceil_div(tiles, RADIX_CHUNK);
     HIP_TRY(e->rcounts.alloc((size_t)tiles * RADIX));
@@ -358,24 +370,25 @@ int radix_sort(rimu_engine* e, int64_t n, int nbits, u128 varying, int in, int* 
 // path: the ranks within a tile and the digit offsets are the same numbers.  FLAG_LOOKBACK
 // in the step's flags reports a look-back that did not complete.  With n_dev the record
 // count is in device memory and n is the most the grids are sized for.
-template <class K, class V>
+template <class K, class V, int RB>
 int radix_sort_lb(rimu_engine* e, int64_t n, int nbits, u128 varying, int in, int* result, int lo,
                   const int64_t* n_dev) {
+    constexpr int NDIG = 1 << RB;
     int src = in;
     PassSet ps{};
-    for (int shift = lo; shift < nbits; shift += RADIX_BITS) {
-        if ((uint32_t)((varying >> shift) & (RADIX - 1)) == 0) continue;  // digit constant: pass is identity
+    for (int shift = lo; shift < nbits; shift += RB) {
+        if ((uint32_t)((varying >> shift) & (NDIG - 1)) == 0) continue;  // digit constant: pass is identity
         if (ps.n == MAX_PASSES) return fail(RIMU_ERR_INTERNAL, "too many radix passes");
         ps.shift[ps.n] = shift;
-        ps.dmask[ps.n] = shift + RADIX_BITS > nbits ? (1u << (nbits - shift)) - 1u : (uint32_t)(RADIX - 1);
+        ps.dmask[ps.n] = shift + RB > nbits ? (1u << (nbits - shift)) - 1u : (uint32_t)(NDIG - 1);
         ++ps.n;
     }
     if (ps.n == 0) { *result = src; return RIMU_OK; }
     if (n > (int64_t)RLB_VALUE) return fail(RIMU_ERR_CAPACITY, "radix sort of 2^32 or more records");
     const int64_t tiles = ceil_div(n, sort_tile<K>::value);
-    const size_t need = (size_t)ps.n * tiles * RADIX;
-    HIP_TRY(e->lb_hist.alloc((size_t)ps.n * RADIX + MAX_PASSES));
-    uint32_t* counters = e->lb_hist.p + (int64_t)ps.n * RADIX;  // tile ids (two-word keys)
+    const size_t need = (size_t)ps.n * tiles * NDIG;
+    HIP_TRY(e->lb_hist.alloc((size_t)ps.n * NDIG + MAX_PASSES));
+    uint32_t* counters = e->lb_hist.p + (int64_t)ps.n * NDIG;  // tile ids (two-word keys)
     int* flags = &((rimu_engine::Misc*)e->misc.p)->flags;
     hipEvent_t ev{};
     if (need > e->lb_status.n || e->lb_epoch >= RLB_EPOCH_MAX) {  // epoch 0: cleared words
@@ -388,17 +401,17 @@ int radix_sort_lb(rimu_engine* e, int64_t n, int nbits, u128 varying, int in, in
     HIP_TRY(hipMemsetAsync(counters, 0, sizeof(uint32_t) * MAX_PASSES, e->stream));
     const int copies = hist_all_copies(ps.n);
     const int hblocks = (int)std::min<int64_t>(tiles, HIST_ALL_BLOCKS);
-    HIP_TRY(e->lb_part.alloc((size_t)HIST_ROWS * ps.n * RADIX));
-    HIP_TRY(hipMemsetAsync(e->lb_part.p, 0, sizeof(uint32_t) * HIST_ROWS * ps.n * RADIX, e->stream));
-    radix_hist_all_kernel<K><<<hblocks, NT, sizeof(uint32_t) * ps.n * copies * HIST_STRIDE, e->stream>>>(
+    HIP_TRY(e->lb_part.alloc((size_t)HIST_ROWS * ps.n * NDIG));
+    HIP_TRY(hipMemsetAsync(e->lb_part.p, 0, sizeof(uint32_t) * HIST_ROWS * ps.n * NDIG, e->stream));
+    radix_hist_all_kernel<K, RB><<<hblocks, NT, sizeof(uint32_t) * ps.n * copies * (NDIG + 1), e->stream>>>(
         (const K*)e->skeys[src].p, Count{n, n_dev, n}, flags, ps, copies, e->lb_part.p);
-    radix_hist_base_kernel<<<ps.n, RADIX, 0, e->stream>>>(e->lb_part.p, ps.n, e->lb_hist.p);
+    radix_hist_base_kernel<RB><<<ps.n, NDIG, 0, e->stream>>>(e->lb_part.p, ps.n, e->lb_hist.p);
     e->timer.end(e->stream);
     for (int p = 0; p < ps.n; ++p) {
         e->timer.begin("radix_scatter", e->stream, &ev);
-        radix_scatter_lb_kernel<K, V><<<tiles, NT, 0, e->stream>>>(
+        radix_scatter_lb_kernel<K, V, RB><<<tiles, NDIG, 0, e->stream>>>(
             (const K*)e->skeys[src].p, (const V*)e->svals[src].p, Count{n, n_dev, n}, ps.shift[p], ps.dmask[p],
-            e->lb_hist.p + (int64_t)p * RADIX, e->lb_status.p + (int64_t)p * tiles * RADIX, epoch, counters + p,
+            e->lb_hist.p + (int64_t)p * NDIG, e->lb_status.p + (int64_t)p * tiles * NDIG, epoch, counters + p,
             flags, LookbackCtl{e->lb_spin_limit, e->lb_withhold},
             (K*)e->skeys[1 - src].p, (V*)e->svals[1 - src].p);
         e->timer.end(e->stream);
@@ -542,25 +555,45 @@ int reorder_on_device(rimu_engine* e, int64_t n, int forward, int* result, Fill&
 // the vector (bk, bv: keys and diagonal survivors, L entries; bo: the old values, which give
 // the entries' initiator class when an initiator rule is set) into (ok, ov) of capacity cap.
 // `tiles` receives the number of buckets (rows of merge_p).
-constexpr double BK_FILL = 1800;    // mean items (records + entries) per bucket aimed at
-constexpr double BK_FILL_MAX = 2050; // highest mean kept to save a radix pass (LDS holds BK_CAP)
 constexpr int64_t BK_MIN_RECORDS = 4096;
 constexpr int BK_MAX_LOWBITS = 48;   // packed words: key bits below the bucket bits + a 12-bit item index
 constexpr int BK_COOLDOWN = 16;      // steps on the merge path after a bucket overflowed
 
-// Top bits that split S records and L entries into buckets of about BK_FILL items; one bit
-// fewer when that saves a radix pass (8 bits each) and keeps the mean below BK_FILL_MAX.
-int bucket_bits(int64_t S, int64_t L, int B) {
-    const double items = (double)S + (double)L;
-    int T = (int)std::ceil(std::log2(std::max(items / BK_FILL, 2.0)));
-    if (T > 1 && T % RADIX_BITS == 1 && items / std::ldexp(1.0, T - 1) <= BK_FILL_MAX) --T;
-    return std::min(std::max(T, 1), std::min(B, 24));
+// How a step's records are cut into buckets: the top T stored-key bits, and the kernel shape
+// (items per thread) that holds a bucket.
+struct BucketCut {
+    int T = 0;    // 0: no bucket merge
+    int ipt = 0;
+};
+
+// The largest mean of a shape: seven standard deviations below its capacity, for counts that
+// vary twice as much as independent ones (records come to addresses in groups).
+double bucket_mean_max(int ipt) {
+    const double cap = (double)BK_NT * ipt, x = std::sqrt(cap + 24.5) - std::sqrt(24.5);
+    return x * x;
 }
 
-template <class V>
-int bucket_merge_into(rimu_engine* e, const StepArgs& a, const uint64_t* ak, const V* av, int64_t S,
+// S records and L entries: the fewest buckets, in the smallest shape (at least `min_ipt` items
+// per thread) that holds them.  A bucket costs its workgroup seven microseconds or more
+// whatever it holds, so more and smaller buckets lose: 1.6e7 items in 2^13, 2^14, 2^15, 2^16
+// buckets take 158, 183, 226, 412 us (the last two with two items per thread and four
+// workgroups on a CU, a shape no step takes now); 1.5e8 items in 2^17 buckets take 2.75 ms with
+// three items per thread (three workgroups on a CU) and 3.22 ms with five (two).
+BucketCut bucket_cut(int64_t S, int64_t L, int B, int min_ipt) {
+    const double items = (double)S + (double)L;
+    BucketCut cut;
+    cut.T = 1;
+    while (cut.T < std::min(B, 24) && std::ldexp(items, -cut.T) > bucket_mean_max(BK_IPT_MAX)) ++cut.T;
+    cut.ipt = min_ipt;
+    while (cut.ipt < BK_IPT_MAX && std::ldexp(items, -cut.T) > bucket_mean_max(cut.ipt)) ++cut.ipt;
+    if (B - cut.T > BK_MAX_LOWBITS) cut.T = 0;
+    return cut;
+}
+
+template <class V, int IPT>
+int bucket_merge_shape(rimu_engine* e, const StepArgs& a, const uint64_t* ak, const V* av, int64_t S,
                       const uint64_t* bk, const V* bv, const V* bo, int64_t L, int T, uint64_t* ok, V* ov,
-                      int64_t cap, rimu_engine::Misc* dm, int64_t* tiles, const int64_t* S_dev = nullptr) {
+                      int64_t cap, rimu_engine::Misc* dm, int64_t* tiles, const int64_t* S_dev) {
     const int B = e->hdev.B;
     const int64_t nbk = (int64_t)1 << T;
     *tiles = nbk;
@@ -580,26 +613,37 @@ int bucket_merge_into(rimu_engine* e, const StepArgs& a, const uint64_t* ak, con
         HIP_TRY(hipDeviceGetAttribute(&e->n_cu, hipDeviceAttributeMultiprocessorCount, e->device));
         if (e->n_cu <= 0) e->n_cu = 1;
     }
-    const int64_t grid = std::min(nbk, (int64_t)e->n_cu * BK_WG_PER_CU);
+    const int64_t grid = std::min(nbk, (int64_t)e->n_cu * BkShape<IPT>::WG_PER_CU);
     e->timer.begin("bucket_merge", e->stream, &ev);
     if (a.init_rule != 0)
-        bucket_merge_kernel<V, true><<<grid, BK_NT, 0, e->stream>>>(
+        bucket_merge_kernel<V, true, IPT><<<grid, BK_NT, 0, e->stream>>>(
             a, ak, av, bk, bv, bo, e->bk_rstart.p, e->bk_vstart.p, nbk, B - T, e->slot_k.p, (V*)e->slot_v.p,
             e->tile_cnt.p, e->merge_p.p, &dm->flags);
     else
-        bucket_merge_kernel<V, false><<<grid, BK_NT, 0, e->stream>>>(
+        bucket_merge_kernel<V, false, IPT><<<grid, BK_NT, 0, e->stream>>>(
             a, ak, av, bk, bv, nullptr, e->bk_rstart.p, e->bk_vstart.p, nbk, B - T, e->slot_k.p, (V*)e->slot_v.p,
             e->tile_cnt.p, e->merge_p.p, &dm->flags);
     e->timer.end(e->stream);
     HIP_TRY(hipGetLastError());
     e->timer.begin("compact", e->stream, &ev);
     if (int rc = scan_inplace_i64(e, e->tile_cnt.p, nbk + 1)) return rc;
-    bucket_compact_kernel<V><<<nbk, NT, 0, e->stream>>>(e->slot_k.p, (const V*)e->slot_v.p, e->bk_rstart.p,
+    bucket_compact_kernel<V, IPT><<<nbk, NT, 0, e->stream>>>(e->slot_k.p, (const V*)e->slot_v.p, e->bk_rstart.p,
                                                         e->bk_vstart.p, e->tile_cnt.p, nbk, ok, ov, cap,
                                                         &dm->L_new, &dm->flags);
     e->timer.end(e->stream);
     HIP_TRY(hipGetLastError());
     return RIMU_OK;
+}
+
+template <class V>
+int bucket_merge_into(rimu_engine* e, const StepArgs& a, const uint64_t* ak, const V* av, int64_t S,
+                      const uint64_t* bk, const V* bv, const V* bo, int64_t L, const BucketCut& cut, uint64_t* ok,
+                      V* ov, int64_t cap, rimu_engine::Misc* dm, int64_t* tiles, const int64_t* S_dev = nullptr) {
+    switch (cut.ipt) {
+        case 3: return bucket_merge_shape<V, 3>(e, a, ak, av, S, bk, bv, bo, L, cut.T, ok, ov, cap, dm, tiles, S_dev);
+        case 4: return bucket_merge_shape<V, 4>(e, a, ak, av, S, bk, bv, bo, L, cut.T, ok, ov, cap, dm, tiles, S_dev);
+        default: return bucket_merge_shape<V, 5>(e, a, ak, av, S, bk, bv, bo, L, cut.T, ok, ov, cap, dm, tiles, S_dev);
+    }
 }
 
 // A HubbardRealSpace model has off-diagonal elements of value zero (which the reference
@@ -637,13 +681,9 @@ int step_impl(rimu_engine* e, int64_t step, double shift, double dtau, double bo
     const int nbits = e->hdev.B;
     const bool bucket_ok = KW == 1 && e->radix_mode == 2 && e->mix.on && e->bucket_cooldown == 0;
     bool spec = e->spec_ok && e->radix_mode != 0 && e->W_prev > 0;
-    int T_spec = 0;
-    if (spec) {  // the path the counts of the last step choose; sorts with a host check stay synchronous
-        if (bucket_ok && e->S_prev >= BK_MIN_RECORDS) {
-            T_spec = bucket_bits(e->S_prev, L, nbits);
-            if (nbits - T_spec > BK_MAX_LOWBITS) T_spec = 0;
-        }
-    }
+    BucketCut cut;
+    // the path the counts of the last step choose; sorts with a host check stay synchronous
+    if (spec && bucket_ok && e->S_prev >= BK_MIN_RECORDS) cut = bucket_cut(e->S_prev, L, nbits, e->bucket_ipt_min);
     const int64_t W_cap = spec ? e->W_prev + e->W_prev / 4 + 16 * SPAWN_TILE : 0;
 
     // 1. plan: diagonal step, attempt offsets and the first entry of each spawn tile (as
@@ -767,11 +807,7 @@ int step_impl(rimu_engine* e, int64_t step, double shift, double dtau, double bo
     const int nxt = 1 - e->cur;
     int64_t merge_tiles = 0;
     int sorted = 0;
-    int T = T_spec;
-    if (!spec && bucket_ok && S >= BK_MIN_RECORDS) {
-        T = bucket_bits(S, L, nbits);
-        if (nbits - T > BK_MAX_LOWBITS) T = 0;
-    }
+    if (!spec && bucket_ok && S >= BK_MIN_RECORDS) cut = bucket_cut(S, L, nbits, e->bucket_ipt_min);
     if (e->bucket_cooldown > 0) --e->bucket_cooldown;
     const int64_t* merge_S_dev = S_dev;  // the merge path after the fallback sort reads S from the host
     auto merge_path = [&]() -> int {
@@ -779,10 +815,10 @@ int step_impl(rimu_engine* e, int64_t step, double shift, double dtau, double bo
                                 (const V*)e->dvals.p, L, (K*)e->vkeys[nxt].p, (V*)e->vvals[nxt].p,
                                 e->max_entries, dm, &merge_tiles, vv, merge_S_dev);
     };
-    if (T > 0) {
-        if (int rc = radix_sort<K, V>(e, S, nbits, kor ^ kand, 0, &sorted, nbits - T, S_dev)) return rc;
+    if (cut.T > 0) {
+        if (int rc = radix_sort<K, V>(e, S, nbits, kor ^ kand, 0, &sorted, nbits - cut.T, S_dev)) return rc;
         if (int rc = bucket_merge_into<V>(e, a, (const uint64_t*)e->skeys[sorted].p, (const V*)e->svals[sorted].p,
-                                          S, (const uint64_t*)vk, (const V*)e->dvals.p, vv, L, T,
+                                          S, (const uint64_t*)vk, (const V*)e->dvals.p, vv, L, cut,
                                           (uint64_t*)e->vkeys[nxt].p, (V*)e->vvals[nxt].p, e->max_entries, dm,
                                           &merge_tiles, S_dev)) return rc;
     } else {
@@ -872,6 +908,7 @@ int step_impl(rimu_engine* e, int64_t step, double shift, double dtau, double bo
         // sort the bucketed records on every bit (stable passes keep their list order within
         // an address) and merge along the merge path
         e->bucket_cooldown = BK_COOLDOWN;
+        e->bucket_ipt_min = BK_IPT_MAX;  // uneven counts: the roomiest buckets from now on
         e->timer.begin("bucket_fallback", e->stream, &ev);
         e->timer.end(e->stream);
         HIP_TRY(hipMemsetAsync(&dm->flags, 0, sizeof(int), e->stream));

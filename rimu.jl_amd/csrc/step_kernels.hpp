@@ -887,6 +887,7 @@ __global__ __launch_bounds__(NT) void radix_scatter_kernel(const K* __restrict__
 // within the tile and the scatter are those of radix_scatter_kernel, so the output is the
 // same.
 // ---------------------------------------------------------------------------------------
+// The digits of a sort have RB = 8 or 9 bits (nine where they save a pass).
 constexpr int MAX_PASSES = 16;
 constexpr int LB_WIN = 8;   // predecessor status words read per look-back round
 // Status words of the radix look-back: flag (2 bits, as LB_FLAG_*), the epoch of the sort
@@ -901,19 +902,20 @@ struct PassSet {
     uint32_t dmask[MAX_PASSES];
 };
 
-// part[(b % HIST_ROWS * ps.n + p) * RADIX + d] += count of digit d of pass p over the tiles
+// part[(b % HIST_ROWS * ps.n + p) * 2^RB + d] += count of digit d of pass p over the tiles
 // of workgroup b (grid-stride over tiles).  The workgroups add into HIST_ROWS rows, not
 // one: 2048 workgroups adding into the same 256 words per pass serialize on them.
-// Dynamic LDS: ps.n * copies * HIST_STRIDE words (copies as in radix_count_kernel; the
+// Dynamic LDS: ps.n * copies * (2^RB + 1) words (copies as in radix_count_kernel; the
 // host takes hist_all_copies(ps.n), which keeps the array within 64 KiB).
 __host__ __device__ inline int hist_all_copies(int npasses) { return npasses <= 8 ? 4 : 2; }
 constexpr int HIST_ALL_BLOCKS = 2048;
 constexpr int HIST_ROWS = 64;
-template <class K>
+template <class K, int RB>
 __global__ __launch_bounds__(NT) void radix_hist_all_kernel(const K* __restrict__ keys, Count cn, int* flags,
                                                             PassSet ps, int copies, uint32_t* __restrict__ part) {
     constexpr int IPT = sort_ipt<K>::value;
     constexpr int TILE = sort_tile<K>::value;
+    constexpr int NDIG = 1 << RB, STRIDE = NDIG + 1;
     extern __shared__ uint32_t h_all[];
     // every thread computes the same n: the early return is uniform
     const int64_t n = count_value(cn);
@@ -921,7 +923,7 @@ __global__ __launch_bounds__(NT) void radix_hist_all_kernel(const K* __restrict_
         if (blockIdx.x == 0 && threadIdx.x == 0) atomicOr(flags, FLAG_SPEC);
         return;
     }
-    const int words = ps.n * copies * HIST_STRIDE;
+    const int words = ps.n * copies * STRIDE;
     for (int j = threadIdx.x; j < words; j += NT) h_all[j] = 0;
     __syncthreads();
     const int copy = threadIdx.x % copies;
@@ -934,7 +936,7 @@ __global__ __launch_bounds__(NT) void radix_hist_all_kernel(const K* __restrict_
         for (int p = 0; p < ps.n; ++p) {
             const int shift = ps.shift[p];
             const uint32_t dmask = ps.dmask[p];
-            uint32_t* mine = h_all + (p * copies + copy) * HIST_STRIDE;
+            uint32_t* mine = h_all + (p * copies + copy) * STRIDE;
 #pragma unroll
             for (int r = 0; r < IPT; ++r)
                 if (base + (int64_t)r * NT + threadIdx.x < n)
@@ -942,45 +944,54 @@ __global__ __launch_bounds__(NT) void radix_hist_all_kernel(const K* __restrict_
         }
     }
     __syncthreads();
-    for (int p = 0; p < ps.n; ++p) {
+    for (int j = threadIdx.x; j < ps.n * NDIG; j += NT) {
+        const int p = j >> RB, d = j & (NDIG - 1);
         uint32_t c = 0;
-        for (int q = 0; q < copies; ++q) c += h_all[(p * copies + q) * HIST_STRIDE + threadIdx.x];
-        if (c) atomicAdd(&part[((int64_t)(blockIdx.x % HIST_ROWS) * ps.n + p) * RADIX + threadIdx.x], c);
+        for (int q = 0; q < copies; ++q) c += h_all[(p * copies + q) * STRIDE + d];
+        if (c) atomicAdd(&part[(int64_t)(blockIdx.x % HIST_ROWS) * ps.n * NDIG + j], c);
     }
 }
 
 // hist[p][d] = sum over d' < d of the digit counts of pass p, the counts summed over the
 // HIST_ROWS rows of part (one workgroup per pass, one thread per digit).
-__global__ __launch_bounds__(RADIX) void radix_hist_base_kernel(const uint32_t* __restrict__ part,
-                                                                int npasses, uint32_t* __restrict__ hist) {
+template <int RB>
+__global__ __launch_bounds__(1 << RB) void radix_hist_base_kernel(const uint32_t* __restrict__ part,
+                                                                  int npasses, uint32_t* __restrict__ hist) {
+    constexpr int NDIG = 1 << RB;
     const int p = blockIdx.x;
     uint32_t c = 0;
 #pragma unroll 16
-    for (int b = 0; b < HIST_ROWS; ++b) c += part[((int64_t)b * npasses + p) * RADIX + threadIdx.x];
+    for (int b = 0; b < HIST_ROWS; ++b) c += part[((int64_t)b * npasses + p) * NDIG + threadIdx.x];
     uint32_t tot;
-    const uint32_t ex = block_exclusive_scan<uint32_t, RADIX>(c, &tot);
-    hist[p * RADIX + threadIdx.x] = ex;
+    const uint32_t ex = block_exclusive_scan<uint32_t, NDIG>(c, &tot);
+    hist[p * NDIG + threadIdx.x] = ex;
 }
 
-template <class K, class V>
-__global__ __launch_bounds__(NT) void radix_scatter_lb_kernel(const K* __restrict__ keys_in,
-                                                              const V* __restrict__ vals_in, Count cn,
-                                                              int shift, uint32_t dmask,
-                                                              const uint32_t* __restrict__ gbase,
-                                                              uint64_t* status, uint32_t epoch,
-                                                              uint32_t* tile_counter, int* flags,
-                                                              LookbackCtl ctl,
-                                                              K* __restrict__ keys_out,
-                                                              V* __restrict__ vals_out) {
-    constexpr int NW = NT / WAVE;
-    constexpr int IPT = sort_ipt<K>::value;
+// One thread per digit: 256 threads for 8-bit digits, 512 for 9-bit ones, on the same tiles.
+// Per-wavefront counts are at most TILE, so 16 bits hold them (a second workgroup of 512
+// threads fits the CU's LDS).
+template <class K, class V, int RB>
+__global__ __launch_bounds__(1 << RB) void radix_scatter_lb_kernel(const K* __restrict__ keys_in,
+                                                                   const V* __restrict__ vals_in, Count cn,
+                                                                   int shift, uint32_t dmask,
+                                                                   const uint32_t* __restrict__ gbase,
+                                                                   uint64_t* status, uint32_t epoch,
+                                                                   uint32_t* tile_counter, int* flags,
+                                                                   LookbackCtl ctl,
+                                                                   K* __restrict__ keys_out,
+                                                                   V* __restrict__ vals_out) {
+    constexpr int NDIG = 1 << RB;
+    constexpr int NTS = NDIG;
+    constexpr int NW = NTS / WAVE;
     constexpr int TILE = sort_tile<K>::value;
+    constexpr int IPT = TILE / NTS;
+    static_assert(TILE % NTS == 0 && TILE <= UINT16_MAX, "whole rounds per thread, 16-bit counts");
     __shared__ K s_k[TILE];
     __shared__ V s_v[TILE];
-    __shared__ uint32_t s_wcnt[NW][RADIX];
-    __shared__ uint32_t s_start[RADIX];
-    __shared__ uint32_t s_run[RADIX];
-    __shared__ uint32_t s_goff[RADIX];
+    __shared__ uint16_t s_wcnt[NW][NDIG];
+    __shared__ uint32_t s_start[NDIG];
+    __shared__ uint32_t s_run[NDIG];
+    __shared__ uint32_t s_goff[NDIG];
 
     // tile ids in start order from a counter: every tile a tile waits for has started,
     // whatever order the workgroups are dispatched in (also measured faster than tile =
@@ -997,13 +1008,13 @@ __global__ __launch_bounds__(NT) void radix_scatter_lb_kernel(const K* __restric
     const int64_t base = (int64_t)tile * TILE;
     const int64_t wbase = base + (int64_t)wid * IPT * WAVE;
 
-    for (int j = threadIdx.x; j < NW * RADIX; j += NT) (&s_wcnt[0][0])[j] = 0;
+    for (int j = threadIdx.x; j < NW * NDIG / 2; j += NTS) ((uint32_t*)&s_wcnt[0][0])[j] = 0;
     __syncthreads();
 
     K k[IPT];
     V v[IPT];
     uint32_t rank[IPT];
-    uint32_t* cnt = s_wcnt[wid];
+    uint16_t* cnt = s_wcnt[wid];
 #pragma unroll
     for (int r = 0; r < IPT; ++r) {
         const int64_t idx = wbase + (int64_t)r * WAVE + lane;
@@ -1018,7 +1029,7 @@ __global__ __launch_bounds__(NT) void radix_scatter_lb_kernel(const K* __restric
         const uint32_t digit = (uint32_t)(k[r] >> shift) & dmask;
         uint64_t peers = __ballot(valid);
 #pragma unroll
-        for (int b = 0; b < RADIX_BITS; ++b) {
+        for (int b = 0; b < RB; ++b) {
             const uint64_t bb = __ballot((digit >> b) & 1u);
             peers &= ((digit >> b) & 1u) ? bb : ~bb;
         }
@@ -1026,7 +1037,7 @@ __global__ __launch_bounds__(NT) void radix_scatter_lb_kernel(const K* __restric
         const uint32_t in_wave = (uint32_t)__popcll(peers & lt_mask);
         rank[r] = before + in_wave;
         __builtin_amdgcn_wave_barrier();
-        if (valid && in_wave == 0) cnt[digit] = before + (uint32_t)__popcll(peers);
+        if (valid && in_wave == 0) cnt[digit] = (uint16_t)(before + (uint32_t)__popcll(peers));
         __builtin_amdgcn_wave_barrier();
     }
     __syncthreads();
@@ -1036,14 +1047,14 @@ __global__ __launch_bounds__(NT) void radix_scatter_lb_kernel(const K* __restric
 #pragma unroll
         for (int w = 0; w < NW; ++w) {
             const uint32_t c = s_wcnt[w][d];
-            s_wcnt[w][d] = run;
+            s_wcnt[w][d] = (uint16_t)run;
             run += c;
         }
         uint32_t tot;
-        s_start[d] = block_exclusive_scan<uint32_t, NT>(run, &tot);
+        s_start[d] = block_exclusive_scan<uint32_t, NTS>(run, &tot);
         s_run[d] = run;
         if (tile != 0 || !ctl.withhold_first)
-            lb_store(&status[(int64_t)tile * RADIX + d], (tile == 0 ? LB_FLAG_PFX : LB_FLAG_AGG) | tag | run);
+            lb_store(&status[(int64_t)tile * NDIG + d], (tile == 0 ? LB_FLAG_PFX : LB_FLAG_AGG) | tag | run);
     }
     __syncthreads();
 #pragma unroll
@@ -1070,7 +1081,7 @@ __global__ __launch_bounds__(NT) void radix_scatter_lb_kernel(const K* __restric
                 uint64_t w[LB_WIN];
 #pragma unroll
                 for (int q = 0; q < LB_WIN; ++q) {
-                    w[q] = j - q >= 0 ? lb_load(&status[(j - q) * RADIX + d]) : (LB_FLAG_PFX | tag);
+                    w[q] = j - q >= 0 ? lb_load(&status[(j - q) * NDIG + d]) : (LB_FLAG_PFX | tag);
                 }
                 int used = 0;
                 bool done = false, empty = false;
@@ -1090,13 +1101,13 @@ __global__ __launch_bounds__(NT) void radix_scatter_lb_kernel(const K* __restric
                     __builtin_amdgcn_s_sleep(1);
                 }
             }
-            lb_store(&status[(int64_t)tile * RADIX + d], LB_FLAG_PFX | tag | (pre + s_run[d]));
+            lb_store(&status[(int64_t)tile * NDIG + d], LB_FLAG_PFX | tag | (pre + s_run[d]));
         }
         s_goff[d] = gbase[d] + (uint32_t)pre;
     }
     __syncthreads();
     const int64_t cnt_tile = min((int64_t)TILE, n - base);
-    for (int i = threadIdx.x; i < cnt_tile; i += NT) {
+    for (int i = threadIdx.x; i < cnt_tile; i += NTS) {
         const K kk = s_k[i];
         const uint32_t digit = (uint32_t)(kk >> shift) & dmask;
         const int64_t g = (int64_t)s_goff[digit] + (i - (int64_t)s_start[digit]);
