@@ -131,29 +131,6 @@ __device__ inline int hop_sum(uint64_t bits, int64_t r, int M, int row_len, uint
     return pairs;
 }
 
-// Sum over the workgroup, the same in every run: a shuffle tree per wavefront, then the
-// wavefronts in order (two barriers; result in thread 0).
-template <int N>
-__device__ inline void dense_block_sums(double (&v)[N], double (*s)[DT / WAVE]) {
-    const int lane = threadIdx.x & (WAVE - 1), wid = threadIdx.x / WAVE;
-#pragma unroll
-    for (int j = 0; j < N; ++j) {
-#pragma unroll
-        for (int off = WAVE / 2; off > 0; off >>= 1) v[j] += __shfl_xor(v[j], off, WAVE);
-        if (lane == 0) s[j][wid] = v[j];
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-#pragma unroll
-        for (int j = 0; j < N; ++j) {
-            double t = s[j][0];
-            for (int w = 1; w < DT / WAVE; ++w) t += s[j][w];
-            v[j] = t;
-        }
-    }
-    __syncthreads();
-}
-
 // w = (a + b H) v, one thread per row.  DOT: also per-block partials[i][block] of <v|w>.
 template <int R, bool DOT>
 __global__ __launch_bounds__(DT) void dense_apply_kernel(const uint64_t* __restrict__ basis,
@@ -182,7 +159,7 @@ __global__ __launch_bounds__(DT) void dense_apply_kernel(const uint64_t* __restr
     }
     if constexpr (DOT) {
         __shared__ double s_sum[R][DT / WAVE];
-        dense_block_sums<R>(dt, s_sum);
+        block_sums<DT, R>(dt, s_sum);
         if (threadIdx.x == 0)
 #pragma unroll
             for (int i = 0; i < R; ++i) partials[(int64_t)i * gridDim.x + tile] = dt[i];
@@ -221,7 +198,7 @@ __global__ __launch_bounds__(DT) void dense_pullback_kernel(const uint64_t* __re
             ps[R + i] = p.b[i] * (vr * ky[i]);
         }
     }
-    dense_block_sums<2 * R>(ps, s_sum);
+    block_sums<DT, 2 * R>(ps, s_sum);
     if (threadIdx.x == 0)
 #pragma unroll
         for (int i = 0; i < 2 * R; ++i) partials[(int64_t)i * gridDim.x + tile] = ps[i];
@@ -236,7 +213,7 @@ __global__ __launch_bounds__(DT) void dense_dot_kernel(const double* __restrict_
     double ps[R];
 #pragma unroll
     for (int i = 0; i < R; ++i) ps[i] = r < D ? x[r * R + i] * y[r * R + i] : 0.0;
-    dense_block_sums<R>(ps, s_sum);
+    block_sums<DT, R>(ps, s_sum);
     if (threadIdx.x == 0)
 #pragma unroll
         for (int i = 0; i < R; ++i) partials[(int64_t)i * gridDim.x + blockIdx.x] = ps[i];
@@ -306,7 +283,7 @@ __global__ __launch_bounds__(DT) void lanczos_orth_kernel(double* __restrict__ w
         }
         ps[i] = x * x;
     }
-    dense_block_sums<R>(ps, s_sum);
+    block_sums<DT, R>(ps, s_sum);
     if (threadIdx.x == 0)
 #pragma unroll
         for (int i = 0; i < R; ++i) partials[(int64_t)i * gridDim.x + blockIdx.x] = ps[i];

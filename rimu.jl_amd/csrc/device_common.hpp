@@ -83,6 +83,29 @@ __device__ inline void block_sum_n(double (&v)[N], double* scratch) {
     __syncthreads();
 }
 
+// N deterministic workgroup sums at once: a shuffle tree per wavefront, then the wavefronts in
+// order (two barriers whatever N is).  Results valid in thread 0.
+template <int NT, int N>
+__device__ inline void block_sums(double (&v)[N], double (*s)[NT / WAVE]) {
+    const int lane = threadIdx.x & (WAVE - 1), wid = threadIdx.x / WAVE;
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+#pragma unroll
+        for (int off = WAVE / 2; off > 0; off >>= 1) v[j] += __shfl_xor(v[j], off, WAVE);
+        if (lane == 0) s[j][wid] = v[j];
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            double t = s[j][0];
+            for (int w = 1; w < NT / WAVE; ++w) t += s[j][w];
+            v[j] = t;
+        }
+    }
+    __syncthreads();
+}
+
 // Three deterministic workgroup sums at once.  Results valid in thread 0.
 template <int NT>
 __device__ inline void block_sum3(double& a, double& b, double& c) {

@@ -15,6 +15,7 @@
 #include <map>
 #include <mutex>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/rimu_hip.h"
@@ -116,9 +117,9 @@ struct rimu_engine {
     DevBuf<uint64_t> pkeys;
     DevBuf<double> pcoef;
     // overlaps (this engine as the right-hand vector)
-    DevBuf<unsigned char> ov_ops;
-    DevBuf<double> ov_part, ov_out;
-    DevBuf<int64_t> ov_ranges, ov_index;
+    DevBuf<double> ov_part;
+    DevBuf<int64_t> ov_ranges;
+    DevBuf<uint32_t> ov_index;
     DevBuf<int64_t> fix_runs;       // runs to reorder after a sort on the top key bits
     DevBuf<int64_t> bk_rstart, bk_vstart;  // bucket merge: first record / vector entry per bucket
     DevBuf<uint64_t> lb_status;     // look-back radix: status words [pass][tile][digit]
@@ -1047,7 +1048,7 @@ int rimu_engine_destroy(rimu_engine* e) {
     e->rtmp.release(); e->plan_status.release(); e->tile_or.release(); e->tile_and.release(); e->plan_p.release(); e->spawn_p.release();
     e->merge_p.release(); e->terms.release(); e->chunk_sums.release(); e->stats_dev.release(); e->shift_state.release(); e->misc.release();
     e->pkeys.release(); e->pcoef.release();
-    e->ov_ops.release(); e->ov_part.release(); e->ov_out.release(); e->ov_ranges.release(); e->ov_index.release();
+    e->ov_part.release(); e->ov_ranges.release(); e->ov_index.release();
     if (e->h_misc) (void)hipHostFree(e->h_misc);
     if (e->h_stats) (void)hipHostFree(e->h_stats);
     if (e->stream) (void)hipStreamDestroy(e->stream);
@@ -1232,80 +1233,102 @@ int overlaps_impl(rimu_engine* left, rimu_engine* right, const rimu_operator* op
                   double* out) {
     if (left->device != right->device) return fail(RIMU_ERR_ARG, "vectors on different devices");
     const int M = right->hdev.M;
-    std::vector<OpDev> dops((size_t)std::max(nops, 1));
+    DiagOps diag{};
+    int diag_out[OV_MAX_OPS], ham_out[OV_MAX_OPS], nham = 0;  // output columns
+    ModelDev ham[OV_MAX_OPS];
     for (int o = 0; o < nops; ++o) {
-        OpDev d{};
-        d.kind = ops[o].kind;
-        d.param = ops[o].param;
-        d.mix = right->mix;
-        if (d.kind == RIMU_OP_HAMILTONIAN) {
+        const int kind = ops[o].kind, param = ops[o].param;
+        if (kind == RIMU_OP_HAMILTONIAN) {
             if (int rc = check_model(&ops[o].model)) return rc;
-            d.h = to_dev(ops[o].model);
-            if (!same_space(d.h, right->hdev))
+            ham[nham] = to_dev(ops[o].model);
+            if (!same_space(ham[nham], right->hdev))
                 return fail(RIMU_ERR_ARG, "operator Hamiltonian on another address space");
-        } else if (right->hdev.kind == RIMU_MODEL_HUBBARD_REAL_SPACE) {
+            ham_out[nham++] = 1 + o;
+            continue;
+        }
+        if (right->hdev.kind == RIMU_MODEL_HUBBARD_REAL_SPACE) {
             return fail(RIMU_ERR_ARG, "G2RealCorrelator and DensityMatrixDiagonal act on one-component 1D BoseFS vectors");
-        } else if (d.kind == RIMU_OP_G2_REAL) {
-            if (d.param <= -M || d.param >= M) return fail(RIMU_ERR_ARG, "G2RealCorrelator needs |d| < M");
-        } else if (d.kind == RIMU_OP_DENSITY_DIAGONAL) {
-            if (d.param < 1 || d.param > M) return fail(RIMU_ERR_ARG, "DensityMatrixDiagonal mode outside 1..M");
+        } else if (kind == RIMU_OP_G2_REAL) {
+            if (param <= -M || param >= M) return fail(RIMU_ERR_ARG, "G2RealCorrelator needs |d| < M");
+        } else if (kind == RIMU_OP_DENSITY_DIAGONAL) {
+            if (param < 1 || param > M) return fail(RIMU_ERR_ARG, "DensityMatrixDiagonal mode outside 1..M");
         } else {
             return fail(RIMU_ERR_ARG, "unknown operator kind");
         }
-        dops[o] = d;
+        diag.kind[diag.n] = kind;
+        diag.param[diag.n] = param;
+        diag_out[diag.n++] = 1 + o;
     }
     for (int o = 0; o <= nops; ++o) out[o] = 0.0;
     const int64_t Lt = left->len, Lu = right->len;
     if (Lt == 0 || Lu == 0) return RIMU_OK;
     rimu_engine* e = right;
-    const int64_t nb = ceil_div(Lu, OV_TILE);
-    HIP_TRY(e->ov_ops.alloc(sizeof(OpDev) * dops.size()));
-    HIP_TRY(e->ov_part.alloc((size_t)nb * (nops + 1)));
-    HIP_TRY(e->ov_out.alloc(OV_MAX_OPS + 1));
+    const bool shorter = ceil_div(Lu, NT * OV_IPT) < OV_MIN_TILES;
+    const int64_t tile = NT * (shorter ? OV_IPT_SHORT : OV_IPT);
+    const int64_t nb = ceil_div(Lu, tile);
+    const int64_t nbh = std::min<int64_t>(ceil_div(Lu, NT / OV_LANES), OV_HAM_GRID);
+    HIP_TRY(e->ov_part.alloc((size_t)(nb * (1 + diag.n) + nbh * nham)));
     HIP_TRY(e->ov_ranges.alloc(nb + 1));
-    HIP_TRY(hipMemcpyAsync(e->ov_ops.p, dops.data(), sizeof(OpDev) * dops.size(), hipMemcpyHostToDevice,
-                           e->stream));
     const K* tk = (const K*)left->vkeys[left->cur].p;
     const void* tv = left->vvals[left->cur].p;
     const K* uk = (const K*)right->vkeys[right->cur].p;
     const void* uv = right->vvals[right->cur].p;
-    const OpDev* dp = (const OpDev*)e->ov_ops.p;
-    int need_split = 0;
-    for (int o = 0; o < nops; ++o) need_split |= dops[o].kind == RIMU_OP_HAMILTONIAN;
-    // mixed keys are spread evenly over their B bits: neighbours are looked up through an
-    // index of t by the top P bits, about 16 keys per index entry
-    const int64_t* tidx = nullptr;
-    int tsh = 0;
     hipEvent_t ev{};
     e->timer.begin("overlap", e->stream, &ev);
-    if (need_split && right->mix.on && Lt >= OV_INDEX_MIN) {
+    overlap_ranges_kernel<K><<<ceil_div(nb + 1, NT), NT, 0, e->stream>>>(tk, Lt, uk, tile, nb, e->ov_ranges.p);
+    // mixed keys are spread evenly over their B bits: neighbours are looked up through an
+    // index of t by the top P bits, one or two keys per index entry
+    const uint32_t* tidx = nullptr;
+    int tsh = 0;
+    if (nham > 0 && right->mix.on && Lt >= OV_INDEX_MIN && Lt < (int64_t)UINT32_MAX) {
         const int B = right->hdev.B;
-        int P = (int)std::floor(std::log2((double)Lt / 16.0));
+        int P = (int)std::floor(std::log2((double)Lt));
         P = std::max(1, std::min({P, OV_INDEX_MAX_BITS, B}));
         tsh = B - P;
         HIP_TRY(e->ov_index.alloc(((size_t)1 << P) + 1));
         overlap_index_kernel<K><<<ceil_div(Lt + 1, NT), NT, 0, e->stream>>>(tk, Lt, B, P, e->ov_index.p);
         tidx = e->ov_index.p;
     }
-    overlap_ranges_kernel<K><<<ceil_div(nb + 1, NT), NT, 0, e->stream>>>(tk, Lt, uk, nb, e->ov_ranges.p);
-    if (left->int_vals && right->int_vals)
-        overlap_kernel<K, int64_t, int64_t><<<nb, NT, 0, e->stream>>>(tk, (const int64_t*)tv, Lt, uk,
-            (const int64_t*)uv, Lu, dp, nops, M, e->ov_ranges.p, need_split, tidx, tsh, e->ov_part.p);
-    else if (left->int_vals)
-        overlap_kernel<K, int64_t, double><<<nb, NT, 0, e->stream>>>(tk, (const int64_t*)tv, Lt, uk,
-            (const double*)uv, Lu, dp, nops, M, e->ov_ranges.p, need_split, tidx, tsh, e->ov_part.p);
-    else if (right->int_vals)
-        overlap_kernel<K, double, int64_t><<<nb, NT, 0, e->stream>>>(tk, (const double*)tv, Lt, uk,
-            (const int64_t*)uv, Lu, dp, nops, M, e->ov_ranges.p, need_split, tidx, tsh, e->ov_part.p);
-    else
-        overlap_kernel<K, double, double><<<nb, NT, 0, e->stream>>>(tk, (const double*)tv, Lt, uk,
-            (const double*)uv, Lu, dp, nops, M, e->ov_ranges.p, need_split, tidx, tsh, e->ov_part.p);
+    auto launch = [&](auto* t, auto* u) {
+        using VT = std::remove_const_t<std::remove_pointer_t<decltype(t)>>;
+        using VU = std::remove_const_t<std::remove_pointer_t<decltype(u)>>;
+        if (shorter)
+            overlap_kernel<K, VT, VU, OV_IPT_SHORT><<<nb, NT, 0, e->stream>>>(tk, t, Lt, uk, u, Lu, diag, right->mix, M,
+                                                                              e->ov_ranges.p, e->ov_part.p);
+        else
+            overlap_kernel<K, VT, VU, OV_IPT><<<nb, NT, 0, e->stream>>>(tk, t, Lt, uk, u, Lu, diag, right->mix, M,
+                                                                        e->ov_ranges.p, e->ov_part.p);
+        for (int q = 0; q < nham; ++q) {
+            double* part = e->ov_part.p + nb * (1 + diag.n) + nbh * q;
+            if (ham[q].kind == RIMU_MODEL_HUBBARD_REAL_SPACE)
+                overlap_ham_kernel<true, K, VT, VU><<<nbh, NT, 0, e->stream>>>(ham[q], right->mix, tk, t, Lt, uk, u, Lu,
+                                                                              tidx, tsh, part);
+            else
+                overlap_ham_kernel<false, K, VT, VU><<<nbh, NT, 0, e->stream>>>(ham[q], right->mix, tk, t, Lt, uk, u, Lu,
+                                                                               tidx, tsh, part);
+        }
+    };
+    if (left->int_vals && right->int_vals) launch((const int64_t*)tv, (const int64_t*)uv);
+    else if (left->int_vals) launch((const int64_t*)tv, (const double*)uv);
+    else if (right->int_vals) launch((const double*)tv, (const int64_t*)uv);
+    else launch((const double*)tv, (const double*)uv);
     e->timer.end(e->stream);
     HIP_TRY(hipGetLastError());
-    overlap_final_kernel<<<nops + 1, NT, 0, e->stream>>>(e->ov_part.p, nb, e->ov_out.p);
+    OvColumns cols{};
+    cols.count[0] = nb;
+    for (int q = 0; q < diag.n; ++q) {
+        cols.first[diag_out[q]] = nb * (1 + q);
+        cols.count[diag_out[q]] = nb;
+    }
+    for (int q = 0; q < nham; ++q) {
+        cols.first[ham_out[q]] = nb * (1 + diag.n) + nbh * q;
+        cols.count[ham_out[q]] = nbh;
+    }
+    static_assert(1 + OV_MAX_OPS <= 16, "the pinned statistics hold the results");
+    overlap_final_kernel<<<nops + 1, NT, 0, e->stream>>>(e->ov_part.p, cols, e->h_stats);
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipMemcpyAsync(out, e->ov_out.p, sizeof(double) * (nops + 1), hipMemcpyDeviceToHost, e->stream));
     HIP_TRY(hipStreamSynchronize(e->stream));
+    std::copy(e->h_stats, e->h_stats + nops + 1, out);
     e->timer.collect();
     return RIMU_OK;
 }
