@@ -511,36 +511,38 @@ int merge_into(rimu_engine* e, const StepArgs& a, const K* ak, const V* av, int6
 }
 
 // Stored keys from addresses (forward) or addresses from stored keys, in place.
-__global__ __launch_bounds__(NT) void mix_keys_kernel(uint64_t* __restrict__ keys, int64_t n, KeyMix m,
-                                                      int forward) {
+template <class K>
+__global__ __launch_bounds__(NT) void mix_keys_kernel(K* __restrict__ keys, int64_t n, KeyMix m, int forward) {
     const int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x;
     if (i >= n) return;
-    keys[i] = forward ? mix_bits<uint64_t>(m, keys[i]) : unmix_bits<uint64_t>(m, keys[i]);
+    keys[i] = forward ? mix_bits<K>(m, keys[i]) : unmix_bits<K>(m, keys[i]);
 }
 
 // Vectors of this many entries or more are reordered between address order and stored-key
-// order on the device (one-word keys, when the spawn buffers can hold them).
-constexpr int64_t DEVICE_REORDER_MIN = 1 << 16;
+// order on the device, when the spawn buffers can hold them.  Reading out 50,000 two-word
+// entries takes 5.2 ms with the host's sort and 0.9 ms with the device's, 5e6 take 650 and 8 ms;
+// a few hundred entries cost the host less than the launches of a sort.
+constexpr int64_t DEVICE_REORDER_MIN = 1024;
 
 bool device_reorder(const rimu_engine* e, int64_t n) {
-    return e->mix.on && e->kw == 1 && n >= DEVICE_REORDER_MIN && n <= e->max_spawns;
+    return e->mix.on && n >= DEVICE_REORDER_MIN && n <= e->max_spawns;
 }
 
 // n (key, value) pairs that fill() puts into spawn buffer 0: turn the keys into stored keys
 // (forward) or back into addresses, sort the pairs on the key and leave them in spawn buffer
 // *result.  A radix look-back that gives up (the sort buffers then hold no list) makes it
 // fill and sort again with the per-pass sort.
-template <class Fill>
+template <class K, class Fill>
 int reorder_on_device(rimu_engine* e, int64_t n, int forward, int* result, Fill&& fill) {
     const int saved = e->radix_mode;
     int rc = RIMU_OK;
     for (int attempt = 0; attempt < 2; ++attempt) {
         if ((rc = fill())) break;
-        mix_keys_kernel<<<ceil_div(n, NT), NT, 0, e->stream>>>(e->skeys[0].p, n, e->mix, forward);
+        mix_keys_kernel<K><<<ceil_div(n, NT), NT, 0, e->stream>>>((K*)e->skeys[0].p, n, e->mix, forward);
         if (hipGetLastError() != hipSuccess) { rc = fail(RIMU_ERR_HIP, "mix_keys_kernel launch"); break; }
         int* flags = &((rimu_engine::Misc*)e->misc.p)->flags;
         if (hipMemsetAsync(flags, 0, sizeof(int), e->stream) != hipSuccess) { rc = fail(RIMU_ERR_HIP, "memset"); break; }
-        if ((rc = radix_sort<uint64_t, uint64_t>(e, n, e->hdev.B, ~(u128)0, 0, result))) break;
+        if ((rc = radix_sort<K, uint64_t>(e, n, e->hdev.B, ~(u128)0, 0, result))) break;
         int h_flags = 0;
         if (hipMemcpyAsync(&h_flags, flags, sizeof(int), hipMemcpyDeviceToHost, e->stream) != hipSuccess ||
             hipStreamSynchronize(e->stream) != hipSuccess) { rc = fail(RIMU_ERR_HIP, "flags"); break; }
@@ -550,6 +552,11 @@ int reorder_on_device(rimu_engine* e, int64_t n, int forward, int* result, Fill&
     }
     e->radix_mode = saved;
     return rc;
+}
+template <class Fill>
+int reorder_on_device(rimu_engine* e, int64_t n, int forward, int* result, Fill&& fill) {
+    return e->kw == 2 ? reorder_on_device<u128>(e, n, forward, result, fill)
+                      : reorder_on_device<uint64_t>(e, n, forward, result, fill);
 }
 
 // Bucket merge (bucket_kernels.hpp) of S spawn records sorted on their top T key bits with
@@ -1110,12 +1117,12 @@ int rimu_vector_upload(rimu_engine* e, const uint64_t* keys, const void* vals, i
     if (on_device && m > 0) {
         int sorted = 0;
         if (int rc = reorder_on_device(e, m, 1, &sorted, [&]() -> int {
-                HIP_TRY(hipMemcpyAsync(e->skeys[0].p, k.data(), m * 8, hipMemcpyHostToDevice, e->stream));
+                HIP_TRY(hipMemcpyAsync(e->skeys[0].p, k.data(), m * 8 * kw, hipMemcpyHostToDevice, e->stream));
                 HIP_TRY(hipMemcpyAsync(e->svals[0].p, e->int_vals ? (const void*)vi.data() : (const void*)vd.data(),
                                        m * 8, hipMemcpyHostToDevice, e->stream));
                 return RIMU_OK;
             })) return rc;
-        HIP_TRY(hipMemcpyAsync(e->vkeys[e->cur].p, e->skeys[sorted].p, m * 8, hipMemcpyDeviceToDevice, e->stream));
+        HIP_TRY(hipMemcpyAsync(e->vkeys[e->cur].p, e->skeys[sorted].p, m * 8 * kw, hipMemcpyDeviceToDevice, e->stream));
         HIP_TRY(hipMemcpyAsync(e->vvals[e->cur].p, e->svals[sorted].p, m * 8, hipMemcpyDeviceToDevice, e->stream));
     } else if (m > 0) {
         HIP_TRY(hipMemcpyAsync(e->vkeys[e->cur].p, k.data(), m * 8 * kw, hipMemcpyHostToDevice, e->stream));
@@ -1140,13 +1147,13 @@ int rimu_vector_download(rimu_engine* e, uint64_t* keys, void* vals, int64_t cap
     if (device_reorder(e, e->len)) {  // addresses back and address order on the device
         int sorted = 0;
         if (int rc = reorder_on_device(e, e->len, 0, &sorted, [&]() -> int {
-                HIP_TRY(hipMemcpyAsync(e->skeys[0].p, e->vkeys[e->cur].p, e->len * 8, hipMemcpyDeviceToDevice,
-                                       e->stream));
+                HIP_TRY(hipMemcpyAsync(e->skeys[0].p, e->vkeys[e->cur].p, e->len * 8 * e->kw,
+                                       hipMemcpyDeviceToDevice, e->stream));
                 HIP_TRY(hipMemcpyAsync(e->svals[0].p, e->vvals[e->cur].p, e->len * 8, hipMemcpyDeviceToDevice,
                                        e->stream));
                 return RIMU_OK;
             })) return rc;
-        HIP_TRY(hipMemcpyAsync(keys, e->skeys[sorted].p, e->len * 8, hipMemcpyDeviceToHost, e->stream));
+        HIP_TRY(hipMemcpyAsync(keys, e->skeys[sorted].p, e->len * 8 * e->kw, hipMemcpyDeviceToHost, e->stream));
         HIP_TRY(hipMemcpyAsync(vals, e->svals[sorted].p, e->len * 8, hipMemcpyDeviceToHost, e->stream));
         HIP_TRY(hipStreamSynchronize(e->stream));
         return RIMU_OK;
