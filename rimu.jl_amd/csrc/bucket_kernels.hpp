@@ -522,18 +522,18 @@ __global__ __launch_bounds__(BK_NT, 2 * BkShape<IPT>::WG_PER_CU) void bucket_mer
 }
 
 // Survivors of bucket b move from its slot range [rstart[b] + vstart[b], ...) to
-// [offs[b], offs[b + 1]) (offs: exclusive scan of the bucket counts; offs[nbuckets] is the new
-// length).  A new length above cap writes nothing and raises FLAG_VECTOR_OVERFLOW.
+// their final place (tile_place of the bucket counts).  A new length above cap writes nothing and raises FLAG_VECTOR_OVERFLOW.
 template <class V, int IPT>
 __global__ __launch_bounds__(NT) void bucket_compact_kernel(const uint64_t* __restrict__ slot_k,
                                                             const V* __restrict__ slot_v,
                                                             const int64_t* __restrict__ rstart,
                                                             const int64_t* __restrict__ vstart,
-                                                            const int64_t* __restrict__ offs, int64_t nbuckets,
+                                                            const int64_t* __restrict__ offs, int64_t nbuckets, int raw,
                                                             uint64_t* __restrict__ ok, V* __restrict__ ov,
                                                             int64_t cap, int64_t* total_out, int* flags) {
     const int64_t b = blockIdx.x;
-    const int64_t total = offs[nbuckets];
+    const TilePlace at = tile_place(offs, nbuckets, b, raw);
+    const int64_t total = at.total;
     if (total > cap) {
         if (b == 0 && threadIdx.x == 0) {
             atomicOr(flags, FLAG_VECTOR_OVERFLOW);
@@ -542,8 +542,8 @@ __global__ __launch_bounds__(NT) void bucket_compact_kernel(const uint64_t* __re
         return;
     }
     if (b == 0 && threadIdx.x == 0) *total_out = total;
-    const int64_t off = offs[b];
-    const int n = (int)(offs[b + 1] - off);
+    const int64_t off = at.off;
+    const int n = (int)at.n;
     const int64_t src = rstart[b] + vstart[b];
     constexpr int CPT = BkShape<IPT>::CAP / NT;
     uint64_t k[CPT];

@@ -111,7 +111,7 @@ struct rimu_engine {
     DevBuf<uint64_t> plan_status, tile_or, tile_and;
     DevBuf<int64_t> tile_first, splits, tile_cnt;
     DevBuf<uint64_t> prevk, slot_k, slot_v;  // merge: per-tile survivor slots (values as raw 8 bytes)
-    DevBuf<double> plan_p, spawn_p, merge_p, terms, stats_dev, chunk_sums;
+    DevBuf<double> plan_p, spawn_p, merge_p, terms, chunk_sums;
     DevBuf<unsigned char> misc;  // counters and totals (see layout below)
     // projector
     DevBuf<uint64_t> pkeys;
@@ -130,8 +130,9 @@ struct rimu_engine {
     int64_t W_prev = 0, S_prev = 0; // spawn attempts and records of the last step
     uint32_t lb_spin_limit = LB_SPIN_LIMIT;  // bound of every look-back wait
     int lb_withhold = 0;            // test of the give-up path (rimu_engine_set_lookback)
-    DevBuf<uint32_t> lb_hist;       // look-back radix: digit bases [pass][digit], tile counters
-    DevBuf<uint32_t> lb_part;       // look-back radix: digit counts [row][pass][digit]
+    DevBuf<uint32_t> lb_hist;       // look-back radix: digit bases [pass][digit]
+    DevBuf<uint32_t> lb_part;       // look-back radix: tile counters, digit counts [row][pass][digit]
+    int64_t lb_cleared = 0;         // words of lb_part that this step has cleared already
     int64_t np = 0, nh = 0;
     // device shift update (rimu_engine_set_shift_update): shift_state holds (shift, pnorm)
     // twice; a step reads half shift_cur and writes the other, and a kept step flips shift_cur
@@ -291,13 +292,15 @@ StepArgs make_args(rimu_engine* e, int64_t step, double shift, double dtau, doub
     return a;
 }
 
-// exclusive scan of n int64 values in place (data has n entries)
-int scan_inplace_i64(rimu_engine* e, int64_t* data, int64_t n) {
-    const int64_t tiles = ceil_div(n, SCAN_TILE);
+// exclusive scan of n counts in place, their total in data[n] (data has n + 1 entries)
+int scan_counts(rimu_engine* e, int64_t* data, int64_t n) {
+    const int64_t tiles = ceil_div(n + 1, SCAN_TILE);
     HIP_TRY(e->scan_tmp.alloc(tiles + 1));
-    scan_tiles_kernel<int64_t><<<tiles, NT, 0, e->stream>>>(data, data, n, e->scan_tmp.p);
-    scan_sums_kernel<int64_t><<<1, 1024, 0, e->stream>>>(e->scan_tmp.p, tiles, nullptr);
-    scan_add_kernel<int64_t><<<tiles, NT, 0, e->stream>>>(data, n, e->scan_tmp.p);
+    scan_tiles_kernel<int64_t><<<tiles, NT, 0, e->stream>>>(data, data, n + 1, n, e->scan_tmp.p);
+    if (tiles > 1) {
+        scan_sums_kernel<int64_t><<<1, 1024, 0, e->stream>>>(e->scan_tmp.p, tiles, nullptr);
+        scan_add_kernel<int64_t><<<tiles, NT, 0, e->stream>>>(data, n + 1, e->scan_tmp.p);
+    }
     HIP_TRY(hipGetLastError());
     return RIMU_OK;
 }
@@ -305,7 +308,7 @@ int scan_inplace_i64(rimu_engine* e, int64_t* data, int64_t n) {
 int scan_u32(rimu_engine* e, const uint32_t* in, uint32_t* out, int64_t n) {
     const int64_t tiles = ceil_div(n, SCAN_TILE);
     HIP_TRY(e->rtmp.alloc(tiles + 1));
-    scan_tiles_kernel<uint32_t><<<tiles, NT, 0, e->stream>>>(in, out, n, e->rtmp.p);
+    scan_tiles_kernel<uint32_t><<<tiles, NT, 0, e->stream>>>(in, out, n, n, e->rtmp.p);
     scan_sums_kernel<uint32_t><<<1, 1024, 0, e->stream>>>(e->rtmp.p, tiles, nullptr);
     scan_add_kernel<uint32_t><<<tiles, NT, 0, e->stream>>>(out, n, e->rtmp.p);
     HIP_TRY(hipGetLastError());
@@ -325,6 +328,13 @@ int radix_sort_lb(rimu_engine* e, int64_t n, int nbits, u128 varying, int in, in
 // of a sort with 512 digits would outgrow the arrays laid out for 256 (rimu_annihilate_noalloc).
 bool nine_bit_digits(int nbits, int lo) {
     return nbits - lo <= 36 && ceil_div(nbits - lo, 9) < ceil_div(nbits - lo, RADIX_BITS);
+}
+
+// Words of lb_part that a look-back sort of key bits [lo, nbits) uses: tile ids, digit counts.
+template <class K>
+int64_t lb_words(int nbits, int lo) {
+    const int rb = sizeof(K) == 8 && nine_bit_digits(nbits, lo) ? 9 : RADIX_BITS;
+    return MAX_PASSES + (int64_t)HIST_ROWS * ceil_div(nbits - lo, rb) * (1 << rb);
 }
 
 template <class K, class V>
@@ -388,8 +398,7 @@ int radix_sort_lb(rimu_engine* e, int64_t n, int nbits, u128 varying, int in, in
     if (n > (int64_t)RLB_VALUE) return fail(RIMU_ERR_CAPACITY, "radix sort of 2^32 or more records");
     const int64_t tiles = ceil_div(n, sort_tile<K>::value);
     const size_t need = (size_t)ps.n * tiles * NDIG;
-    HIP_TRY(e->lb_hist.alloc((size_t)ps.n * NDIG + MAX_PASSES));
-    uint32_t* counters = e->lb_hist.p + (int64_t)ps.n * NDIG;  // tile ids (two-word keys)
+    HIP_TRY(e->lb_hist.alloc((size_t)ps.n * NDIG));
     int* flags = &((rimu_engine::Misc*)e->misc.p)->flags;
     hipEvent_t ev{};
     if (need > e->lb_status.n || e->lb_epoch >= RLB_EPOCH_MAX) {  // epoch 0: cleared words
@@ -399,14 +408,19 @@ int radix_sort_lb(rimu_engine* e, int64_t n, int nbits, u128 varying, int in, in
     }
     const uint32_t epoch = ++e->lb_epoch;
     e->timer.begin("radix_count", e->stream, &ev);
-    HIP_TRY(hipMemsetAsync(counters, 0, sizeof(uint32_t) * MAX_PASSES, e->stream));
     const int copies = hist_all_copies(ps.n);
     const int hblocks = (int)std::min<int64_t>(tiles, HIST_ALL_BLOCKS);
-    HIP_TRY(e->lb_part.alloc((size_t)HIST_ROWS * ps.n * NDIG));
-    HIP_TRY(hipMemsetAsync(e->lb_part.p, 0, sizeof(uint32_t) * HIST_ROWS * ps.n * NDIG, e->stream));
+    const int64_t words = MAX_PASSES + (int64_t)HIST_ROWS * ps.n * NDIG;  // tile ids, then digit counts
+    if (e->lb_cleared < words) {
+        HIP_TRY(e->lb_part.alloc(words));
+        HIP_TRY(hipMemsetAsync(e->lb_part.p, 0, sizeof(uint32_t) * words, e->stream));
+    }
+    e->lb_cleared = 0;
+    uint32_t* counters = e->lb_part.p;
+    uint32_t* part = e->lb_part.p + MAX_PASSES;
     radix_hist_all_kernel<K, RB><<<hblocks, NT, sizeof(uint32_t) * ps.n * copies * (NDIG + 1), e->stream>>>(
-        (const K*)e->skeys[src].p, Count{n, n_dev, n}, flags, ps, copies, e->lb_part.p);
-    radix_hist_base_kernel<RB><<<ps.n, NDIG, 0, e->stream>>>(e->lb_part.p, ps.n, e->lb_hist.p);
+        (const K*)e->skeys[src].p, Count{n, n_dev, n}, flags, ps, copies, part);
+    radix_hist_base_kernel<RB><<<ps.n, NDIG, 0, e->stream>>>(part, ps.n, e->lb_hist.p);
     e->timer.end(e->stream);
     for (int p = 0; p < ps.n; ++p) {
         e->timer.begin("radix_scatter", e->stream, &ev);
@@ -485,7 +499,6 @@ int merge_into(rimu_engine* e, const StepArgs& a, const K* ak, const V* av, int6
     HIP_TRY(e->tile_cnt.alloc(nt + 1));
     HIP_TRY(e->slot_k.alloc((size_t)nt * TILE * KW));
     HIP_TRY(e->slot_v.alloc((size_t)nt * TILE));
-    HIP_TRY(hipMemsetAsync(e->tile_cnt.p + nt, 0, sizeof(int64_t), e->stream));
     merge_split_kernel<K><<<ceil_div(nt + 1, NT), NT, 0, e->stream>>>(
         ak, Count{S, S_dev, S}, bk, L, TILE, nt, init ? (K)~class_bit<K>() : (K)~(K)0, e->splits.p, (K*)e->prevk.p);
     hipEvent_t ev{};
@@ -502,9 +515,11 @@ int merge_into(rimu_engine* e, const StepArgs& a, const K* ak, const V* av, int6
     e->timer.end(e->stream);
     HIP_TRY(hipGetLastError());
     e->timer.begin("compact", e->stream, &ev);
-    if (int rc = scan_inplace_i64(e, e->tile_cnt.p, nt + 1)) return rc;
+    const bool raw = nt <= COMPACT_RAW_MAX;
+    if (!raw)
+        if (int rc = scan_counts(e, e->tile_cnt.p, nt)) return rc;
     compact_kernel<K, V, merge_ipt<K>::value, FLAG_VECTOR_OVERFLOW><<<nt, NT, 0, e->stream>>>(
-        (const K*)e->slot_k.p, (const V*)e->slot_v.p, e->tile_cnt.p, nt, ok, ov, cap, &dm->L_new, &dm->flags);
+        (const K*)e->slot_k.p, (const V*)e->slot_v.p, e->tile_cnt.p, nt, raw, ok, ov, cap, &dm->L_new, &dm->flags);
     e->timer.end(e->stream);
     HIP_TRY(hipGetLastError());
     return RIMU_OK;
@@ -598,6 +613,13 @@ BucketCut bucket_cut(int64_t S, int64_t L, int B, int min_ipt) {
     return cut;
 }
 
+// Lowest key bit a step's sort covers: the bucket bits, the top bits of wide mixed keys, or all.
+int sort_from(const rimu_engine* e, const BucketCut& cut) {
+    const int B = e->hdev.B;
+    if (cut.T > 0) return B - cut.T;
+    return e->mix.on && B > e->sort_bits ? B - e->sort_bits : 0;
+}
+
 template <class V, int IPT>
 int bucket_merge_shape(rimu_engine* e, const StepArgs& a, const uint64_t* ak, const V* av, int64_t S,
                       const uint64_t* bk, const V* bv, const V* bo, int64_t L, int T, uint64_t* ok, V* ov,
@@ -616,7 +638,6 @@ int bucket_merge_shape(rimu_engine* e, const StepArgs& a, const uint64_t* ak, co
     bucket_bounds_kernel<<<ceil_div(2 * nbk + 2, NT), NT, 0, e->stream>>>(ak, Count{S, S_dev, S}, bk, L, B - T, nbk,
                                                                           e->bk_rstart.p, e->bk_vstart.p);
     e->timer.end(e->stream);
-    HIP_TRY(hipMemsetAsync(e->tile_cnt.p + nbk, 0, sizeof(int64_t), e->stream));
     if (e->n_cu == 0) {
         HIP_TRY(hipDeviceGetAttribute(&e->n_cu, hipDeviceAttributeMultiprocessorCount, e->device));
         if (e->n_cu <= 0) e->n_cu = 1;
@@ -634,10 +655,12 @@ int bucket_merge_shape(rimu_engine* e, const StepArgs& a, const uint64_t* ak, co
     e->timer.end(e->stream);
     HIP_TRY(hipGetLastError());
     e->timer.begin("compact", e->stream, &ev);
-    if (int rc = scan_inplace_i64(e, e->tile_cnt.p, nbk + 1)) return rc;
+    const bool raw = nbk <= COMPACT_RAW_MAX;
+    if (!raw)
+        if (int rc = scan_counts(e, e->tile_cnt.p, nbk)) return rc;
     bucket_compact_kernel<V, IPT><<<nbk, NT, 0, e->stream>>>(e->slot_k.p, (const V*)e->slot_v.p, e->bk_rstart.p,
-                                                        e->bk_vstart.p, e->tile_cnt.p, nbk, ok, ov, cap,
-                                                        &dm->L_new, &dm->flags);
+                                                             e->bk_vstart.p, e->tile_cnt.p, nbk, raw, ok, ov, cap,
+                                                             &dm->L_new, &dm->flags);
     e->timer.end(e->stream);
     HIP_TRY(hipGetLastError());
     return RIMU_OK;
@@ -677,8 +700,6 @@ int step_impl(rimu_engine* e, int64_t step, double shift, double dtau, double bo
     rimu_engine::Misc* dm = (rimu_engine::Misc*)e->misc.p;
     hipEvent_t ev{};
 
-    HIP_TRY(hipMemsetAsync(dm, 0, sizeof(rimu_engine::Misc), e->stream));
-
     // Grids of the spawn, sort and merge kernels: sized from the counts of this step, read back
     // after the plan and after the spawn (synchronous step), or -- once a step has run -- from
     // the last step's counts with headroom, the kernels reading this step's counts from device
@@ -699,7 +720,15 @@ int step_impl(rimu_engine* e, int64_t step, double shift, double dtau, double bo
     const int64_t plan_tiles = ceil_div(L + 1, PLAN_TILE);
     HIP_TRY(e->plan_p.alloc((size_t)plan_tiles * 6));
     HIP_TRY(e->plan_status.alloc(plan_tiles));
-    HIP_TRY(hipMemsetAsync(e->plan_status.p, 0, sizeof(uint64_t) * plan_tiles, e->stream));
+    // tile ids and digit counts of the sort to come (a synchronous step's sort clears its own)
+    const int64_t sort_words = spec ? lb_words<K>(nbits, sort_from(e, cut)) : 0;
+    HIP_TRY(e->lb_part.alloc(sort_words));
+    e->lb_cleared = sort_words;
+    const ClearSet clear{{{(uint32_t*)dm, (int64_t)sizeof(rimu_engine::Misc) / 4},
+                          {(uint32_t*)e->plan_status.p, 2 * plan_tiles},
+                          {e->lb_part.p, sort_words}}};
+    static_assert(sizeof(rimu_engine::Misc) % 4 == 0 && sizeof(rimu_engine::Misc) / 4 <= WAVE, "cleared and copied as words");
+    clear_kernel<<<std::min<int64_t>(ceil_div(2 * plan_tiles + sort_words, NT), 256), NT, 0, e->stream>>>(clear);
     if (spec) HIP_TRY(e->tile_first.alloc(ceil_div(W_cap, SPAWN_TILE) + 1));
     const int64_t tf_cap = (int64_t)e->tile_first.n;
     e->timer.begin("plan", e->stream, &ev);
@@ -750,7 +779,6 @@ int step_impl(rimu_engine* e, int64_t step, double shift, double dtau, double bo
             HIP_TRY(e->slot_k.alloc((size_t)spawn_tiles * SPAWN_TILE * KW));
             HIP_TRY(e->slot_v.alloc((size_t)spawn_tiles * SPAWN_TILE));
             HIP_TRY(e->tile_cnt.alloc(spawn_tiles + 1));
-            HIP_TRY(hipMemsetAsync(e->tile_cnt.p + spawn_tiles, 0, sizeof(int64_t), e->stream));
             sk = (K*)e->slot_k.p;
             sv = (V*)e->slot_v.p;
         }
@@ -779,9 +807,11 @@ int step_impl(rimu_engine* e, int64_t step, double shift, double dtau, double bo
                                                           spawn_tiles, (K*)&dm->key_or, (K*)&dm->key_and);
         if (!dense) {
             e->timer.begin("spawn_compact", e->stream, &ev);
-            if (int rc = scan_inplace_i64(e, e->tile_cnt.p, spawn_tiles + 1)) return rc;
+            const bool raw = spawn_tiles <= COMPACT_RAW_MAX;
+            if (!raw)
+                if (int rc = scan_counts(e, e->tile_cnt.p, spawn_tiles)) return rc;
             compact_kernel<K, V, SPAWN_ITEMS, FLAG_SPAWN_OVERFLOW><<<spawn_tiles, NT, 0, e->stream>>>(
-                (const K*)e->slot_k.p, (const V*)e->slot_v.p, e->tile_cnt.p, spawn_tiles, (K*)e->skeys[0].p,
+                (const K*)e->slot_k.p, (const V*)e->slot_v.p, e->tile_cnt.p, spawn_tiles, raw, (K*)e->skeys[0].p,
                 (V*)e->svals[0].p, e->max_spawns, &dm->S, &dm->flags);
             e->timer.end(e->stream);
         }
@@ -842,12 +872,14 @@ int step_impl(rimu_engine* e, int64_t step, double shift, double dtau, double bo
 
     // 5. projections and statistics
     auto finish = [&]() -> int {
-        if (e->np + e->nh > 0) {
-            project_kernel<K, V><<<ceil_div(e->np + e->nh, NT), NT, 0, e->stream>>>(
-                (const K*)e->vkeys[nxt].p, (const V*)e->vvals[nxt].p, &dm->L_new, (const K*)e->pkeys.p, e->pcoef.p,
-                e->np + e->nh, e->terms.p);
-            HIP_TRY(hipGetLastError());
-        }
+        ProjectArgs pa{};
+        pa.keys = e->vkeys[nxt].p;
+        pa.vals = e->vvals[nxt].p;
+        pa.len = &dm->L_new;
+        pa.pk = e->pkeys.p;
+        pa.pc = e->pcoef.p;
+        pa.np = e->np + e->nh;
+        pa.terms = e->terms.p;
         PartialSet ps{};
         // plan partials rows: deaths, clones, zombies, exact, inexact, attempts
         const int plan_map[6] = {4, 5, 6, 1, 2, 0};
@@ -865,7 +897,6 @@ int step_impl(rimu_engine* e, int64_t step, double shift, double dtau, double bo
         ps.n[10] = e->np;
         ps.p[11] = e->terms.p + e->np;
         ps.n[11] = e->nh;
-        partial_sums_kernel<<<dim3(PARTIAL_BLOCKS, NSTAT), NT, 0, e->stream>>>(ps, e->chunk_sums.p);
         ShiftUpdate su{};
         if (e->shift_mode) {
             su.in = a.shift_dev;
@@ -875,11 +906,17 @@ int step_impl(rimu_engine* e, int64_t step, double shift, double dtau, double bo
             su.zeta = e->dlu_zeta;
             su.xi = e->dlu_xi;
         }
-        finalize_kernel<<<1, 64, 0, e->stream>>>(e->chunk_sums.p, PARTIAL_BLOCKS, e->stats_dev.p, su);
+        const StepOut so{e->h_stats, (const uint32_t*)dm, (uint32_t*)e->h_misc, (int)(sizeof(rimu_engine::Misc) / 4)};
+        bool small = true;
+        for (int j = 0; j < NSTAT; ++j) small = small && ps.n[j] <= STATS_SMALL;
+        if (small) {
+            stats_small_kernel<K, V><<<1, STATS_NT, 0, e->stream>>>(ps, pa, so, su);
+        } else {
+            if (pa.np > 0) project_kernel<K, V><<<ceil_div(pa.np, NT), NT, 0, e->stream>>>(pa);
+            partial_sums_kernel<<<dim3(PARTIAL_BLOCKS, NSTAT), NT, 0, e->stream>>>(ps, e->chunk_sums.p);
+            finalize_kernel<<<1, STATS_NT, 0, e->stream>>>(e->chunk_sums.p, so, su);
+        }
         HIP_TRY(hipGetLastError());
-        HIP_TRY(hipMemcpyAsync(e->h_stats, e->stats_dev.p, (NSTAT + 2) * sizeof(double), hipMemcpyDeviceToHost,
-                               e->stream));
-        HIP_TRY(hipMemcpyAsync(e->h_misc, dm, sizeof(rimu_engine::Misc), hipMemcpyDeviceToHost, e->stream));
         HIP_TRY(hipStreamSynchronize(e->stream));
         e->timer.collect();
         return RIMU_OK;
@@ -1028,7 +1065,6 @@ int rimu_engine_create(const rimu_model* model, const rimu_style* style, uint64_
     if ((err = e->dvals.alloc(max_entries * 8)) != hipSuccess) return bad("diagonal values", err);
     if ((err = e->woff.alloc(max_entries + 1)) != hipSuccess) return bad("work offsets", err);
     if ((err = e->misc.alloc(sizeof(rimu_engine::Misc))) != hipSuccess) return bad("misc", err);
-    if ((err = e->stats_dev.alloc(16)) != hipSuccess) return bad("stats", err);
     if ((err = e->terms.alloc(16)) != hipSuccess) return bad("terms", err);
     if ((err = e->chunk_sums.alloc(PARTIAL_BLOCKS * NSTAT)) != hipSuccess) return bad("chunk sums", err);
     if ((err = e->spawn_p.alloc(16)) != hipSuccess) return bad("partials", err);
@@ -1053,7 +1089,7 @@ int rimu_engine_destroy(rimu_engine* e) {
     e->prevk.release(); e->slot_k.release(); e->slot_v.release();
     e->dvals.release(); e->woff.release(); e->scan_tmp.release(); e->rcounts.release(); e->rchunks.release();
     e->rtmp.release(); e->plan_status.release(); e->tile_or.release(); e->tile_and.release(); e->plan_p.release(); e->spawn_p.release();
-    e->merge_p.release(); e->terms.release(); e->chunk_sums.release(); e->stats_dev.release(); e->shift_state.release(); e->misc.release();
+    e->merge_p.release(); e->terms.release(); e->chunk_sums.release(); e->shift_state.release(); e->misc.release();
     e->pkeys.release(); e->pcoef.release();
     e->ov_part.release(); e->ov_ranges.release(); e->ov_index.release();
     if (e->h_misc) (void)hipHostFree(e->h_misc);
@@ -1602,9 +1638,9 @@ constexpr size_t NA_KEYS0 = 0, NA_KEYS1 = NA_REC, NA_VALS0 = 2 * NA_REC, NA_VALS
 constexpr size_t NA_STATUS = 4 * NA_REC;
 constexpr size_t NA_STATUS_BYTES = align256((size_t)NOALLOC_PASSES * NOALLOC_SORT_TILES * RADIX * 8);
 constexpr size_t NA_PART = NA_STATUS + NA_STATUS_BYTES;
-constexpr size_t NA_PART_BYTES = align256((size_t)HIST_ROWS * NOALLOC_PASSES * RADIX * 4);
+constexpr size_t NA_PART_BYTES = align256(((size_t)HIST_ROWS * NOALLOC_PASSES * RADIX + MAX_PASSES) * 4);
 constexpr size_t NA_HIST = NA_PART + NA_PART_BYTES;
-constexpr size_t NA_HIST_BYTES = align256((size_t)(NOALLOC_PASSES * RADIX + MAX_PASSES) * 4);
+constexpr size_t NA_HIST_BYTES = align256((size_t)NOALLOC_PASSES * RADIX * 4);
 constexpr size_t NA_MERGE_P = NA_HIST + NA_HIST_BYTES;
 constexpr size_t NA_MERGE_P_BYTES = align256((size_t)NOALLOC_MERGE_TILES * 3 * 8);
 constexpr size_t NA_SPLITS = NA_MERGE_P + NA_MERGE_P_BYTES;

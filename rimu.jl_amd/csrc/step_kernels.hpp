@@ -143,6 +143,16 @@ __device__ inline ColumnPlan plan_column(const StepArgs& a, K k, V v) {
     return c;
 }
 
+// Counters, flags and status words of a step, cleared in one launch.
+struct ClearRange { uint32_t* p; int64_t n; };
+struct ClearSet { ClearRange r[3]; };
+__global__ __launch_bounds__(NT) void clear_kernel(ClearSet cs) {
+    const int64_t stride = (int64_t)gridDim.x * NT;
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+        for (int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x; i < cs.r[q].n; i += stride) cs.r[q].p[i] = 0;
+}
+
 // ---------------------------------------------------------------------------------------
 // plan: the diagonal step and the number of spawn attempts of every entry, the exclusive
 // scan of the attempt counts (aoff, L + 1 values; aoff[L] = W, also written to *W_out), and
@@ -255,21 +265,22 @@ __global__ __launch_bounds__(NT) void plan_kernel(StepArgs a, const K* __restric
 }
 
 // ---------------------------------------------------------------------------------------
-// Exclusive scan of int64 counts (three kernels; deterministic).
+// Exclusive scan of n values, those past `valid` taken as zero (three kernels, or the first
+// alone where one tile holds them; deterministic).
 // ---------------------------------------------------------------------------------------
 constexpr int SCAN_IPT = 8;
 constexpr int SCAN_TILE = NT * SCAN_IPT;
 
 template <class T>
 __global__ __launch_bounds__(NT) void scan_tiles_kernel(const T* __restrict__ in, T* __restrict__ out,
-                                                        int64_t n, T* __restrict__ tile_sums) {
+                                                        int64_t n, int64_t valid, T* __restrict__ tile_sums) {
     const int64_t base = (int64_t)blockIdx.x * SCAN_TILE + (int64_t)threadIdx.x * SCAN_IPT;
     T loc[SCAN_IPT];
     T sum = 0;
 #pragma unroll
     for (int j = 0; j < SCAN_IPT; ++j) {
         const int64_t idx = base + j;
-        loc[j] = idx < n ? in[idx] : (T)0;
+        loc[j] = idx < valid ? in[idx] : (T)0;
         sum += loc[j];
     }
     T total;
@@ -1391,19 +1402,51 @@ __global__ __launch_bounds__(NT) void merge_kernel(StepArgs a, const K* __restri
     }
 }
 
+// Where a tile's records go: with raw, offs holds the tiles' counts, which every workgroup adds
+// up for itself (at most COMPACT_RAW_MAX tiles: one read of 8 KB instead of a scan's launches
+// before the compaction); else their exclusive scan with the total in offs[ntiles].
+constexpr int64_t COMPACT_RAW_MAX = 4 * NT;
+struct TilePlace { int64_t off, n, total; };
+__device__ inline TilePlace tile_place(const int64_t* __restrict__ offs, int64_t ntiles, int64_t tile, int raw) {
+    if (!raw) return TilePlace{offs[tile], offs[tile + 1] - offs[tile], offs[ntiles]};
+    __shared__ int64_t s[2][NT / WAVE];
+    int64_t before = 0, total = 0;
+#pragma unroll
+    for (int r = 0; r < (int)(COMPACT_RAW_MAX / NT); ++r) {
+        const int64_t t = (int64_t)r * NT + threadIdx.x;
+        const int64_t c = t < ntiles ? offs[t] : 0;
+        total += c;
+        before += t < tile ? c : 0;
+    }
+#pragma unroll
+    for (int off = WAVE / 2; off > 0; off >>= 1) {
+        total += __shfl_xor(total, off, WAVE);
+        before += __shfl_xor(before, off, WAVE);
+    }
+    if ((threadIdx.x & (WAVE - 1)) == 0) {
+        s[0][threadIdx.x / WAVE] = total;
+        s[1][threadIdx.x / WAVE] = before;
+    }
+    __syncthreads();
+    total = before = 0;
+#pragma unroll
+    for (int w = 0; w < NT / WAVE; ++w) { total += s[0][w]; before += s[1][w]; }
+    return TilePlace{before, offs[tile], total};
+}
+
 // compact: tile t's records (merge survivors or spawns; NT * IPT slots per tile) move from
-// its slot range to [offs[t], offs[t+1]) (offs is the exclusive scan of the tile counts,
-// offs[ntiles] the new length).  If the new length exceeds cap nothing is written and
-// FLAG is raised.
+// its slot range to their final place (tile_place).  If the new length exceeds cap nothing is
+// written and FLAG is raised.
 template <class K, class V, int IPT, int FLAG>
 __global__ __launch_bounds__(NT) void compact_kernel(const K* __restrict__ slot_k,
                                                      const V* __restrict__ slot_v,
-                                                     const int64_t* __restrict__ offs, int64_t ntiles,
+                                                     const int64_t* __restrict__ offs, int64_t ntiles, int raw,
                                                      K* __restrict__ ok, V* __restrict__ ov,
                                                      int64_t cap, int64_t* total_out, int* flags) {
     constexpr int TILE = NT * IPT;
     const int64_t tile = blockIdx.x;
-    const int64_t total = offs[ntiles];
+    const TilePlace at = tile_place(offs, ntiles, tile, raw);
+    const int64_t total = at.total;
     if (total > cap) {
         if (tile == 0 && threadIdx.x == 0) {
             atomicOr(flags, FLAG);
@@ -1412,8 +1455,8 @@ __global__ __launch_bounds__(NT) void compact_kernel(const K* __restrict__ slot_
         return;
     }
     if (tile == 0 && threadIdx.x == 0) *total_out = total;
-    const int64_t off = offs[tile];
-    const int n = (int)(offs[tile + 1] - off);
+    const int64_t off = at.off;
+    const int n = (int)at.n;
     const int64_t src = tile * TILE;
     K k[IPT];
     V v[IPT];
@@ -1432,23 +1475,31 @@ __global__ __launch_bounds__(NT) void compact_kernel(const K* __restrict__ slot_
 // ---------------------------------------------------------------------------------------
 // project: terms[i] = coef_i * v[key_i] (0 if absent) by binary search in the new vector.
 // ---------------------------------------------------------------------------------------
+struct ProjectArgs {
+    const void *keys, *vals;   // the new vector
+    const int64_t* len;
+    const void* pk;
+    const double* pc;
+    int64_t np;
+    double* terms;
+};
 template <class K, class V>
-__global__ __launch_bounds__(NT) void project_kernel(const K* __restrict__ keys,
-                                                     const V* __restrict__ vals, const int64_t* len_p,
-                                                     const K* __restrict__ pk,
-                                                     const double* __restrict__ pc, int64_t np,
-                                                     double* __restrict__ terms) {
-    const int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x;
-    if (i >= np) return;
-    const int64_t L = *len_p;
-    const K key = pk[i];
+__device__ inline double project_term(const ProjectArgs& p, int64_t i) {
+    const K* keys = (const K*)p.keys;
+    const int64_t L = *p.len;
+    const K key = ((const K*)p.pk)[i];
     int64_t lo = 0, hi = L;
     while (lo < hi) {
         const int64_t mid = (lo + hi) >> 1;
         if (keys[mid] < key) lo = mid + 1; else hi = mid;
     }
-    const double x = (lo < L && keys[lo] == key) ? (double)vals[lo] : 0.0;
-    terms[i] = x * pc[i];
+    const double x = (lo < L && keys[lo] == key) ? (double)((const V*)p.vals)[lo] : 0.0;
+    return x * p.pc[i];
+}
+template <class K, class V>
+__global__ __launch_bounds__(NT) void project_kernel(ProjectArgs p) {
+    const int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x;
+    if (i < p.np) p.terms[i] = project_term<K, V>(p, i);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1498,21 +1549,80 @@ __device__ inline double double_log_update(const ShiftUpdate& su, double norm) {
                        su.zeta / su.dtau * log_or_minf(norm / su.in[1]));
 }
 
-// out[0..NSTAT-1]: the statistics; with a device shift update also out[NSTAT] = S' and
-// out[NSTAT + 1] = N_prev' (the norm is statistic 9).
-__global__ __launch_bounds__(64) void finalize_kernel(const double* __restrict__ chunk_sums, int nchunks,
-                                                      double* __restrict__ out, ShiftUpdate su) {
-    const int j = threadIdx.x;
-    if (j >= NSTAT) return;
-    double acc = 0;
-    for (int b = 0; b < nchunks; ++b) acc += chunk_sums[j * nchunks + b];
-    out[j] = acc;
+// The step's results, written straight to pinned host memory (no copy follows): out[0..NSTAT-1]
+// the statistics, with a device shift update out[NSTAT] = S' and out[NSTAT + 1] = N_prev' (the
+// norm is statistic 9), and the step's counters and flags, misc_words of them.
+struct StepOut {
+    double* out;
+    const uint32_t* misc;
+    uint32_t* misc_out;
+    int misc_words;
+};
+__device__ inline void step_out(const StepOut& so, const ShiftUpdate& su, int j, double acc) {
+    so.out[j] = acc;
     if (j == 9 && su.in) {
         const double s = double_log_update(su, acc);
         su.out[0] = s;
         su.out[1] = acc;
-        out[NSTAT] = s;
-        out[NSTAT + 1] = acc;
+        so.out[NSTAT] = s;
+        so.out[NSTAT + 1] = acc;
+    }
+}
+
+constexpr int STATS_NT = 1024;
+static_assert(NSTAT * PARTIAL_BLOCKS <= STATS_NT, "one thread per chunk sum");
+__global__ __launch_bounds__(STATS_NT) void finalize_kernel(const double* __restrict__ chunk_sums, StepOut so,
+                                                            ShiftUpdate su) {
+    __shared__ double s[NSTAT][PARTIAL_BLOCKS];
+    const int t = threadIdx.x;
+    if (t < NSTAT * PARTIAL_BLOCKS) s[t / PARTIAL_BLOCKS][t % PARTIAL_BLOCKS] = chunk_sums[t];
+    if (t >= STATS_NT - WAVE && t - (STATS_NT - WAVE) < so.misc_words)
+        so.misc_out[t - (STATS_NT - WAVE)] = so.misc[t - (STATS_NT - WAVE)];
+    __syncthreads();
+    if (t < NSTAT) {
+        double acc = 0;
+        for (int b = 0; b < PARTIAL_BLOCKS; ++b) acc += s[t][b];
+        step_out(so, su, t, acc);
+    }
+}
+
+// The same statistics in one workgroup where every partial array has at most STATS_SMALL
+// elements: the projections, then row r of an array (its elements r*NT .. r*NT + NT - 1) by one
+// wavefront in block_sum's tree order, then the rows in order -- the same additions, so the
+// same bits, as partial_sums_kernel and finalize_kernel, whose two launches and the
+// projections' one cost more than the work (13.5 us of kernels on a run of 1e4 entries).
+constexpr int STATS_ROWS = 4;
+constexpr int64_t STATS_SMALL = STATS_ROWS * NT;
+template <class K, class V>
+__global__ __launch_bounds__(STATS_NT) void stats_small_kernel(PartialSet ps, ProjectArgs p, StepOut so,
+                                                               ShiftUpdate su) {
+    static_assert(NT == 4 * WAVE, "four elements per lane and row");
+    __shared__ double s[NSTAT][STATS_ROWS];
+    for (int64_t i = threadIdx.x; i < p.np; i += STATS_NT) p.terms[i] = project_term<K, V>(p, i);
+    __syncthreads();  // the terms are read back by other threads of this workgroup
+    const int lane = threadIdx.x & (WAVE - 1);
+    for (int q = threadIdx.x / WAVE; q < NSTAT * STATS_ROWS; q += STATS_NT / WAVE) {
+        const int j = q / STATS_ROWS, r = q % STATS_ROWS;
+        const int64_t n = ps.n[j] - (int64_t)r * NT;
+        const double* x = ps.p[j] + (int64_t)r * NT;
+        double v = 0;
+        if (n > 0) {
+            double e[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) e[c] = lane + c * WAVE < n ? x[lane + c * WAVE] : 0.0;
+            v = (e[0] + e[2]) + (e[1] + e[3]);
+#pragma unroll
+            for (int off = WAVE / 2; off > 0; off >>= 1) v += __shfl_down(v, off, WAVE);
+        }
+        if (lane == 0) s[j][r] = v;
+    }
+    if (threadIdx.x < so.misc_words) so.misc_out[threadIdx.x] = so.misc[threadIdx.x];
+    __syncthreads();
+    if (threadIdx.x < NSTAT) {
+        double acc = 0;
+#pragma unroll
+        for (int r = 0; r < STATS_ROWS; ++r) acc += s[threadIdx.x][r];
+        step_out(so, su, (int)threadIdx.x, acc);
     }
 }
 
