@@ -56,15 +56,17 @@ constexpr int FLAG_BUCKET_OVERFLOW = 16;
 
 // First record and first vector entry of every bucket: rstart[b] = lower bound of b among
 // the records' top T bits (records sorted on them), vstart[b] likewise in the vector;
-// b = 0 .. 2^T (the last is S, resp. L).
+// b = 0 .. 2^T (the last is S, resp. L).  T = 0: one bucket of everything, in list order.
 __global__ __launch_bounds__(NT) void bucket_bounds_kernel(const uint64_t* __restrict__ ak, Count cS,
                                                            const uint64_t* __restrict__ bk, int64_t L,
                                                            int shift, int64_t nbuckets,
                                                            int64_t* __restrict__ rstart,
-                                                           int64_t* __restrict__ vstart) {
+                                                           int64_t* __restrict__ vstart, int* flags) {
     const int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x;
     if (i > 2 * nbuckets + 1) return;
-    const int64_t S = min(count_value(cS), cS.cap);  // more records raise FLAG_SPEC earlier
+    const int64_t S = min(count_value(cS), cS.cap);
+    // more records than the grids cover (a sort raises this itself; one bucket needs none)
+    if (i == 0 && count_value(cS) > cS.cap) atomicOr(flags, FLAG_SPEC);
     const bool rec = i <= nbuckets;
     const int64_t b = rec ? i : i - nbuckets - 1;
     const uint64_t* k = rec ? ak : bk;

@@ -578,14 +578,13 @@ int reorder_on_device(rimu_engine* e, int64_t n, int forward, int* result, Fill&
 // the vector (bk, bv: keys and diagonal survivors, L entries; bo: the old values, which give
 // the entries' initiator class when an initiator rule is set) into (ok, ov) of capacity cap.
 // `tiles` receives the number of buckets (rows of merge_p).
-constexpr int64_t BK_MIN_RECORDS = 4096;
 constexpr int BK_MAX_LOWBITS = 48;   // packed words: key bits below the bucket bits + a 12-bit item index
 constexpr int BK_COOLDOWN = 16;      // steps on the merge path after a bucket overflowed
 
 // How a step's records are cut into buckets: the top T stored-key bits, and the kernel shape
-// (items per thread) that holds a bucket.
+// (items per thread) that holds a bucket.  T = 0: one bucket, no radix pass.
 struct BucketCut {
-    int T = 0;    // 0: no bucket merge
+    int T = -1;    // negative: no bucket merge
     int ipt = 0;
 };
 
@@ -602,21 +601,24 @@ double bucket_mean_max(int ipt) {
 // buckets take 158, 183, 226, 412 us (the last two with two items per thread and four
 // workgroups on a CU, a shape no step takes now); 1.5e8 items in 2^17 buckets take 2.75 ms with
 // three items per thread (three workgroups on a CU) and 3.22 ms with five (two).
-BucketCut bucket_cut(int64_t S, int64_t L, int B, int min_ipt) {
+// A step of up to 2092 items is one bucket, sorted without a radix pass, whether its keys are
+// mixed or not (1000 integer walkers on 19-bit keys: 99 us a step with three radix passes and
+// the merge path, 66 us so); more buckets need mixed keys, whose top bits are spread evenly.
+BucketCut bucket_cut(int64_t S, int64_t L, int B, bool mixed, int min_ipt) {
     const double items = (double)S + (double)L;
     BucketCut cut;
-    cut.T = 1;
+    cut.T = 0;
     while (cut.T < std::min(B, 24) && std::ldexp(items, -cut.T) > bucket_mean_max(BK_IPT_MAX)) ++cut.T;
     cut.ipt = min_ipt;
     while (cut.ipt < BK_IPT_MAX && std::ldexp(items, -cut.T) > bucket_mean_max(cut.ipt)) ++cut.ipt;
-    if (B - cut.T > BK_MAX_LOWBITS) cut.T = 0;
+    if (B - cut.T > BK_MAX_LOWBITS || (cut.T > 0 && !mixed)) cut.T = -1;
     return cut;
 }
 
 // Lowest key bit a step's sort covers: the bucket bits, the top bits of wide mixed keys, or all.
 int sort_from(const rimu_engine* e, const BucketCut& cut) {
     const int B = e->hdev.B;
-    if (cut.T > 0) return B - cut.T;
+    if (cut.T >= 0) return B - cut.T;
     return e->mix.on && B > e->sort_bits ? B - e->sort_bits : 0;
 }
 
@@ -636,7 +638,7 @@ int bucket_merge_shape(rimu_engine* e, const StepArgs& a, const uint64_t* ak, co
     hipEvent_t ev{};
     e->timer.begin("bucket_bounds", e->stream, &ev);
     bucket_bounds_kernel<<<ceil_div(2 * nbk + 2, NT), NT, 0, e->stream>>>(ak, Count{S, S_dev, S}, bk, L, B - T, nbk,
-                                                                          e->bk_rstart.p, e->bk_vstart.p);
+                                                                          e->bk_rstart.p, e->bk_vstart.p, &dm->flags);
     e->timer.end(e->stream);
     if (e->n_cu == 0) {
         HIP_TRY(hipDeviceGetAttribute(&e->n_cu, hipDeviceAttributeMultiprocessorCount, e->device));
@@ -708,11 +710,11 @@ int step_impl(rimu_engine* e, int64_t step, double shift, double dtau, double bo
     const bool rs = e->hdev.kind == RIMU_MODEL_HUBBARD_REAL_SPACE;
     const bool dense = !e->int_vals && e->style.proj_threshold == 0 && (!rs || !rs_zero_channels(e->hdev));
     const int nbits = e->hdev.B;
-    const bool bucket_ok = KW == 1 && e->radix_mode == 2 && e->mix.on && e->bucket_cooldown == 0;
+    const bool bucket_ok = KW == 1 && e->radix_mode == 2 && e->bucket_cooldown == 0;
     bool spec = e->spec_ok && e->radix_mode != 0 && e->W_prev > 0;
     BucketCut cut;
     // the path the counts of the last step choose; sorts with a host check stay synchronous
-    if (spec && bucket_ok && e->S_prev >= BK_MIN_RECORDS) cut = bucket_cut(e->S_prev, L, nbits, e->bucket_ipt_min);
+    if (spec && bucket_ok) cut = bucket_cut(e->S_prev, L, nbits, e->mix.on, e->bucket_ipt_min);
     const int64_t W_cap = spec ? e->W_prev + e->W_prev / 4 + 16 * SPAWN_TILE : 0;
 
     // 1. plan: diagonal step, attempt offsets and the first entry of each spawn tile (as
@@ -845,7 +847,7 @@ int step_impl(rimu_engine* e, int64_t step, double shift, double dtau, double bo
     const int nxt = 1 - e->cur;
     int64_t merge_tiles = 0;
     int sorted = 0;
-    if (!spec && bucket_ok && S >= BK_MIN_RECORDS) cut = bucket_cut(S, L, nbits, e->bucket_ipt_min);
+    if (!spec && bucket_ok) cut = bucket_cut(S, L, nbits, e->mix.on, e->bucket_ipt_min);
     if (e->bucket_cooldown > 0) --e->bucket_cooldown;
     const int64_t* merge_S_dev = S_dev;  // the merge path after the fallback sort reads S from the host
     auto merge_path = [&]() -> int {
@@ -853,7 +855,7 @@ int step_impl(rimu_engine* e, int64_t step, double shift, double dtau, double bo
                                 (const V*)e->dvals.p, L, (K*)e->vkeys[nxt].p, (V*)e->vvals[nxt].p,
                                 e->max_entries, dm, &merge_tiles, vv, merge_S_dev);
     };
-    if (cut.T > 0) {
+    if (cut.T >= 0) {
         if (int rc = radix_sort<K, V>(e, S, nbits, kor ^ kand, 0, &sorted, nbits - cut.T, S_dev)) return rc;
         if (int rc = bucket_merge_into<V>(e, a, (const uint64_t*)e->skeys[sorted].p, (const V*)e->svals[sorted].p,
                                           S, (const uint64_t*)vk, (const V*)e->dvals.p, vv, L, cut,
