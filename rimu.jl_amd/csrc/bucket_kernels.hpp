@@ -1,5 +1,4 @@
-// bucket_kernels.hpp -- annihilation of a step's spawn records by buckets of the stored key
-// (one-word mixed keys).
+// bucket_kernels.hpp -- annihilation of a step's spawn records by buckets of the stored key.
 //
 // The stored keys are a bijective mix of the addresses, so their top bits are spread evenly.
 // The spawn records are radix-sorted (stable, look-back scatters of step_kernels.hpp) on the
@@ -27,6 +26,11 @@
 // draws; with an initiator rule each address folds three components instead of one, as on
 // the merge path.  A bucket larger than its LDS arrays raises FLAG_BUCKET_OVERFLOW and writes
 // nothing; the host then sorts on every bit and merges along the merge path.
+//
+// Two-word keys have more bits below the bucket bits than a packed word holds: the word takes
+// the upper 52 of them and the key's low word is kept in LDS by item index.  Addresses are told
+// apart by the word; two addresses that agree in all its key bits (about one pair in 2^(T + 52)
+// of mixed keys) are noticed by their low words and raise FLAG_BUCKET_OVERFLOW too.
 #pragma once
 
 #include "step_kernels.hpp"
@@ -42,12 +46,12 @@ constexpr int BK_FOLD_EXTRA = 4;              // positions read past a thread's 
 // A bucket kernel is built for buckets of up to IPT * BK_NT items (records + vector entries).
 // A bucket's LDS and the registers of its threads grow with IPT, so the smallest that holds
 // the step's buckets keeps the most workgroups on a CU and the fewest idle item slots:
-// BkShape::WG_PER_CU workgroups of 512 threads.
+// wgs() workgroups of 512 threads.
 template <int IPT> struct BkShape {
     static constexpr int CAP = BK_NT * IPT;
     static constexpr int SUB_BITS = 11;  // sub-buckets of the LDS sort
     static constexpr int NSUB = 1 << SUB_BITS;
-    static constexpr int WG_PER_CU = IPT == 3 ? 3 : 2;
+    static constexpr int wgs(size_t key_bytes) { return key_bytes == 8 && IPT == 3 ? 3 : 2; }  // per CU
     static_assert(CAP <= (1 << BK_IDX_BITS), "item indices fit their bits");
     static_assert(NSUB % BK_NT == 0, "whole rounds per thread");
     static_assert(IPT < 8, "survivor masks are 32-bit; per-thread counts fit three bits");
@@ -57,9 +61,12 @@ constexpr int FLAG_BUCKET_OVERFLOW = 16;
 // First record and first vector entry of every bucket: rstart[b] = lower bound of b among
 // the records' top T bits (records sorted on them), vstart[b] likewise in the vector;
 // b = 0 .. 2^T (the last is S, resp. L).  T = 0: one bucket of everything, in list order.
-__global__ __launch_bounds__(NT) void bucket_bounds_kernel(const uint64_t* __restrict__ ak, Count cS,
-                                                           const uint64_t* __restrict__ bk, int64_t L,
-                                                           int shift, int64_t nbuckets,
+// kmask clears the initiator class bit (all ones without initiators: the bit is an address
+// bit of 64- and 128-bit keys).
+template <class K>
+__global__ __launch_bounds__(NT) void bucket_bounds_kernel(const K* __restrict__ ak, Count cS,
+                                                           const K* __restrict__ bk, int64_t L,
+                                                           int shift, int64_t nbuckets, K kmask,
                                                            int64_t* __restrict__ rstart,
                                                            int64_t* __restrict__ vstart, int* flags) {
     const int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x;
@@ -69,11 +76,11 @@ __global__ __launch_bounds__(NT) void bucket_bounds_kernel(const uint64_t* __res
     if (i == 0 && count_value(cS) > cS.cap) atomicOr(flags, FLAG_SPEC);
     const bool rec = i <= nbuckets;
     const int64_t b = rec ? i : i - nbuckets - 1;
-    const uint64_t* k = rec ? ak : bk;
+    const K* k = rec ? ak : bk;
     int64_t lo = 0, hi = rec ? S : L;
     while (lo < hi) {
         const int64_t mid = (lo + hi) >> 1;
-        if ((int64_t)((k[mid] & ~CLASS_BIT) >> shift) < b) lo = mid + 1; else hi = mid;
+        if ((int64_t)((k[mid] & kmask) >> shift) < b) lo = mid + 1; else hi = mid;
     }
     (rec ? rstart : vstart)[b] = lo;
 }
@@ -121,9 +128,10 @@ __device__ inline T bk_block_exclusive_scan(T v, int lane, int wid, T* s_wave, T
 // LDS of one bucket workgroup.  `vin` holds the items' values by item index and `place`
 // their packed words sub-bucket by sub-bucket; `sk` receives the words in order.  After the
 // fold `place` and `vin` stage the values that ThresholdCompression draws for.
-template <class V, bool INIT, int IPT>
+template <class K, class V, bool INIT, int IPT>
 struct BucketLds {
     static constexpr int CAP = BkShape<IPT>::CAP;
+    uint64_t klo[sizeof(K) == 8 ? 1 : CAP];  // two-word keys: the items' low words by item index
     uint64_t place[CAP];
     uint64_t sk[CAP];
     V vin[CAP];
@@ -143,17 +151,19 @@ struct BucketLds {
 // each address folds three components in list order -- safe (entries with the class, records
 // without), unsafe (records with the class), initiator (entries without) -- exists when one
 // is nonzero and takes the rule's value (initiator_value), as merge_kernel<K, V, true> does.
-template <class V, bool INIT, int IPT>
-__global__ __launch_bounds__(BK_NT, 2 * BkShape<IPT>::WG_PER_CU) void bucket_merge_kernel(
-    StepArgs a, const uint64_t* __restrict__ ak, const V* __restrict__ av, const uint64_t* __restrict__ bk,
+template <class K, class V, bool INIT, int IPT>
+__global__ __launch_bounds__(BK_NT, 2 * BkShape<IPT>::wgs(sizeof(K))) void bucket_merge_kernel(
+    StepArgs a, const K* __restrict__ ak, const V* __restrict__ av, const K* __restrict__ bk,
     const V* __restrict__ bv, const V* __restrict__ bo, const int64_t* __restrict__ rstart, const int64_t* __restrict__ vstart, int64_t nbk,
-    int lowbits, uint64_t* __restrict__ slot_k, V* __restrict__ slot_v, int64_t* __restrict__ bucket_cnt,
+    int lowbits, K* __restrict__ slot_k, V* __restrict__ slot_v, int64_t* __restrict__ bucket_cnt,
     double* __restrict__ partials, int* flags) {
     constexpr int NW = BK_NT / WAVE;
     constexpr uint64_t IDX_MASK = (1ull << BK_IDX_BITS) - 1ull;
     constexpr int BK_IPT = IPT, BK_CAP = BkShape<IPT>::CAP;
     constexpr int BK_SUB_BITS = BkShape<IPT>::SUB_BITS, BK_NSUB = BkShape<IPT>::NSUB;
-    __shared__ BucketLds<V, INIT, IPT> sm;
+    constexpr bool WIDE = sizeof(K) == 16;
+    constexpr int WORD_KEY_BITS = 64 - BK_IDX_BITS;  // key bits of a packed word
+    __shared__ BucketLds<K, V, INIT, IPT> sm;
     // no sorted list to merge (raised by earlier kernels only: every wave reads the same bits)
     if (*flags & (FLAG_LOOKBACK | FLAG_SPEC)) {
         for (int64_t b = blockIdx.x; b < nbk; b += gridDim.x) {
@@ -166,23 +176,25 @@ __global__ __launch_bounds__(BK_NT, 2 * BkShape<IPT>::WG_PER_CU) void bucket_mer
         }
         return;
     }
-    const uint64_t lowmask = lowbits >= 64 ? ~0ull : (1ull << lowbits) - 1ull;
+    const K lowmask = low_maskA<K>(lowbits);
+    const int drop = WIDE ? max(lowbits - WORD_KEY_BITS, 0) : 0;  // key bits below the packed word's
     // sub-bucket digit: the top BK_SUB_BITS key bits below the bucket bits (all of them when
     // fewer remain)
-    const int dsh = BK_IDX_BITS + (lowbits > BK_SUB_BITS ? lowbits - BK_SUB_BITS : 0);
-    const uint32_t dmask = lowbits >= BK_SUB_BITS ? (uint32_t)(BK_NSUB - 1) : (1u << lowbits) - 1u;
+    const int wbits = lowbits - drop;
+    const int dsh = BK_IDX_BITS + (wbits > BK_SUB_BITS ? wbits - BK_SUB_BITS : 0);
+    const uint32_t dmask = wbits >= BK_SUB_BITS ? (uint32_t)(BK_NSUB - 1) : (1u << wbits) - 1u;
     for (int j = threadIdx.x; j < BK_NSUB + 1; j += BK_NT) sm.sub[j] = 0;
 
     // items of the first bucket; later ones are loaded during the bucket before them.  Item
     // i < nb is vector entry v0 + i, item nb + r is record r0 + r: the item index orders each
     // address's items as the fold takes them (diagonal value first, spawns in list order).
     int64_t b = blockIdx.x;
-    uint64_t ck[BK_IPT];
+    K ck[BK_IPT];
     V cv[BK_IPT];
     uint32_t ccls = 0;  // INIT: bit j = class of item slot j
     int64_t r0 = 0, v0 = 0;
     int na = 0, nb = 0;
-    auto load = [&](int t, int64_t bb, uint64_t* qk, V* qv, uint32_t& q_cls, int64_t& q_r0, int64_t& q_v0,
+    auto load = [&](int t, int64_t bb, K* qk, V* qv, uint32_t& q_cls, int64_t& q_r0, int64_t& q_v0,
                     int& q_na, int& q_nb) {
         q_r0 = rstart[bb];
         q_v0 = vstart[bb];
@@ -190,9 +202,9 @@ __global__ __launch_bounds__(BK_NT, 2 * BkShape<IPT>::WG_PER_CU) void bucket_mer
         q_nb = (int)(vstart[bb + 1] - q_v0);
         const int q_n = q_na + q_nb;
         if (q_n > BK_CAP) return;  // overflow: nothing is read
-        const uint64_t* ek_b = bk + q_v0;  // uniform bases, 32-bit offsets
+        const K* ek_b = bk + q_v0;  // uniform bases, 32-bit offsets
         const V* ev_b = bv + q_v0;
-        const uint64_t* rk_b = ak + q_r0;
+        const K* rk_b = ak + q_r0;
         const V* rv_b = av + q_r0;
         q_cls = 0;
 #pragma unroll
@@ -209,7 +221,7 @@ __global__ __launch_bounds__(BK_NT, 2 * BkShape<IPT>::WG_PER_CU) void bucket_mer
                 qk[j] = rk_b[i - (uint32_t)q_nb];
                 qv[j] = rv_b[i - (uint32_t)q_nb];
                 if constexpr (INIT) {
-                    if (qk[j] & CLASS_BIT) q_cls |= 1u << j;
+                    if (qk[j] & class_bit<K>()) q_cls |= 1u << j;
                 }
             }
         }
@@ -224,7 +236,7 @@ __global__ __launch_bounds__(BK_NT, 2 * BkShape<IPT>::WG_PER_CU) void bucket_mer
         asm volatile("v_mov_b32 %0, %1" : "=v"(tid) : "v"((int)threadIdx.x));
         const int lane = tid & (WAVE - 1);
         const int wid = __builtin_amdgcn_readfirstlane(tid / WAVE);
-        uint64_t nk[BK_IPT];
+        K nk[BK_IPT];
         V nv[BK_IPT];
         uint32_t ncls = 0;
         int64_t n_r0 = 0, n_v0 = 0;
@@ -233,12 +245,22 @@ __global__ __launch_bounds__(BK_NT, 2 * BkShape<IPT>::WG_PER_CU) void bucket_mer
 
         const int n = na + nb;
         const bool fits = n <= BK_CAP;  // uniform over the workgroup
-        uint64_t okey[BK_IPT];
+        // the key of a survivor: one-word keys from its bits below the bucket bits, two-word keys
+        // from its packed word (the low word by the item index in it)
+        auto key_of = [&](uint64_t x) -> K {
+            const K top = shlA((K)b, lowbits);
+            if constexpr (WIDE) {
+                const K k = top | shlA((K)(x >> BK_IDX_BITS), drop);
+                return (K)(k >> 64) << 64 | (K)sm.klo[(int)(x & IDX_MASK)];
+            } else {
+                return top | x;
+            }
+        };
+        uint64_t okey[BK_IPT];  // key_of's argument
         V oval[BK_IPT];
         uint32_t cvalid = 0;
         int n_before = 0;  // len_before: folded values that are not zero
         if (fits) {
-            const uint64_t bucket_key = lowbits >= 64 ? 0ull : (uint64_t)b << lowbits;
             // ---- 1. pack (key bits below the bucket bits, item index), values by item
             // index, drop every word into its sub-bucket (arrival order is arbitrary) ---------
             uint64_t w[BK_IPT];
@@ -247,7 +269,8 @@ __global__ __launch_bounds__(BK_NT, 2 * BkShape<IPT>::WG_PER_CU) void bucket_mer
             for (int j = 0; j < BK_IPT; ++j) {
                 const int i = tid + j * BK_NT;
                 if (i < n) {
-                    w[j] = ((ck[j] & lowmask) << BK_IDX_BITS) | (uint64_t)i;
+                    w[j] = ((uint64_t)((ck[j] & lowmask) >> drop) << BK_IDX_BITS) | (uint64_t)i;
+                    if constexpr (WIDE) sm.klo[i] = (uint64_t)(INIT ? ck[j] & (K)~class_bit<K>() : ck[j]);
                     sm.vin[i] = cv[j];
                     if constexpr (INIT) sm.cls[i] = (uint8_t)((ccls >> j) & 1u);
                     dg[j] = (uint32_t)(w[j] >> dsh) & dmask;
@@ -321,7 +344,7 @@ __global__ __launch_bounds__(BK_NT, 2 * BkShape<IPT>::WG_PER_CU) void bucket_mer
             for (int k = 0; k <= NWIN; ++k) {
                 const int p = p0 + k;
                 const uint64_t wd = p < n ? sm.sk[p] : NOKEY;
-                kk[k] = p < n ? wd >> BK_IDX_BITS : NOKEY;
+                kk[k] = WIDE || p >= n ? wd : wd >> BK_IDX_BITS;
                 if (k < NWIN) {
                     const int idx = (int)(wd & IDX_MASK);
                     vv[k] = p < n ? sm.vin[idx] : (V)0;
@@ -333,20 +356,37 @@ __global__ __launch_bounds__(BK_NT, 2 * BkShape<IPT>::WG_PER_CU) void bucket_mer
                     }
                 }
             }
-            const uint64_t kprev = p0 > 0 && p0 < n ? sm.sk[p0 - 1] >> BK_IDX_BITS : NOKEY;
+            const uint64_t wprev = p0 > 0 && p0 < n ? sm.sk[p0 - 1] : NOKEY;
+            const uint64_t kprev = WIDE || p0 == 0 || p0 >= n ? wprev : wprev >> BK_IDX_BITS;
+            // whether position p0 + k holds another address than the one before it
+            auto differ = [&](int k, uint64_t x, uint64_t before) {
+                if constexpr (WIDE) return p0 + k == 0 || ((x ^ before) >> BK_IDX_BITS) != 0;
+                else return x != before;
+            };
+            if constexpr (WIDE) {
+                // the same packed key bits must be the same address
+                bool tie = false;
+#pragma unroll
+                for (int k = 0; k < BK_IPT; ++k) {
+                    const uint64_t before = k > 0 ? kk[k - 1] : kprev;
+                    if (p0 + k < n && !differ(k, kk[k], before))
+                        tie |= sm.klo[(int)(kk[k] & IDX_MASK)] != sm.klo[(int)(before & IDX_MASK)];
+                }
+                if (tie) atomicOr(flags, FLAG_BUCKET_OVERFLOW);
+            }
             if constexpr (!INIT) {
                 bool own = false;
                 V acc = (V)0;
 #pragma unroll
                 for (int k = 0; k < NWIN; ++k) {
                     const bool valid = p0 + k < n;
-                    const bool start = valid && kk[k] != (k > 0 ? kk[k - 1] : kprev);
+                    const bool start = valid && differ(k, kk[k], k > 0 ? kk[k - 1] : kprev);
                     if (start) own = k < BK_IPT;
                     acc = (start ? (V)0 : acc) + vv[k];
-                    const bool end = valid && kk[k + 1] != kk[k];
+                    const bool end = valid && ((WIDE && p0 + k + 1 >= n) || differ(k + 1, kk[k + 1], kk[k]));
                     const int slot_k = k < BK_IPT - 1 ? k : BK_IPT - 1;
                     if (own && end) {
-                        okey[slot_k] = bucket_key | kk[k];
+                        okey[slot_k] = kk[k];
                         oval[slot_k] = acc;
                         if (acc != (V)0) cvalid |= 1u << slot_k;
                         own = false;
@@ -356,10 +396,10 @@ __global__ __launch_bounds__(BK_NT, 2 * BkShape<IPT>::WG_PER_CU) void bucket_mer
                     const uint64_t key = kk[NWIN - 1];
                     for (int q = p0 + NWIN; q < n; ++q) {
                         const uint64_t wd = sm.sk[q];
-                        if ((wd >> BK_IDX_BITS) != key) break;
+                        if ((wd >> BK_IDX_BITS) != (WIDE ? key >> BK_IDX_BITS : key)) break;
                         acc = acc + sm.vin[(int)(wd & IDX_MASK)];
                     }
-                    okey[BK_IPT - 1] = bucket_key | key;
+                    okey[BK_IPT - 1] = key;
                     oval[BK_IPT - 1] = acc;
                     if (acc != (V)0) cvalid |= 1u << (BK_IPT - 1);
                 }
@@ -383,7 +423,7 @@ __global__ __launch_bounds__(BK_NT, 2 * BkShape<IPT>::WG_PER_CU) void bucket_mer
                         cpres |= 1u << slot_k;
                         const V val = initiator_value<V>(a, cs, cu, ci);
                         if (val != (V)0 || keep_zero) {
-                            okey[slot_k] = bucket_key | key;
+                            okey[slot_k] = key;
                             oval[slot_k] = val;
                             cvalid |= 1u << slot_k;
                         }
@@ -393,13 +433,13 @@ __global__ __launch_bounds__(BK_NT, 2 * BkShape<IPT>::WG_PER_CU) void bucket_mer
                 for (int k = 0; k < NWIN; ++k) {
                     const int p = p0 + k;
                     const bool valid = p < n;
-                    const bool start = valid && kk[k] != (k > 0 ? kk[k - 1] : kprev);
+                    const bool start = valid && differ(k, kk[k], k > 0 ? kk[k - 1] : kprev);
                     if (start) {
                         own = k < BK_IPT;
                         cs = cu = ci = (V)0;
                     }
                     if (valid && own) dep((emask >> k) & 1u, (cmask >> k) & 1u, vv[k]);
-                    const bool end = valid && kk[k + 1] != kk[k];
+                    const bool end = valid && ((WIDE && p0 + k + 1 >= n) || differ(k + 1, kk[k + 1], kk[k]));
                     if (own && end) {
                         close_run(k < BK_IPT - 1 ? k : BK_IPT - 1, kk[k]);
                         own = false;
@@ -409,7 +449,7 @@ __global__ __launch_bounds__(BK_NT, 2 * BkShape<IPT>::WG_PER_CU) void bucket_mer
                     const uint64_t key = kk[NWIN - 1];
                     for (int q = p0 + NWIN; q < n; ++q) {
                         const uint64_t wd = sm.sk[q];
-                        if ((wd >> BK_IDX_BITS) != key) break;
+                        if ((wd >> BK_IDX_BITS) != (WIDE ? key >> BK_IDX_BITS : key)) break;
                         const int idx = (int)(wd & IDX_MASK);
                         dep(idx < nb, sm.cls[idx] != 0, sm.vin[idx]);
                     }
@@ -458,7 +498,7 @@ __global__ __launch_bounds__(BK_NT, 2 * BkShape<IPT>::WG_PER_CU) void bucket_mer
                     uint64_t seed;
                     asm volatile("s_mov_b64 %0, %1" : "=s"(seed) : "s"(a.seed));
                     for (int q = lane; q < wtot; q += WAVE) {
-                        const uint64_t key = wk[q];
+                        const K key = key_of(wk[q]);
                         const double x = (double)wv[q];
                         const U4 r = draw(seed, unmix_key(a.mix, key), 0, a.step, TAG_COMPRESS);
                         wv[q] = (fabs(x) / th > u53(r.x, r.y)) ? th * sgn(x) : 0.0;
@@ -488,7 +528,7 @@ __global__ __launch_bounds__(BK_NT, 2 * BkShape<IPT>::WG_PER_CU) void bucket_mer
             for (int j = 0; j < BK_IPT; ++j) {
                 if ((cvalid >> j) & 1u) {
                     const int q = __popc(cvalid & ((1u << j) - 1u));
-                    slot_k[base + q] = okey[j];
+                    slot_k[base + q] = key_of(okey[j]);
                     slot_v[base + q] = oval[j];
                 }
             }
@@ -525,13 +565,13 @@ __global__ __launch_bounds__(BK_NT, 2 * BkShape<IPT>::WG_PER_CU) void bucket_mer
 
 // Survivors of bucket b move from its slot range [rstart[b] + vstart[b], ...) to
 // their final place (tile_place of the bucket counts).  A new length above cap writes nothing and raises FLAG_VECTOR_OVERFLOW.
-template <class V, int IPT>
-__global__ __launch_bounds__(NT) void bucket_compact_kernel(const uint64_t* __restrict__ slot_k,
+template <class K, class V, int IPT>
+__global__ __launch_bounds__(NT) void bucket_compact_kernel(const K* __restrict__ slot_k,
                                                             const V* __restrict__ slot_v,
                                                             const int64_t* __restrict__ rstart,
                                                             const int64_t* __restrict__ vstart,
                                                             const int64_t* __restrict__ offs, int64_t nbuckets, int raw,
-                                                            uint64_t* __restrict__ ok, V* __restrict__ ov,
+                                                            K* __restrict__ ok, V* __restrict__ ov,
                                                             int64_t cap, int64_t* total_out, int* flags) {
     const int64_t b = blockIdx.x;
     const TilePlace at = tile_place(offs, nbuckets, b, raw);
@@ -548,7 +588,7 @@ __global__ __launch_bounds__(NT) void bucket_compact_kernel(const uint64_t* __re
     const int n = (int)at.n;
     const int64_t src = rstart[b] + vstart[b];
     constexpr int CPT = BkShape<IPT>::CAP / NT;
-    uint64_t k[CPT];
+    K k[CPT];
     V v[CPT];
 #pragma unroll
     for (int r = 0; r < CPT; ++r) {

@@ -125,7 +125,7 @@ struct rimu_engine {
     DevBuf<uint64_t> lb_status;     // look-back radix: status words [pass][tile][digit]
     uint32_t lb_epoch = 0;          // sort calls since lb_status was last cleared
     int bucket_cooldown = 0;        // steps left on the merge path after a bucket overflow
-    int bucket_ipt_min = BK_IPT_MIN;  // smallest bucket shape (items per thread) the steps may take
+    int bucket_roomy = 0;           // steps left that take the roomiest buckets, after an overflow
     bool spec_ok = false;           // the grids of the next step may be sized from W_prev, S_prev
     int64_t W_prev = 0, S_prev = 0; // spawn attempts and records of the last step
     uint32_t lb_spin_limit = LB_SPIN_LIMIT;  // bound of every look-back wait
@@ -331,9 +331,8 @@ bool nine_bit_digits(int nbits, int lo) {
 }
 
 // Words of lb_part that a look-back sort of key bits [lo, nbits) uses: tile ids, digit counts.
-template <class K>
 int64_t lb_words(int nbits, int lo) {
-    const int rb = sizeof(K) == 8 && nine_bit_digits(nbits, lo) ? 9 : RADIX_BITS;
+    const int rb = nine_bit_digits(nbits, lo) ? 9 : RADIX_BITS;
     return MAX_PASSES + (int64_t)HIST_ROWS * ceil_div(nbits - lo, rb) * (1 << rb);
 }
 
@@ -343,8 +342,7 @@ int radix_sort(rimu_engine* e, int64_t n, int nbits, u128 varying, int in, int* 
     int src = in;
     if (n <= 1 && !n_dev) { *result = src; return RIMU_OK; }
     if (e->radix_mode != 0 || n_dev) {
-        if constexpr (sizeof(K) == 8)
-            if (nine_bit_digits(nbits, lo)) return radix_sort_lb<K, V, 9>(e, n, nbits, varying, in, result, lo, n_dev);
+        if (nine_bit_digits(nbits, lo)) return radix_sort_lb<K, V, 9>(e, n, nbits, varying, in, result, lo, n_dev);
         return radix_sort_lb<K, V, 8>(e, n, nbits, varying, in, result, lo, n_dev);
     }
     const int64_t tiles = ceil_div(n, sort_tile<K>::value);
@@ -578,8 +576,12 @@ int reorder_on_device(rimu_engine* e, int64_t n, int forward, int* result, Fill&
 // the vector (bk, bv: keys and diagonal survivors, L entries; bo: the old values, which give
 // the entries' initiator class when an initiator rule is set) into (ok, ov) of capacity cap.
 // `tiles` receives the number of buckets (rows of merge_p).
-constexpr int BK_MAX_LOWBITS = 48;   // packed words: key bits below the bucket bits + a 12-bit item index
+// key bits below the bucket bits: in a packed word beside a 12-bit item index, or for two-word
+// keys 52 of them there and the rest in the low word
+constexpr int BK_MAX_LOWBITS = 48, BK_MAX_LOWBITS_WIDE = 116;
+constexpr int BK_IPT_MAX_WIDE = 4;   // two-word buckets of five items per thread leave one workgroup a CU
 constexpr int BK_COOLDOWN = 16;      // steps on the merge path after a bucket overflowed
+constexpr int BK_ROOMY = 256;        // steps with the largest shape after that
 
 // How a step's records are cut into buckets: the top T stored-key bits, and the kernel shape
 // (items per thread) that holds a bucket.  T = 0: one bucket, no radix pass.
@@ -606,12 +608,14 @@ double bucket_mean_max(int ipt) {
 // the merge path, 66 us so); more buckets need mixed keys, whose top bits are spread evenly.
 BucketCut bucket_cut(int64_t S, int64_t L, int B, bool mixed, int min_ipt) {
     const double items = (double)S + (double)L;
+    const int max_ipt = B > 64 ? BK_IPT_MAX_WIDE : BK_IPT_MAX;
+    const int max_low = B > 64 ? BK_MAX_LOWBITS_WIDE : BK_MAX_LOWBITS;
     BucketCut cut;
-    cut.T = 0;
-    while (cut.T < std::min(B, 24) && std::ldexp(items, -cut.T) > bucket_mean_max(BK_IPT_MAX)) ++cut.T;
-    cut.ipt = min_ipt;
-    while (cut.ipt < BK_IPT_MAX && std::ldexp(items, -cut.T) > bucket_mean_max(cut.ipt)) ++cut.ipt;
-    if (B - cut.T > BK_MAX_LOWBITS || (cut.T > 0 && !mixed)) cut.T = -1;
+    cut.T = B > 64 ? std::max(B - max_low, 0) : 0;  // at most 2^12 buckets more than the items need
+    while (cut.T < std::min(B, 24) && std::ldexp(items, -cut.T) > bucket_mean_max(max_ipt)) ++cut.T;
+    cut.ipt = std::min(min_ipt, max_ipt);
+    while (cut.ipt < max_ipt && std::ldexp(items, -cut.T) > bucket_mean_max(cut.ipt)) ++cut.ipt;
+    if (B - cut.T > max_low || (cut.T > 0 && !mixed)) cut.T = -1;
     return cut;
 }
 
@@ -622,10 +626,11 @@ int sort_from(const rimu_engine* e, const BucketCut& cut) {
     return e->mix.on && B > e->sort_bits ? B - e->sort_bits : 0;
 }
 
-template <class V, int IPT>
-int bucket_merge_shape(rimu_engine* e, const StepArgs& a, const uint64_t* ak, const V* av, int64_t S,
-                      const uint64_t* bk, const V* bv, const V* bo, int64_t L, int T, uint64_t* ok, V* ov,
+template <class K, class V, int IPT>
+int bucket_merge_shape(rimu_engine* e, const StepArgs& a, const K* ak, const V* av, int64_t S,
+                      const K* bk, const V* bv, const V* bo, int64_t L, int T, K* ok, V* ov,
                       int64_t cap, rimu_engine::Misc* dm, int64_t* tiles, const int64_t* S_dev) {
+    constexpr int KW = sizeof(K) / 8;
     const int B = e->hdev.B;
     const int64_t nbk = (int64_t)1 << T;
     *tiles = nbk;
@@ -633,26 +638,27 @@ int bucket_merge_shape(rimu_engine* e, const StepArgs& a, const uint64_t* ak, co
     HIP_TRY(e->bk_vstart.alloc(nbk + 1));
     HIP_TRY(e->tile_cnt.alloc(nbk + 1));
     HIP_TRY(e->merge_p.alloc((size_t)nbk * 3));
-    HIP_TRY(e->slot_k.alloc((size_t)(S + L)));
+    HIP_TRY(e->slot_k.alloc((size_t)(S + L) * KW));
     HIP_TRY(e->slot_v.alloc((size_t)(S + L)));
     hipEvent_t ev{};
+    const K kmask = a.init_rule != 0 ? (K)~class_bit<K>() : (K)~(K)0;
     e->timer.begin("bucket_bounds", e->stream, &ev);
-    bucket_bounds_kernel<<<ceil_div(2 * nbk + 2, NT), NT, 0, e->stream>>>(ak, Count{S, S_dev, S}, bk, L, B - T, nbk,
+    bucket_bounds_kernel<K><<<ceil_div(2 * nbk + 2, NT), NT, 0, e->stream>>>(ak, Count{S, S_dev, S}, bk, L, B - T, nbk, kmask,
                                                                           e->bk_rstart.p, e->bk_vstart.p, &dm->flags);
     e->timer.end(e->stream);
     if (e->n_cu == 0) {
         HIP_TRY(hipDeviceGetAttribute(&e->n_cu, hipDeviceAttributeMultiprocessorCount, e->device));
         if (e->n_cu <= 0) e->n_cu = 1;
     }
-    const int64_t grid = std::min(nbk, (int64_t)e->n_cu * BkShape<IPT>::WG_PER_CU);
+    const int64_t grid = std::min(nbk, (int64_t)e->n_cu * BkShape<IPT>::wgs(sizeof(K)));
     e->timer.begin("bucket_merge", e->stream, &ev);
     if (a.init_rule != 0)
-        bucket_merge_kernel<V, true, IPT><<<grid, BK_NT, 0, e->stream>>>(
-            a, ak, av, bk, bv, bo, e->bk_rstart.p, e->bk_vstart.p, nbk, B - T, e->slot_k.p, (V*)e->slot_v.p,
+        bucket_merge_kernel<K, V, true, IPT><<<grid, BK_NT, 0, e->stream>>>(
+            a, ak, av, bk, bv, bo, e->bk_rstart.p, e->bk_vstart.p, nbk, B - T, (K*)e->slot_k.p, (V*)e->slot_v.p,
             e->tile_cnt.p, e->merge_p.p, &dm->flags);
     else
-        bucket_merge_kernel<V, false, IPT><<<grid, BK_NT, 0, e->stream>>>(
-            a, ak, av, bk, bv, nullptr, e->bk_rstart.p, e->bk_vstart.p, nbk, B - T, e->slot_k.p, (V*)e->slot_v.p,
+        bucket_merge_kernel<K, V, false, IPT><<<grid, BK_NT, 0, e->stream>>>(
+            a, ak, av, bk, bv, nullptr, e->bk_rstart.p, e->bk_vstart.p, nbk, B - T, (K*)e->slot_k.p, (V*)e->slot_v.p,
             e->tile_cnt.p, e->merge_p.p, &dm->flags);
     e->timer.end(e->stream);
     HIP_TRY(hipGetLastError());
@@ -660,7 +666,7 @@ int bucket_merge_shape(rimu_engine* e, const StepArgs& a, const uint64_t* ak, co
     const bool raw = nbk <= COMPACT_RAW_MAX;
     if (!raw)
         if (int rc = scan_counts(e, e->tile_cnt.p, nbk)) return rc;
-    bucket_compact_kernel<V, IPT><<<nbk, NT, 0, e->stream>>>(e->slot_k.p, (const V*)e->slot_v.p, e->bk_rstart.p,
+    bucket_compact_kernel<K, V, IPT><<<nbk, NT, 0, e->stream>>>((const K*)e->slot_k.p, (const V*)e->slot_v.p, e->bk_rstart.p,
                                                              e->bk_vstart.p, e->tile_cnt.p, nbk, raw, ok, ov, cap,
                                                              &dm->L_new, &dm->flags);
     e->timer.end(e->stream);
@@ -668,15 +674,17 @@ int bucket_merge_shape(rimu_engine* e, const StepArgs& a, const uint64_t* ak, co
     return RIMU_OK;
 }
 
-template <class V>
-int bucket_merge_into(rimu_engine* e, const StepArgs& a, const uint64_t* ak, const V* av, int64_t S,
-                      const uint64_t* bk, const V* bv, const V* bo, int64_t L, const BucketCut& cut, uint64_t* ok,
+template <class K, class V>
+int bucket_merge_into(rimu_engine* e, const StepArgs& a, const K* ak, const V* av, int64_t S,
+                      const K* bk, const V* bv, const V* bo, int64_t L, const BucketCut& cut, K* ok,
                       V* ov, int64_t cap, rimu_engine::Misc* dm, int64_t* tiles, const int64_t* S_dev = nullptr) {
-    switch (cut.ipt) {
-        case 3: return bucket_merge_shape<V, 3>(e, a, ak, av, S, bk, bv, bo, L, cut.T, ok, ov, cap, dm, tiles, S_dev);
-        case 4: return bucket_merge_shape<V, 4>(e, a, ak, av, S, bk, bv, bo, L, cut.T, ok, ov, cap, dm, tiles, S_dev);
-        default: return bucket_merge_shape<V, 5>(e, a, ak, av, S, bk, bv, bo, L, cut.T, ok, ov, cap, dm, tiles, S_dev);
+    if (cut.ipt == 3)
+        return bucket_merge_shape<K, V, 3>(e, a, ak, av, S, bk, bv, bo, L, cut.T, ok, ov, cap, dm, tiles, S_dev);
+    if constexpr (sizeof(K) == 8) {
+        if (cut.ipt == 5)
+            return bucket_merge_shape<K, V, 5>(e, a, ak, av, S, bk, bv, bo, L, cut.T, ok, ov, cap, dm, tiles, S_dev);
     }
+    return bucket_merge_shape<K, V, 4>(e, a, ak, av, S, bk, bv, bo, L, cut.T, ok, ov, cap, dm, tiles, S_dev);
 }
 
 // A HubbardRealSpace model has off-diagonal elements of value zero (which the reference
@@ -710,11 +718,12 @@ int step_impl(rimu_engine* e, int64_t step, double shift, double dtau, double bo
     const bool rs = e->hdev.kind == RIMU_MODEL_HUBBARD_REAL_SPACE;
     const bool dense = !e->int_vals && e->style.proj_threshold == 0 && (!rs || !rs_zero_channels(e->hdev));
     const int nbits = e->hdev.B;
-    const bool bucket_ok = KW == 1 && e->radix_mode == 2 && e->bucket_cooldown == 0;
+    const bool bucket_ok = e->radix_mode == 2 && e->bucket_cooldown == 0;
     bool spec = e->spec_ok && e->radix_mode != 0 && e->W_prev > 0;
+    const int min_ipt = e->bucket_roomy > 0 ? BK_IPT_MAX : BK_IPT_MIN;
     BucketCut cut;
     // the path the counts of the last step choose; sorts with a host check stay synchronous
-    if (spec && bucket_ok) cut = bucket_cut(e->S_prev, L, nbits, e->mix.on, e->bucket_ipt_min);
+    if (spec && bucket_ok) cut = bucket_cut(e->S_prev, L, nbits, e->mix.on, min_ipt);
     const int64_t W_cap = spec ? e->W_prev + e->W_prev / 4 + 16 * SPAWN_TILE : 0;
 
     // 1. plan: diagonal step, attempt offsets and the first entry of each spawn tile (as
@@ -723,7 +732,7 @@ int step_impl(rimu_engine* e, int64_t step, double shift, double dtau, double bo
     HIP_TRY(e->plan_p.alloc((size_t)plan_tiles * 6));
     HIP_TRY(e->plan_status.alloc(plan_tiles));
     // tile ids and digit counts of the sort to come (a synchronous step's sort clears its own)
-    const int64_t sort_words = spec ? lb_words<K>(nbits, sort_from(e, cut)) : 0;
+    const int64_t sort_words = spec ? lb_words(nbits, sort_from(e, cut)) : 0;
     HIP_TRY(e->lb_part.alloc(sort_words));
     e->lb_cleared = sort_words;
     const ClearSet clear{{{(uint32_t*)dm, (int64_t)sizeof(rimu_engine::Misc) / 4},
@@ -847,8 +856,9 @@ int step_impl(rimu_engine* e, int64_t step, double shift, double dtau, double bo
     const int nxt = 1 - e->cur;
     int64_t merge_tiles = 0;
     int sorted = 0;
-    if (!spec && bucket_ok) cut = bucket_cut(S, L, nbits, e->mix.on, e->bucket_ipt_min);
+    if (!spec && bucket_ok) cut = bucket_cut(S, L, nbits, e->mix.on, min_ipt);
     if (e->bucket_cooldown > 0) --e->bucket_cooldown;
+    else if (e->bucket_roomy > 0) --e->bucket_roomy;
     const int64_t* merge_S_dev = S_dev;  // the merge path after the fallback sort reads S from the host
     auto merge_path = [&]() -> int {
         return merge_into<K, V>(e, a, (const K*)e->skeys[sorted].p, (const V*)e->svals[sorted].p, S, vk,
@@ -857,10 +867,10 @@ int step_impl(rimu_engine* e, int64_t step, double shift, double dtau, double bo
     };
     if (cut.T >= 0) {
         if (int rc = radix_sort<K, V>(e, S, nbits, kor ^ kand, 0, &sorted, nbits - cut.T, S_dev)) return rc;
-        if (int rc = bucket_merge_into<V>(e, a, (const uint64_t*)e->skeys[sorted].p, (const V*)e->svals[sorted].p,
-                                          S, (const uint64_t*)vk, (const V*)e->dvals.p, vv, L, cut,
-                                          (uint64_t*)e->vkeys[nxt].p, (V*)e->vvals[nxt].p, e->max_entries, dm,
-                                          &merge_tiles, S_dev)) return rc;
+        if (int rc = bucket_merge_into<K, V>(e, a, (const K*)e->skeys[sorted].p, (const V*)e->svals[sorted].p,
+                                             S, vk, (const V*)e->dvals.p, vv, L, cut,
+                                             (K*)e->vkeys[nxt].p, (V*)e->vvals[nxt].p, e->max_entries, dm,
+                                             &merge_tiles, S_dev)) return rc;
     } else {
         if (S > 1 || S_dev) {
             if (!e->mix.on || nbits <= e->sort_bits) {
@@ -955,7 +965,7 @@ int step_impl(rimu_engine* e, int64_t step, double shift, double dtau, double bo
         // sort the bucketed records on every bit (stable passes keep their list order within
         // an address) and merge along the merge path
         e->bucket_cooldown = BK_COOLDOWN;
-        e->bucket_ipt_min = BK_IPT_MAX;  // uneven counts: the roomiest buckets from now on
+        e->bucket_roomy = BK_ROOMY;  // uneven counts: the roomiest buckets for a while
         e->timer.begin("bucket_fallback", e->stream, &ev);
         e->timer.end(e->stream);
         HIP_TRY(hipMemsetAsync(&dm->flags, 0, sizeof(int), e->stream));
