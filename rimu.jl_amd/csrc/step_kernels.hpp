@@ -174,6 +174,11 @@ __global__ __launch_bounds__(NT) void plan_kernel(StepArgs a, const K* __restric
                                                   double* __restrict__ partials, int64_t* W_out) {
     __shared__ int64_t s_cnt[PLAN_TILE];  // counts, then exclusive offsets, in entry order
     __shared__ int64_t s_prefix;
+    // the dispersion table: every lane reads its own modes, one after another, which from the
+    // kernel arguments is a memory round trip each (1.25e7 entries on 16 modes 297 us, from
+    // LDS 224 us); the barriers of next_tile_id order it before its readers
+    __shared__ double s_kes[RS ? 1 : 64];
+    if (!RS && a.h.kind == 2 && threadIdx.x < 64) s_kes[threadIdx.x] = a.h.kes[threadIdx.x];
     const uint32_t tile = next_tile_id(tile_counter);
     const int64_t t0 = (int64_t)tile * PLAN_TILE;
     const double shift = a.shift_dev ? a.shift_dev[0] : a.shift;
@@ -195,7 +200,7 @@ __global__ __launch_bounds__(NT) void plan_kernel(StepArgs a, const K* __restric
             const K k = unmix_key(a.mix, kk[j]);  // the address
             const V v = vv[j];
             // diagonal_step!, spawning.jl:73-77 with diagonal_element(T) fciqmc.jl:93-96
-            const double hd = model_diagonal_element<RS>(a.h, k);
+            const double hd = model_diagonal_element<RS>(a.h, k, s_kes);
             const double d = 1 - a.dtau * (hd - shift);
             const double x = d * (double)v;
             double U = 0;
