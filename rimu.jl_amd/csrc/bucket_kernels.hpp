@@ -85,6 +85,23 @@ __global__ __launch_bounds__(NT) void bucket_bounds_kernel(const K* __restrict__
     (rec ? rstart : vstart)[b] = lo;
 }
 
+// First position in k[0, n) whose bucket (top bits, k >> shift) is at least b, by one
+// wavefront: 64 evenly spaced keys per round (three rounds for 2^18 keys).  Valid in every lane.
+template <class K>
+__device__ inline int64_t wave_bucket_bound(const K* __restrict__ k, int64_t n, int shift, K kmask, int64_t b, int lane) {
+    int64_t lo = 0, hi = n;
+    while (lo < hi) {
+        const int64_t step = (hi - lo + WAVE - 1) / WAVE;
+        const int64_t p = lo + lane * step;
+        const bool below = p < hi && (int64_t)((k[min(p, hi - 1)] & kmask) >> shift) < b;
+        const int c = __popcll(__ballot(below));  // the keys ascend: the first c probes are below
+        if (c == 0) break;
+        hi = min(hi, lo + c * step);
+        lo = lo + (c - 1) * step + 1;
+    }
+    return lo;
+}
+
 // LDS stores of this wavefront's lanes are seen by all its lanes after this point (the LDS
 // performs one wavefront's operations in order; the fences keep the compiler from moving
 // loads or stores across it).
@@ -142,8 +159,16 @@ struct BucketLds {
     int scan_i[BK_NT / WAVE];
 };
 
+// Where the workgroups find the bucket bounds themselves (no bucket_bounds_kernel, whose launch
+// and dependent searches took 5 to 8 us of a step): while every bucket has its own workgroup.
+struct OwnBounds {
+    int on;
+    Count S;
+    int64_t L;
+};
+
 // Bucket b = blockIdx.x, blockIdx.x + gridDim.x, ...; nbk buckets of which rstart/vstart give
-// the record and vector ranges.  Outputs per bucket: survivors at slot[rstart[b] + vstart[b]
+// the record and vector ranges (with own.on they are written first).  Outputs per bucket: survivors at slot[rstart[b] + vstart[b]
 // + i], their count in bucket_cnt[b], and partials[b], [nbk + b], [2 nbk + b] = len_before,
 // len, norm.
 // INIT (initiator rules): a record's key carries CLASS_BIT when its parent was not above the
@@ -154,8 +179,8 @@ struct BucketLds {
 template <class K, class V, bool INIT, int IPT>
 __global__ __launch_bounds__(BK_NT, 2 * BkShape<IPT>::wgs(sizeof(K))) void bucket_merge_kernel(
     StepArgs a, const K* __restrict__ ak, const V* __restrict__ av, const K* __restrict__ bk,
-    const V* __restrict__ bv, const V* __restrict__ bo, const int64_t* __restrict__ rstart, const int64_t* __restrict__ vstart, int64_t nbk,
-    int lowbits, K* __restrict__ slot_k, V* __restrict__ slot_v, int64_t* __restrict__ bucket_cnt,
+    const V* __restrict__ bv, const V* __restrict__ bo, int64_t* rstart, int64_t* vstart, int64_t nbk,
+    OwnBounds own, int lowbits, K* __restrict__ slot_k, V* __restrict__ slot_v, int64_t* __restrict__ bucket_cnt,
     double* __restrict__ partials, int* flags) {
     constexpr int NW = BK_NT / WAVE;
     constexpr uint64_t IDX_MASK = (1ull << BK_IDX_BITS) - 1ull;
@@ -164,8 +189,11 @@ __global__ __launch_bounds__(BK_NT, 2 * BkShape<IPT>::wgs(sizeof(K))) void bucke
     constexpr bool WIDE = sizeof(K) == 16;
     constexpr int WORD_KEY_BITS = 64 - BK_IDX_BITS;  // key bits of a packed word
     __shared__ BucketLds<K, V, INIT, IPT> sm;
-    // no sorted list to merge (raised by earlier kernels only: every wave reads the same bits)
-    if (*flags & (FLAG_LOOKBACK | FLAG_SPEC)) {
+    // no sorted list to merge (raised by earlier kernels, or by every workgroup's own look at the
+    // count: every wave takes the same branch)
+    const bool spec_miss = own.on && count_value(own.S) > own.S.cap;
+    if (spec_miss && blockIdx.x == 0 && threadIdx.x == 0) atomicOr(flags, FLAG_SPEC);
+    if (spec_miss || (*flags & (FLAG_LOOKBACK | FLAG_SPEC))) {
         for (int64_t b = blockIdx.x; b < nbk; b += gridDim.x) {
             if (threadIdx.x == 0) {
                 bucket_cnt[b] = 0;
@@ -226,6 +254,19 @@ __global__ __launch_bounds__(BK_NT, 2 * BkShape<IPT>::wgs(sizeof(K))) void bucke
             }
         }
     };
+    if (own.on) {
+        // one bucket per workgroup: wavefronts 0..3 find the bounds of its records and entries
+        // (neighbours write the same values)
+        const int w = threadIdx.x / WAVE;
+        if (w < 4) {
+            const K kmask = INIT ? (K)~class_bit<K>() : (K)~(K)0;
+            const int64_t bb = b + (w & 1);
+            const int64_t at = w < 2 ? wave_bucket_bound<K>(ak, count_value(own.S), lowbits, kmask, bb, threadIdx.x % WAVE)
+                                     : wave_bucket_bound<K>(bk, own.L, lowbits, kmask, bb, threadIdx.x % WAVE);
+            if (threadIdx.x % WAVE == 0) (w < 2 ? rstart : vstart)[bb] = at;
+        }
+        __syncthreads();
+    }
     if (b < nbk) load((int)threadIdx.x, b, ck, cv, ccls, r0, v0, na, nb);
     __syncthreads();  // sub-bucket counters cleared
 

@@ -418,13 +418,14 @@ int radix_sort_lb(rimu_engine* e, int64_t n, int nbits, u128 varying, int in, in
     uint32_t* part = e->lb_part.p + MAX_PASSES;
     radix_hist_all_kernel<K, RB><<<hblocks, NT, sizeof(uint32_t) * ps.n * copies * (NDIG + 1), e->stream>>>(
         (const K*)e->skeys[src].p, Count{n, n_dev, n}, flags, ps, copies, part);
-    radix_hist_base_kernel<RB><<<ps.n, NDIG, 0, e->stream>>>(part, ps.n, e->lb_hist.p);
+    const int rows = tiles <= SCATTER_BASE_TILES ? (int)std::min<int64_t>(hblocks, HIST_ROWS) : 0;
+    if (rows == 0) radix_hist_base_kernel<RB><<<ps.n, NDIG, 0, e->stream>>>(part, ps.n, e->lb_hist.p);
     e->timer.end(e->stream);
     for (int p = 0; p < ps.n; ++p) {
         e->timer.begin("radix_scatter", e->stream, &ev);
         radix_scatter_lb_kernel<K, V, RB><<<tiles, NDIG, 0, e->stream>>>(
             (const K*)e->skeys[src].p, (const V*)e->svals[src].p, Count{n, n_dev, n}, ps.shift[p], ps.dmask[p],
-            e->lb_hist.p + (int64_t)p * NDIG, e->lb_status.p + (int64_t)p * tiles * NDIG, epoch, counters + p,
+            DigitBase{e->lb_hist.p + (int64_t)p * NDIG, part + (int64_t)p * NDIG, rows, ps.n * NDIG}, e->lb_status.p + (int64_t)p * tiles * NDIG, epoch, counters + p,
             flags, LookbackCtl{e->lb_spin_limit, e->lb_withhold},
             (K*)e->skeys[1 - src].p, (V*)e->svals[1 - src].p);
         e->timer.end(e->stream);
@@ -641,24 +642,27 @@ int bucket_merge_shape(rimu_engine* e, const StepArgs& a, const K* ak, const V* 
     HIP_TRY(e->slot_k.alloc((size_t)(S + L) * KW));
     HIP_TRY(e->slot_v.alloc((size_t)(S + L)));
     hipEvent_t ev{};
-    const K kmask = a.init_rule != 0 ? (K)~class_bit<K>() : (K)~(K)0;
-    e->timer.begin("bucket_bounds", e->stream, &ev);
-    bucket_bounds_kernel<K><<<ceil_div(2 * nbk + 2, NT), NT, 0, e->stream>>>(ak, Count{S, S_dev, S}, bk, L, B - T, nbk, kmask,
-                                                                          e->bk_rstart.p, e->bk_vstart.p, &dm->flags);
-    e->timer.end(e->stream);
     if (e->n_cu == 0) {
         HIP_TRY(hipDeviceGetAttribute(&e->n_cu, hipDeviceAttributeMultiprocessorCount, e->device));
         if (e->n_cu <= 0) e->n_cu = 1;
     }
     const int64_t grid = std::min(nbk, (int64_t)e->n_cu * BkShape<IPT>::wgs(sizeof(K)));
+    const OwnBounds own{grid == nbk, Count{S, S_dev, S}, L};
+    if (!own.on) {
+        const K kmask = a.init_rule != 0 ? (K)~class_bit<K>() : (K)~(K)0;
+        e->timer.begin("bucket_bounds", e->stream, &ev);
+        bucket_bounds_kernel<K><<<ceil_div(2 * nbk + 2, NT), NT, 0, e->stream>>>(
+            ak, Count{S, S_dev, S}, bk, L, B - T, nbk, kmask, e->bk_rstart.p, e->bk_vstart.p, &dm->flags);
+        e->timer.end(e->stream);
+    }
     e->timer.begin("bucket_merge", e->stream, &ev);
     if (a.init_rule != 0)
         bucket_merge_kernel<K, V, true, IPT><<<grid, BK_NT, 0, e->stream>>>(
-            a, ak, av, bk, bv, bo, e->bk_rstart.p, e->bk_vstart.p, nbk, B - T, (K*)e->slot_k.p, (V*)e->slot_v.p,
+            a, ak, av, bk, bv, bo, e->bk_rstart.p, e->bk_vstart.p, nbk, own, B - T, (K*)e->slot_k.p, (V*)e->slot_v.p,
             e->tile_cnt.p, e->merge_p.p, &dm->flags);
     else
         bucket_merge_kernel<K, V, false, IPT><<<grid, BK_NT, 0, e->stream>>>(
-            a, ak, av, bk, bv, nullptr, e->bk_rstart.p, e->bk_vstart.p, nbk, B - T, (K*)e->slot_k.p, (V*)e->slot_v.p,
+            a, ak, av, bk, bv, nullptr, e->bk_rstart.p, e->bk_vstart.p, nbk, own, B - T, (K*)e->slot_k.p, (V*)e->slot_v.p,
             e->tile_cnt.p, e->merge_p.p, &dm->flags);
     e->timer.end(e->stream);
     HIP_TRY(hipGetLastError());

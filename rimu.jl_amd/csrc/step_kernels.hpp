@@ -983,6 +983,16 @@ __global__ __launch_bounds__(1 << RB) void radix_hist_base_kernel(const uint32_t
     hist[p * NDIG + threadIdx.x] = ex;
 }
 
+// Digit bases of a scatter: gbase[d] from radix_hist_base_kernel, or, with rows > 0, each tile
+// adds up the rows of digit counts itself (part[row * stride + d]) and scans them: for sorts of
+// a few tiles, whose rows are few, one launch less.
+struct DigitBase {
+    const uint32_t* gbase;
+    const uint32_t* part;
+    int rows, stride;
+};
+constexpr int64_t SCATTER_BASE_TILES = 64;  // most tiles (and rows) of a sort that does so
+
 // One thread per digit: 256 threads for 8-bit digits, 512 for 9-bit ones, on the same tiles.
 // Per-wavefront counts are at most TILE, so 16 bits hold them (a second workgroup of 512
 // threads fits the CU's LDS).
@@ -990,7 +1000,7 @@ template <class K, class V, int RB>
 __global__ __launch_bounds__(1 << RB) void radix_scatter_lb_kernel(const K* __restrict__ keys_in,
                                                                    const V* __restrict__ vals_in, Count cn,
                                                                    int shift, uint32_t dmask,
-                                                                   const uint32_t* __restrict__ gbase,
+                                                                   DigitBase base_of,
                                                                    uint64_t* status, uint32_t epoch,
                                                                    uint32_t* tile_counter, int* flags,
                                                                    LookbackCtl ctl,
@@ -1026,6 +1036,10 @@ __global__ __launch_bounds__(1 << RB) void radix_scatter_lb_kernel(const K* __re
 
     for (int j = threadIdx.x; j < NW * NDIG / 2; j += NTS) ((uint32_t*)&s_wcnt[0][0])[j] = 0;
     __syncthreads();
+
+    uint32_t digit_total = 0;  // of digit threadIdx.x over the whole list
+#pragma unroll 8
+    for (int b = 0; b < base_of.rows; ++b) digit_total += base_of.part[(int64_t)b * base_of.stride + threadIdx.x];
 
     K k[IPT];
     V v[IPT];
@@ -1068,6 +1082,7 @@ __global__ __launch_bounds__(1 << RB) void radix_scatter_lb_kernel(const K* __re
         }
         uint32_t tot;
         s_start[d] = block_exclusive_scan<uint32_t, NTS>(run, &tot);
+        s_goff[d] = base_of.rows > 0 ? block_exclusive_scan<uint32_t, NTS>(digit_total, &tot) : base_of.gbase[d];
         s_run[d] = run;
         if (tile != 0 || !ctl.withhold_first)
             lb_store(&status[(int64_t)tile * NDIG + d], (tile == 0 ? LB_FLAG_PFX : LB_FLAG_AGG) | tag | run);
@@ -1119,7 +1134,7 @@ __global__ __launch_bounds__(1 << RB) void radix_scatter_lb_kernel(const K* __re
             }
             lb_store(&status[(int64_t)tile * NDIG + d], LB_FLAG_PFX | tag | (pre + s_run[d]));
         }
-        s_goff[d] = gbase[d] + (uint32_t)pre;
+        s_goff[d] += (uint32_t)pre;
     }
     __syncthreads();
     const int64_t cnt_tile = min((int64_t)TILE, n - base);
