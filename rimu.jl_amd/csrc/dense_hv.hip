@@ -262,46 +262,58 @@ __global__ __launch_bounds__(DT) void rq_gradient_kernel(const double* __restric
     }
 }
 
-// One three-term Lanczos update per right-hand side: w -= alpha_j v_j + beta_j v_{j-1},
-// with alpha_j and beta_j^2 read from device memory, and the partial sums of |w|^2 of each
-// block written to partials[R][blocks] (reduced in order afterwards).
+// 1 / sqrt(n2), or zero where the norm has fallen to `floor2` or below: a right-hand side whose
+// Krylov space is exhausted goes on with zero vectors.
+__device__ inline double lanczos_scale(double n2, double floor2) { return n2 > floor2 ? 1.0 / sqrt(n2) : 0.0; }
+
+// One three-term Lanczos update per right-hand side.  The vectors are kept unnormalised with
+// their squared norms in device memory: v_j = x / sqrt(x2), v_{j-1} = y / sqrt(y2), and w = H x,
+// so H v_j = w / sqrt(x2) and alpha_j = <v_j|H v_j> = xw / x2.  Writes
+// w <- H v_j - alpha_j v_j - beta_j v_{j-1} (beta_j = sqrt(x2), the norm x had as w) with the
+// partial sums of |w|^2 of each block in partials[R][blocks], and alpha_j.  (Writing v_{j+1} out
+// was a pass of its own: 7.7 of 46 us an iteration at dimension 352,716, R = 4.)
 template <int R>
-__global__ __launch_bounds__(DT) void lanczos_orth_kernel(double* __restrict__ w, const double* __restrict__ v,
-                                                          const double* __restrict__ vprev,
-                                                          const double* __restrict__ alpha,
-                                                          const double* __restrict__ beta2, int64_t D,
+__global__ __launch_bounds__(DT) void lanczos_orth_kernel(double* __restrict__ w, const double* __restrict__ x,
+                                                          const double* __restrict__ y,
+                                                          const double* __restrict__ xw, const double* __restrict__ x2,
+                                                          const double* __restrict__ y2, double floor_x, double floor_y, int first,
+                                                          int64_t D, double* __restrict__ alpha,
                                                           double* __restrict__ partials) {
     __shared__ double s_sum[R][DT / WAVE];
+    __shared__ double s_c[4][R];
+    // the row's loads travel while one thread per right-hand side prepares the scalars (square
+    // roots and divisions in every thread, or before the loads, cost 15 to 19 us a call)
     const int64_t r = (int64_t)blockIdx.x * DT + threadIdx.x;
+    const int64_t rc = min(r, D - 1);
+    double wr[R], xr[R], yr[R];
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+        wr[i] = w[rc * R + i];
+        xr[i] = x[rc * R + i];
+        yr[i] = first ? 0.0 : y[rc * R + i];
+    }
+    if (threadIdx.x < R) {
+        const int i = threadIdx.x;
+        const double s = lanczos_scale(x2[i], floor_x);
+        s_c[0][i] = s;
+        s_c[1][i] = first ? 0.0 : lanczos_scale(y2[i], floor_y);
+        s_c[2][i] = (xw[i] * s) * s;
+        s_c[3][i] = first ? 0.0 : sqrt(x2[i]);
+        if (blockIdx.x == 0) alpha[i] = s_c[2][i];
+    }
+    __syncthreads();
     double ps[R];
 #pragma unroll
     for (int i = 0; i < R; ++i) {
-        double x = 0;
-        if (r < D) {
-            x = w[r * R + i] - alpha[i] * v[r * R + i] - sqrt(beta2[i]) * vprev[r * R + i];
-            w[r * R + i] = x;
-        }
-        ps[i] = x * x;
+        const double sx = s_c[0][i], vp = yr[i] * s_c[1][i];
+        const double z = wr[i] * sx - s_c[2][i] * (xr[i] * sx) - s_c[3][i] * vp;
+        if (r < D) w[r * R + i] = z;
+        ps[i] = r < D ? z * z : 0.0;
     }
     block_sums<DT, R>(ps, s_sum);
     if (threadIdx.x == 0)
 #pragma unroll
         for (int i = 0; i < R; ++i) partials[(int64_t)i * gridDim.x + blockIdx.x] = ps[i];
-}
-
-// out = w / sqrt(norm2) per right-hand side; a right-hand side whose norm fell to
-// `floor2` or below (its Krylov space is exhausted) gets the zero vector.
-template <int R>
-__global__ __launch_bounds__(DT) void lanczos_scale_kernel(const double* __restrict__ w,
-                                                           const double* __restrict__ norm2, double floor2,
-                                                           int64_t D, double* __restrict__ out) {
-    const int64_t r = (int64_t)blockIdx.x * DT + threadIdx.x;
-    if (r >= D) return;
-#pragma unroll
-    for (int i = 0; i < R; ++i) {
-        const double n2 = norm2[i];
-        out[r * R + i] = n2 > floor2 ? w[r * R + i] / sqrt(n2) : 0.0;
-    }
 }
 
 }  // namespace
@@ -439,28 +451,30 @@ int rq_gradient(rimu_dense* d, const double* v, const double* hv, const double* 
 }
 
 template <int R>
-int launch_lanczos(rimu_dense* d, double* w, const double* v, const double* vprev, const double* alpha,
-                   const double* beta2, double* norm2_out, double* vnext, double floor2) {
+int launch_lanczos(rimu_dense* d, double* w, const double* x, const double* y, const double* xw, const double* x2,
+                   const double* y2, double floor_x, double floor_y, int first, double* alpha,
+                   double* norm2_out) {
     const int64_t blocks = ceil_div(d->D, DT);
     HIP_TRY(d->partials.alloc((size_t)blocks * R));
-    lanczos_orth_kernel<R><<<blocks, DT, 0, d->stream>>>(w, v, vprev, alpha, beta2, d->D, d->partials.p);
+    lanczos_orth_kernel<R><<<blocks, DT, 0, d->stream>>>(w, x, y, xw, x2, y2, floor_x, floor_y, first, d->D, alpha,
+                                                         d->partials.p);
     reduce_rows_kernel<<<R, RED_NT, 0, d->stream>>>(d->partials.p, blocks, norm2_out, 0);
-    lanczos_scale_kernel<R><<<blocks, DT, 0, d->stream>>>(w, norm2_out, floor2, d->D, vnext);
     HIP_TRY(hipGetLastError());
     return RIMU_OK;
 }
 
-int lanczos_update(rimu_dense* d, double* w, const double* v, const double* vprev, const double* alpha,
-                   const double* beta2, double* norm2_out, double* vnext, double floor2) {
+int lanczos_update(rimu_dense* d, double* w, const double* x, const double* y, const double* xw, const double* x2,
+                   const double* y2, double floor_x, double floor_y, int first, double* alpha,
+                   double* norm2_out) {
     switch (d->R) {
-        case 1: return launch_lanczos<1>(d, w, v, vprev, alpha, beta2, norm2_out, vnext, floor2);
-        case 2: return launch_lanczos<2>(d, w, v, vprev, alpha, beta2, norm2_out, vnext, floor2);
-        case 3: return launch_lanczos<3>(d, w, v, vprev, alpha, beta2, norm2_out, vnext, floor2);
-        case 4: return launch_lanczos<4>(d, w, v, vprev, alpha, beta2, norm2_out, vnext, floor2);
-        case 5: return launch_lanczos<5>(d, w, v, vprev, alpha, beta2, norm2_out, vnext, floor2);
-        case 6: return launch_lanczos<6>(d, w, v, vprev, alpha, beta2, norm2_out, vnext, floor2);
-        case 7: return launch_lanczos<7>(d, w, v, vprev, alpha, beta2, norm2_out, vnext, floor2);
-        default: return launch_lanczos<8>(d, w, v, vprev, alpha, beta2, norm2_out, vnext, floor2);
+        case 1: return launch_lanczos<1>(d, w, x, y, xw, x2, y2, floor_x, floor_y, first, alpha, norm2_out);
+        case 2: return launch_lanczos<2>(d, w, x, y, xw, x2, y2, floor_x, floor_y, first, alpha, norm2_out);
+        case 3: return launch_lanczos<3>(d, w, x, y, xw, x2, y2, floor_x, floor_y, first, alpha, norm2_out);
+        case 4: return launch_lanczos<4>(d, w, x, y, xw, x2, y2, floor_x, floor_y, first, alpha, norm2_out);
+        case 5: return launch_lanczos<5>(d, w, x, y, xw, x2, y2, floor_x, floor_y, first, alpha, norm2_out);
+        case 6: return launch_lanczos<6>(d, w, x, y, xw, x2, y2, floor_x, floor_y, first, alpha, norm2_out);
+        case 7: return launch_lanczos<7>(d, w, x, y, xw, x2, y2, floor_x, floor_y, first, alpha, norm2_out);
+        default: return launch_lanczos<8>(d, w, x, y, xw, x2, y2, floor_x, floor_y, first, alpha, norm2_out);
     }
 }
 
@@ -743,29 +757,30 @@ int rimu_dense_ground_state(rimu_dense* d, const double* v0, int64_t max_iters, 
     double a_h[MAXR], b_h[MAXR];
     for (int i = 0; i < R; ++i) { a_h[i] = 0; b_h[i] = 1; }
     const DenseParams pH = params(d, a_h, b_h);
-    DevBuf<double>&v = d->x, &vprev = d->y, &w = d->z, &hist = d->hist;  // kept with the handle
-    // hist: alpha [cap][R], then beta^2 [cap + 1][R] (beta^2[0] = 0), then |v0|^2 [R]
+    DevBuf<double>&x = d->x, &y = d->y, &w = d->z, &hist = d->hist;  // kept with the handle
+    // hist: alpha [cap][R], then beta^2 [cap + 1][R] (beta^2[0] = 0 in the tridiagonal matrix, its
+    // place holds |v0|^2 = x2 of the first iteration on the device), then <x|Hx> [R]
     auto run = [&]() -> int {
-        HIP_TRY(v.alloc(n));
-        HIP_TRY(vprev.alloc(n));
+        HIP_TRY(x.alloc(n));
+        HIP_TRY(y.alloc(n));
         HIP_TRY(w.alloc(n));
         HIP_TRY(hist.alloc((size_t)(2 * cap + 2) * R));
         double* alpha = hist.p;
         double* beta2 = hist.p + cap * R;
-        double* n0 = hist.p + (2 * cap + 1) * R;
-        HIP_TRY(hipMemsetAsync(hist.p, 0, (size_t)(2 * cap + 2) * R * 8, d->stream));
-        HIP_TRY(hipMemsetAsync(vprev.p, 0, n * 8, d->stream));
-        HIP_TRY(hipMemcpyAsync(w.p, v0, n * 8, hipMemcpyHostToDevice, d->stream));
-        // v_0 = v0 / |v0| (lanczos_update with alpha = beta = 0 only normalises)
-        if (int rc = lanczos_update(d, w.p, vprev.p, vprev.p, beta2, beta2, n0, v.p, 0.0)) return rc;
+        double* xw = hist.p + (2 * cap + 1) * R;
+        HIP_TRY(hipMemcpyAsync(x.p, v0, n * 8, hipMemcpyHostToDevice, d->stream));
+        if (int rc = dot(d, x.p, x.p, beta2)) return rc;
         std::vector<double> h_a, h_b2, h_n0(R), last(R, INFINITY), cur(R);
         std::vector<int64_t> m_eff(R, -1);
         int64_t j = 0;
         for (; j < cap; ++j) {
-            if (int rc = apply(d, pH, v.p, w.p, alpha + j * R)) return rc;
-            if (int rc = lanczos_update(d, w.p, v.p, vprev.p, alpha + j * R, beta2 + j * R,
-                                        beta2 + (j + 1) * R, vprev.p, FLOOR2)) return rc;
-            std::swap(v, vprev);
+            // x: the unnormalised v_j of squared norm beta2[j], y: that of v_{j-1}
+            if (int rc = apply(d, pH, x.p, w.p, xw)) return rc;
+            if (int rc = lanczos_update(d, w.p, x.p, y.p, xw, beta2 + j * R, beta2 + (j > 0 ? j - 1 : 0) * R,
+                                        j > 0 ? FLOOR2 : 0.0, j > 1 ? FLOOR2 : 0.0, j == 0, alpha + j * R,
+                                        beta2 + (j + 1) * R)) return rc;
+            std::swap(y, x);
+            std::swap(x, w);
             const bool last_iter = j + 1 == cap;
             if ((j + 1) % CHECK != 0 && !last_iter) continue;
             const int64_t m = j + 1;
@@ -773,8 +788,8 @@ int rimu_dense_ground_state(rimu_dense* d, const double* v0, int64_t max_iters, 
             h_b2.resize((size_t)(m + 1) * R);
             HIP_TRY(hipMemcpyAsync(h_a.data(), alpha, (size_t)m * R * 8, hipMemcpyDeviceToHost, d->stream));
             HIP_TRY(hipMemcpyAsync(h_b2.data(), beta2, (size_t)(m + 1) * R * 8, hipMemcpyDeviceToHost, d->stream));
-            HIP_TRY(hipMemcpyAsync(h_n0.data(), n0, R * 8, hipMemcpyDeviceToHost, d->stream));
             HIP_TRY(hipStreamSynchronize(d->stream));
+            for (int i = 0; i < R; ++i) h_n0[i] = h_b2[i];
             bool done = true;
             std::vector<double> a(m), b2(m + 1);
             for (int i = 0; i < R; ++i) {
