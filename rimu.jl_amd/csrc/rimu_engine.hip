@@ -3,9 +3,10 @@
 // One engine = one FCIQMC state: a sorted device vector (keys u64, values int64 or f64),
 // double buffered, plus the working memory of a step (diagonal values, work offsets, the
 // spawn list and its sort buffers, look-back status words, per-tile partial sums).
-// All work of an engine is ordered on its own HIP stream.  A step synchronises with the
-// host three times (work-item count, spawn count, statistics) so that every grid is sized
-// to the data it covers.
+// All work of an engine is ordered on its own HIP stream.  A step's grids
+// are sized from the last step's counts and it synchronises with the host once, for its
+// statistics; the first step after an upload, and one whose counts outgrew its grids, reads the
+// work-item and spawn counts back as well.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -702,6 +703,10 @@ bool rs_zero_channels(const ModelDev& h) {
     return false;
 }
 
+// One attempt per thread, four times as many spawn tiles, while the compaction still places so
+// many without a scan.
+bool short_spawn_tiles(int64_t W) { return ceil_div(W, spawn_tile(SPAWN_ITEMS_SHORT)) <= COMPACT_RAW_MAX; }
+
 template <class K, class V>
 int step_impl(rimu_engine* e, int64_t step, double shift, double dtau, double boost,
               rimu_step_stats* out) {
@@ -728,11 +733,13 @@ int step_impl(rimu_engine* e, int64_t step, double shift, double dtau, double bo
     BucketCut cut;
     // the path the counts of the last step choose; sorts with a host check stay synchronous
     if (spec && bucket_ok) cut = bucket_cut(e->S_prev, L, nbits, e->mix.on, min_ipt);
-    const int64_t W_cap = spec ? e->W_prev + e->W_prev / 4 + 16 * SPAWN_TILE : 0;
+    const int64_t W_cap = spec ? e->W_prev + e->W_prev / 4 + 16 * spawn_tile(SPAWN_ITEMS) : 0;
+    int spawn_items = spec && short_spawn_tiles(W_cap) ? SPAWN_ITEMS_SHORT : SPAWN_ITEMS;
 
     // 1. plan: diagonal step, attempt offsets and the first entry of each spawn tile (as
     // many as the tile_first buffer holds; the rest below if W needs more)
-    const int64_t plan_tiles = ceil_div(L + 1, PLAN_TILE);
+    const bool short_plan = L < PLAN_SHORT_MAX;
+    const int64_t plan_tiles = ceil_div(L + 1, NT * (short_plan ? PLAN_IPT_SHORT : PLAN_IPT));
     HIP_TRY(e->plan_p.alloc((size_t)plan_tiles * 6));
     HIP_TRY(e->plan_status.alloc(plan_tiles));
     // tile ids and digit counts of the sort to come (a synchronous step's sort clears its own)
@@ -744,17 +751,17 @@ int step_impl(rimu_engine* e, int64_t step, double shift, double dtau, double bo
                           {e->lb_part.p, sort_words}}};
     static_assert(sizeof(rimu_engine::Misc) % 4 == 0 && sizeof(rimu_engine::Misc) / 4 <= WAVE, "cleared and copied as words");
     clear_kernel<<<std::min<int64_t>(ceil_div(2 * plan_tiles + sort_words, NT), 256), NT, 0, e->stream>>>(clear);
-    if (spec) HIP_TRY(e->tile_first.alloc(ceil_div(W_cap, SPAWN_TILE) + 1));
-    const int64_t tf_cap = (int64_t)e->tile_first.n;
+    // a synchronous step chooses its spawn tiles when it knows the number of attempts
+    if (spec) HIP_TRY(e->tile_first.alloc(ceil_div(W_cap, spawn_tile(spawn_items)) + 1));
+    const int64_t tf_cap = spec ? (int64_t)e->tile_first.n : 0;
     e->timer.begin("plan", e->stream, &ev);
-    if (rs)
-        plan_kernel<K, V, true><<<plan_tiles, NT, 0, e->stream>>>(a, vk, vv, L, (V*)e->dvals.p, e->woff.p,
-                                                               e->tile_first.p, tf_cap, e->plan_status.p,
-                                                               &dm->plan_counter, &dm->flags, e->plan_p.p, &dm->W);
-    else
-        plan_kernel<K, V, false><<<plan_tiles, NT, 0, e->stream>>>(a, vk, vv, L, (V*)e->dvals.p, e->woff.p,
-                                                                e->tile_first.p, tf_cap, e->plan_status.p,
-                                                                &dm->plan_counter, &dm->flags, e->plan_p.p, &dm->W);
+    auto plan = [&](auto kernel) {
+        kernel<<<plan_tiles, NT, 0, e->stream>>>(a, vk, vv, L, (V*)e->dvals.p, e->woff.p, e->tile_first.p, tf_cap,
+                                                 spawn_shift(spawn_items), e->plan_status.p, &dm->plan_counter,
+                                                 &dm->flags, e->plan_p.p, &dm->W);
+    };
+    if (short_plan) plan(rs ? plan_kernel<K, V, true, PLAN_IPT_SHORT> : plan_kernel<K, V, false, PLAN_IPT_SHORT>);
+    else plan(rs ? plan_kernel<K, V, true, PLAN_IPT> : plan_kernel<K, V, false, PLAN_IPT>);
     e->timer.end(e->stream);
     HIP_TRY(hipGetLastError());
     int64_t W = W_cap;  // synchronous: the count; speculative: the most the grids are sized for
@@ -773,7 +780,9 @@ int step_impl(rimu_engine* e, int64_t step, double shift, double dtau, double bo
     u128 kor = 0, kand = ~(u128)0;
     const int64_t* S_dev = nullptr;  // speculative: the record count in device memory
     if (W > 0) {
-        spawn_tiles = ceil_div(W, SPAWN_TILE);
+        if (!spec && short_spawn_tiles(W)) spawn_items = SPAWN_ITEMS_SHORT;
+        const int64_t tile_size = spawn_tile(spawn_items);
+        spawn_tiles = ceil_div(W, tile_size);
         // every attempt yields a record when values are floating and deposits unprojected,
         // unless the model has zero-valued channels (hard walls, Pauli blocking: the
         // reference never deposits their spawns)
@@ -786,35 +795,32 @@ int step_impl(rimu_engine* e, int64_t step, double shift, double dtau, double bo
         HIP_TRY(e->tile_and.alloc((size_t)spawn_tiles * KW));
         if (spawn_tiles > tf_cap) {  // plan filled only the first tf_cap tile heads
             HIP_TRY(e->tile_first.alloc(spawn_tiles));
-            tile_first_kernel<<<ceil_div(L, NT), NT, 0, e->stream>>>(e->woff.p, L, e->tile_first.p);
+            tile_first_kernel<<<ceil_div(L, NT), NT, 0, e->stream>>>(e->woff.p, L, spawn_shift(spawn_items),
+                                                                     e->tile_first.p);
         }
         K* sk = (K*)e->skeys[0].p;
         V* sv = (V*)e->svals[0].p;
         if (!dense) {
-            HIP_TRY(e->slot_k.alloc((size_t)spawn_tiles * SPAWN_TILE * KW));
-            HIP_TRY(e->slot_v.alloc((size_t)spawn_tiles * SPAWN_TILE));
+            HIP_TRY(e->slot_k.alloc((size_t)spawn_tiles * tile_size * KW));
+            HIP_TRY(e->slot_v.alloc((size_t)spawn_tiles * tile_size));
             HIP_TRY(e->tile_cnt.alloc(spawn_tiles + 1));
             sk = (K*)e->slot_k.p;
             sv = (V*)e->slot_v.p;
         }
-        const Count cA{W, spec ? &dm->W : nullptr, spawn_tiles * SPAWN_TILE};
+        const Count cA{W, spec ? &dm->W : nullptr, spawn_tiles * tile_size};
         e->timer.begin("spawn", e->stream, &ev);
-        if (dense && rs)
-            spawn_kernel<K, V, true, true><<<spawn_tiles, NT, 0, e->stream>>>(
-                a, vk, vv, L, e->woff.p, cA, e->max_spawns, &dm->flags, sk, sv, e->tile_cnt.p, e->spawn_p.p,
-                e->tile_first.p, (K*)e->tile_or.p, (K*)e->tile_and.p);
-        else if (dense)
-            spawn_kernel<K, V, true, false><<<spawn_tiles, NT, 0, e->stream>>>(
-                a, vk, vv, L, e->woff.p, cA, e->max_spawns, &dm->flags, sk, sv, e->tile_cnt.p, e->spawn_p.p,
-                e->tile_first.p, (K*)e->tile_or.p, (K*)e->tile_and.p);
-        else if (rs)
-            spawn_kernel<K, V, false, true><<<spawn_tiles, NT, 0, e->stream>>>(
-                a, vk, vv, L, e->woff.p, cA, e->max_spawns, &dm->flags, sk, sv, e->tile_cnt.p, e->spawn_p.p,
-                e->tile_first.p, (K*)e->tile_or.p, (K*)e->tile_and.p);
-        else
-            spawn_kernel<K, V, false, false><<<spawn_tiles, NT, 0, e->stream>>>(
-                a, vk, vv, L, e->woff.p, cA, e->max_spawns, &dm->flags, sk, sv, e->tile_cnt.p, e->spawn_p.p,
-                e->tile_first.p, (K*)e->tile_or.p, (K*)e->tile_and.p);
+        auto spawn = [&](auto kernel) {
+            kernel<<<spawn_tiles, NT, 0, e->stream>>>(a, vk, vv, L, e->woff.p, cA, e->max_spawns, &dm->flags, sk, sv,
+                                                      e->tile_cnt.p, e->spawn_p.p, e->tile_first.p,
+                                                      (K*)e->tile_or.p, (K*)e->tile_and.p);
+        };
+        auto spawn_by = [&](auto items) {
+            constexpr int N = decltype(items)::value;
+            if (dense) spawn(rs ? spawn_kernel<K, V, true, true, N> : spawn_kernel<K, V, true, false, N>);
+            else spawn(rs ? spawn_kernel<K, V, false, true, N> : spawn_kernel<K, V, false, false, N>);
+        };
+        if (spawn_items == SPAWN_ITEMS) spawn_by(std::integral_constant<int, SPAWN_ITEMS>{});
+        else spawn_by(std::integral_constant<int, SPAWN_ITEMS_SHORT>{});
         e->timer.end(e->stream);
         HIP_TRY(hipGetLastError());
         if (!spec)  // a speculative step sorts every digit and reads no OR/AND back
@@ -825,7 +831,9 @@ int step_impl(rimu_engine* e, int64_t step, double shift, double dtau, double bo
             const bool raw = spawn_tiles <= COMPACT_RAW_MAX;
             if (!raw)
                 if (int rc = scan_counts(e, e->tile_cnt.p, spawn_tiles)) return rc;
-            compact_kernel<K, V, SPAWN_ITEMS, FLAG_SPAWN_OVERFLOW><<<spawn_tiles, NT, 0, e->stream>>>(
+            const auto compact = spawn_items == SPAWN_ITEMS ? compact_kernel<K, V, SPAWN_ITEMS, FLAG_SPAWN_OVERFLOW>
+                                                            : compact_kernel<K, V, SPAWN_ITEMS_SHORT, FLAG_SPAWN_OVERFLOW>;
+            compact<<<spawn_tiles, NT, 0, e->stream>>>(
                 (const K*)e->slot_k.p, (const V*)e->slot_v.p, e->tile_cnt.p, spawn_tiles, raw, (K*)e->skeys[0].p,
                 (V*)e->svals[0].p, e->max_spawns, &dm->S, &dm->flags);
             e->timer.end(e->stream);

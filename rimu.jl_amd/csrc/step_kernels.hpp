@@ -27,7 +27,6 @@ constexpr int MERGE_IPT = 8;     // merged positions per thread (one-chunk keys)
 // against 3.67 ms with 8, 3.20 with 10, 3.17 with 14 and 5.36 ms with 16; the 64-bit merge
 // is fastest with 8 (1.09 ms against 1.82 ms with 12).
 template <class K> struct merge_ipt { static constexpr int value = sizeof(K) == 8 ? MERGE_IPT : 12; };
-constexpr int SPAWN_TILE_SIZE = 1024;  // attempts per spawn tile (NT * SPAWN_ITEMS)
 constexpr int RADIX_BITS = 8;
 constexpr int RADIX = 1 << RADIX_BITS;
 constexpr int SORT_IPT = 16;     // keys per thread per radix tile
@@ -156,23 +155,26 @@ __global__ __launch_bounds__(NT) void clear_kernel(ClearSet cs) {
 // ---------------------------------------------------------------------------------------
 // plan: the diagonal step and the number of spawn attempts of every entry, the exclusive
 // scan of the attempt counts (aoff, L + 1 values; aoff[L] = W, also written to *W_out), and
-// the first entry of every spawn tile (tile_first[t] = entry holding attempt t*SPAWN_TILE,
-// for t < tf_cap).  Thread x of tile t handles the PLAN_IPT consecutive entries
-// t*PLAN_TILE + x*PLAN_IPT + j; tiles are placed by the decoupled look-back (tile ids in
+// the first entry of every spawn tile (tile_first[t] = entry holding attempt t << sp_shift,
+// for t < tf_cap).  A tile has NT * IPT entries, thread x scans IPT consecutive ones; tiles are placed by the decoupled look-back (tile ids in
 // start order, so every tile waited on is running).
 // partials[j * gridDim.x + tile], j = 0..5: deaths, clones, zombies, exact, inexact, attempts.
 // ---------------------------------------------------------------------------------------
-constexpr int PLAN_IPT = 8;
-constexpr int PLAN_TILE = NT * PLAN_IPT;
+// A short vector (up to one short tile per CU) takes tiles of two entries per thread: its tiles
+// run side by side and a tile's time is the length of a thread's work.  One entry per thread is no
+// faster (more tiles to look back over), and long vectors keep eight for the same reason.
+constexpr int PLAN_IPT = 8, PLAN_IPT_SHORT = 2;
+constexpr int64_t PLAN_SHORT_MAX = 256 * NT * PLAN_IPT_SHORT;
 
-template <class K, class V, bool RS>
+template <class K, class V, bool RS, int IPT>
 __global__ __launch_bounds__(NT) void plan_kernel(StepArgs a, const K* __restrict__ keys,
                                                   const V* __restrict__ vals, int64_t L,
                                                   V* __restrict__ dvals, int64_t* __restrict__ aoff,
-                                                  int64_t* __restrict__ tile_first, int64_t tf_cap,
+                                                  int64_t* __restrict__ tile_first, int64_t tf_cap, int sp_shift,
                                                   uint64_t* status, uint32_t* tile_counter, int* flags,
                                                   double* __restrict__ partials, int64_t* W_out) {
-    __shared__ int64_t s_cnt[PLAN_TILE];  // counts, then exclusive offsets, in entry order
+    constexpr int TILE = NT * IPT;
+    __shared__ int64_t s_cnt[TILE > 6 * NT ? TILE : 6 * NT];  // counts, then exclusive offsets, in entry order
     __shared__ int64_t s_prefix;
     // the dispersion table: every lane reads its own modes, one after another, which from the
     // kernel arguments is a memory round trip each (1.25e7 entries on 16 modes 297 us, from
@@ -180,20 +182,20 @@ __global__ __launch_bounds__(NT) void plan_kernel(StepArgs a, const K* __restric
     __shared__ double s_kes[RS ? 1 : 64];
     if (!RS && a.h.kind == 2 && threadIdx.x < 64) s_kes[threadIdx.x] = a.h.kes[threadIdx.x];
     const uint32_t tile = next_tile_id(tile_counter);
-    const int64_t t0 = (int64_t)tile * PLAN_TILE;
+    const int64_t t0 = (int64_t)tile * TILE;
     const double shift = a.shift_dev ? a.shift_dev[0] : a.shift;
     double st[6] = {0, 0, 0, 0, 0, 0};
     // striped: entry t0 + j*NT + x (coalesced loads and stores)
-    K kk[PLAN_IPT];
-    V vv[PLAN_IPT];
+    K kk[IPT];
+    V vv[IPT];
 #pragma unroll
-    for (int j = 0; j < PLAN_IPT; ++j) {  // all loads in flight before any is used
+    for (int j = 0; j < IPT; ++j) {  // all loads in flight before any is used
         const int64_t i = min(t0 + j * NT + threadIdx.x, max(L - 1, (int64_t)0));
         kk[j] = L > 0 ? keys[i] : 0;
         vv[j] = L > 0 ? vals[i] : (V)0;
     }
 #pragma unroll
-    for (int j = 0; j < PLAN_IPT; ++j) {
+    for (int j = 0; j < IPT; ++j) {
         const int64_t i = t0 + j * NT + threadIdx.x;
         int64_t n_items = 0;
         if (i < L) {
@@ -225,11 +227,11 @@ __global__ __launch_bounds__(NT) void plan_kernel(StepArgs a, const K* __restric
         s_cnt[j * NT + threadIdx.x] = n_items;
     }
     __syncthreads();
-    // blocked: thread x scans the PLAN_IPT consecutive entries x*PLAN_IPT + j
-    const int b0 = (int)threadIdx.x * PLAN_IPT;
+    // blocked: thread x scans the IPT consecutive entries x*IPT + j
+    const int b0 = (int)threadIdx.x * IPT;
     int64_t sum = 0;
 #pragma unroll
-    for (int j = 0; j < PLAN_IPT; ++j) sum += s_cnt[b0 + j];
+    for (int j = 0; j < IPT; ++j) sum += s_cnt[b0 + j];
     int64_t total;
     const int64_t ex = block_exclusive_scan<int64_t, NT>(sum, &total);  // ends with a barrier
     if (threadIdx.x < WAVE) {
@@ -239,13 +241,13 @@ __global__ __launch_bounds__(NT) void plan_kernel(StepArgs a, const K* __restric
     __syncthreads();
     int64_t run = s_prefix + ex;
 #pragma unroll
-    for (int j = 0; j < PLAN_IPT; ++j) {
+    for (int j = 0; j < IPT; ++j) {
         const int64_t i = t0 + b0 + j;
         const int64_t c = s_cnt[b0 + j];
         s_cnt[b0 + j] = run;
         if (i < L) {
             const int64_t end = run + c;
-            for (int64_t t = (run + SPAWN_TILE_SIZE - 1) / SPAWN_TILE_SIZE; t * SPAWN_TILE_SIZE < end && t < tf_cap; ++t)
+            for (int64_t t = (run + (1 << sp_shift) - 1) >> sp_shift; t << sp_shift < end && t < tf_cap; ++t)
                 tile_first[t] = i;
         } else if (i == L) {
             aoff[L] = run;
@@ -255,7 +257,7 @@ __global__ __launch_bounds__(NT) void plan_kernel(StepArgs a, const K* __restric
     }
     __syncthreads();
 #pragma unroll
-    for (int j = 0; j < PLAN_IPT; ++j) {
+    for (int j = 0; j < IPT; ++j) {
         const int64_t i = t0 + j * NT + threadIdx.x;
         if (i < L) aoff[i] = s_cnt[j * NT + threadIdx.x];
     }
@@ -335,20 +337,24 @@ __global__ __launch_bounds__(NT) void scan_add_kernel(T* __restrict__ out, int64
 // ---------------------------------------------------------------------------------------
 // spawn: one thread per spawn attempt.  Attempts are numbered entry by entry (attempt j of
 // entry i is aoff[i] + j), so consecutive lanes hold consecutive attempts and the lane
-// order is the (entry, attempt) order.  Each thread handles SPAWN_ITEMS attempts, strided
-// by NT within the tile.  Nonzero records are compacted with a wavefront ballot and
+// order is the (entry, attempt) order.  Each thread handles ITEMS attempts, strided by NT
+// within the tile.  Nonzero records are compacted with a wavefront ballot and
 // popcount prefix; the (item, wavefront) counts are scanned across the workgroup and the
 // tile's records go to its own slot range with their count in tile_cnt (compact_kernel
 // places them).  When every attempt yields a record (DENSE: floating values without
 // projection) the record of attempt a is simply written at position a.
 // Also writes sum |spawn| and the key OR/AND (which radix digits vary) of the tile.
 // ---------------------------------------------------------------------------------------
-constexpr int SPAWN_ITEMS = 4;
-constexpr int SPAWN_TILE = NT * SPAWN_ITEMS;
-static_assert(SPAWN_TILE % NT == 0, "whole slots per thread in the entry scan");
-static_assert(SPAWN_TILE == SPAWN_TILE_SIZE, "plan and spawn agree on the spawn tile");
+// Short lists of attempts take one per thread, which fills four times as many wavefronts; longer
+// ones four, for fewer tiles to scan and place.  With the short plan tiles: 1000 steps of 5e4
+// walkers on 50 sites 104 -> 93.5 ms, 1500 of 4e4 initiator walkers in momentum space 147 -> 135 ms.
+constexpr int SPAWN_ITEMS = 4, SPAWN_ITEMS_SHORT = 1;
+constexpr int64_t spawn_tile(int items) { return (int64_t)NT * items; }
+constexpr int spawn_shift(int items) { return items == SPAWN_ITEMS ? 10 : 8; }
+static_assert((1 << spawn_shift(SPAWN_ITEMS)) == spawn_tile(SPAWN_ITEMS) &&
+              (1 << spawn_shift(SPAWN_ITEMS_SHORT)) == spawn_tile(SPAWN_ITEMS_SHORT), "tiles are powers of two");
 
-template <class K, class V, bool DENSE, bool RS>
+template <class K, class V, bool DENSE, bool RS, int ITEMS>
 __global__ __launch_bounds__(NT) void spawn_kernel(StepArgs a, const K* __restrict__ keys,
                                                    const V* __restrict__ vals, int64_t L,
                                                    const int64_t* __restrict__ aoff, Count cA,
@@ -361,11 +367,12 @@ __global__ __launch_bounds__(NT) void spawn_kernel(StepArgs a, const K* __restri
                                                    K* __restrict__ tile_or,
                                                    K* __restrict__ tile_and) {
     constexpr int NW = NT / WAVE;
-    constexpr int WIN = SPAWN_TILE + 1;
+    constexpr int TILE = NT * ITEMS;
+    constexpr int WIN = TILE + 1;
     __shared__ int64_t s_aoff[WIN];
-    __shared__ int s_head[SPAWN_TILE];  // per attempt slot: window index of its entry
+    __shared__ int s_head[TILE];  // per attempt slot: window index of its entry
     __shared__ int s_wmax[NW];
-    __shared__ int s_cnt[SPAWN_ITEMS * NW];
+    __shared__ int s_cnt[ITEMS * NW];
     __shared__ int s_total;
     __shared__ K s_kor[NW], s_kand[NW];
 
@@ -373,7 +380,7 @@ __global__ __launch_bounds__(NT) void spawn_kernel(StepArgs a, const K* __restri
     const int lane = threadIdx.x & (WAVE - 1);
     const int wid = threadIdx.x / WAVE;
     const uint64_t lt_mask = (1ull << lane) - 1ull;
-    const int64_t a0 = (int64_t)tile * SPAWN_TILE;
+    const int64_t a0 = (int64_t)tile * TILE;
     const int64_t A = count_value(cA);
     // attempts beyond the grid (FLAG_SPEC) or, dense, beyond the spawn buffer: nothing is
     // written; tiles past the attempts leave neutral partials (uniform branches)
@@ -405,7 +412,7 @@ __global__ __launch_bounds__(NT) void spawn_kernel(StepArgs a, const K* __restri
             if (t < WIN) s_aoff[t] = w[r];
         }
 #pragma unroll
-        for (int r = 0; r < SPAWN_ITEMS; ++r) s_head[(int)threadIdx.x + r * NT] = 0;
+        for (int r = 0; r < ITEMS; ++r) s_head[(int)threadIdx.x + r * NT] = 0;
         __syncthreads();
         // entry t of the window (0 < t < WIN-1) starts at attempt s_aoff[t]: mark that slot.
         // Entries without attempts share the start of the next one; the larger index wins,
@@ -415,13 +422,13 @@ __global__ __launch_bounds__(NT) void spawn_kernel(StepArgs a, const K* __restri
             const int t = (int)threadIdx.x + r * NT;
             if (t >= 1 && t < WIN - 1 && e0 + t < L) {
                 const int64_t p = w[r] - a0;
-                if (p >= 0 && p < SPAWN_TILE) atomicMax(&s_head[p], t);
+                if (p >= 0 && p < TILE) atomicMax(&s_head[p], t);
             }
         }
         __syncthreads();
         // inclusive max-scan over the slots: slot q then holds the entry of attempt a0 + q
         {
-            constexpr int Q = SPAWN_TILE / NT;
+            constexpr int Q = TILE / NT;
             const int q0 = (int)threadIdx.x * Q;
             int m[Q];
             int run = 0;
@@ -449,17 +456,17 @@ __global__ __launch_bounds__(NT) void spawn_kernel(StepArgs a, const K* __restri
     }
     __syncthreads();
 
-    K rk[SPAWN_ITEMS];
-    V rv[SPAWN_ITEMS];
-    int rpos[SPAWN_ITEMS];
-    bool rok[SPAWN_ITEMS];
+    K rk[ITEMS];
+    V rv[ITEMS];
+    int rpos[ITEMS];
+    bool rok[ITEMS];
     double spawned = 0;
     K kor = 0, kand = (K)~(K)0;
     // entry of each attempt: last i with aoff[i] <= att (every entry has at least one
     // attempt unless it has no off-diagonals; outside the window: global search)
-    int64_t ent[SPAWN_ITEMS], aidx[SPAWN_ITEMS];
+    int64_t ent[ITEMS], aidx[ITEMS];
 #pragma unroll
-    for (int it = 0; it < SPAWN_ITEMS; ++it) {
+    for (int it = 0; it < ITEMS; ++it) {
         const int64_t att = a0 + (int64_t)it * NT + threadIdx.x;
         int64_t i = e0, ai = att;
         if (att < A) {
@@ -481,18 +488,18 @@ __global__ __launch_bounds__(NT) void spawn_kernel(StepArgs a, const K* __restri
         aidx[it] = ai;
     }
     // the entries' keys and values, all loads in flight at once (e0 < L whenever A > 0)
-    K ekey[SPAWN_ITEMS];
-    V eval[SPAWN_ITEMS];
+    K ekey[ITEMS];
+    V eval[ITEMS];
 #pragma unroll
-    for (int it = 0; it < SPAWN_ITEMS; ++it) {
+    for (int it = 0; it < ITEMS; ++it) {
         const int64_t i = min(ent[it], L - 1);
         ekey[it] = keys[i];
         eval[it] = vals[i];
     }
 #pragma unroll
-    for (int it = 0; it < SPAWN_ITEMS; ++it) ekey[it] = unmix_key(a.mix, ekey[it]);  // addresses
+    for (int it = 0; it < ITEMS; ++it) ekey[it] = unmix_key(a.mix, ekey[it]);  // addresses
 #pragma unroll
-    for (int it = 0; it < SPAWN_ITEMS; ++it) {
+    for (int it = 0; it < ITEMS; ++it) {
         const int64_t att = a0 + (int64_t)it * NT + threadIdx.x;
         bool ok = false;
         K nb = 0;
@@ -541,14 +548,14 @@ __global__ __launch_bounds__(NT) void spawn_kernel(StepArgs a, const K* __restri
         // exclusive scan of the (item, wavefront) counts: attempt order within the tile
         if (threadIdx.x == 0) {
             int run = 0;
-            for (int q = 0; q < SPAWN_ITEMS * NW; ++q) { const int c = s_cnt[q]; s_cnt[q] = run; run += c; }
+            for (int q = 0; q < ITEMS * NW; ++q) { const int c = s_cnt[q]; s_cnt[q] = run; run += c; }
             s_total = run;
         }
         __syncthreads();
         total = s_total;
     }
 #pragma unroll
-    for (int it = 0; it < SPAWN_ITEMS; ++it) {
+    for (int it = 0; it < ITEMS; ++it) {
         if (rok[it]) {
             const int64_t pos = DENSE ? a0 + (int64_t)it * NT + threadIdx.x
                                       : a0 + s_cnt[it * NW + wid] + rpos[it];
@@ -641,13 +648,13 @@ __global__ __launch_bounds__(NT) void fixup_sort_kernel(K* __restrict__ keys, V*
 }
 
 // First entry of every spawn tile: entry i owns attempts [aoff[i], aoff[i+1]); the tile
-// starting at attempt t*SPAWN_TILE belongs first to the entry whose range contains it.
+// starting at attempt t << sp_shift belongs first to the entry whose range contains it.
 __global__ __launch_bounds__(NT) void tile_first_kernel(const int64_t* __restrict__ aoff, int64_t L,
-                                                        int64_t* __restrict__ tile_first) {
+                                                        int sp_shift, int64_t* __restrict__ tile_first) {
     const int64_t i = (int64_t)blockIdx.x * NT + threadIdx.x;
     if (i >= L) return;
     const int64_t c0 = aoff[i], c1 = aoff[i + 1];
-    for (int64_t t = (c0 + SPAWN_TILE - 1) / SPAWN_TILE; t * SPAWN_TILE < c1; ++t) tile_first[t] = i;
+    for (int64_t t = (c0 + (1 << sp_shift) - 1) >> sp_shift; t << sp_shift < c1; ++t) tile_first[t] = i;
 }
 
 // Merge-path split of every merge tile boundary d = t*TILE (clamped to S+L): number of A
