@@ -161,25 +161,30 @@ struct BucketLds {
 
 // Where the workgroups find the bucket bounds themselves (no bucket_bounds_kernel, whose launch
 // and dependent searches took 5 to 8 us of a step): while every bucket has its own workgroup.
+// The kernel is built without that part for larger steps: with it the bounds are no longer
+// read-only to the compiler, which then reads them through the vector cache (1.5e8 items in 2^17
+// buckets 2.95 ms with the part compiled in, 2.80 without).
 struct OwnBounds {
-    int on;
     Count S;
     int64_t L;
 };
 
 // Bucket b = blockIdx.x, blockIdx.x + gridDim.x, ...; nbk buckets of which rstart/vstart give
-// the record and vector ranges (with own.on they are written first).  Outputs per bucket: survivors at slot[rstart[b] + vstart[b]
-// + i], their count in bucket_cnt[b], and partials[b], [nbk + b], [2 nbk + b] = len_before,
+// the record and vector ranges (OWN: they are written first).  Outputs per bucket: survivors at
+// slot[rstart[b] + vstart[b] + i], their count in bucket_cnt[b], and partials[b], [nbk + b], [2 nbk + b] = len_before,
 // len, norm.
 // INIT (initiator rules): a record's key carries CLASS_BIT when its parent was not above the
 // initiator threshold, a vector entry has the class when its old value bo is not above it;
 // each address folds three components in list order -- safe (entries with the class, records
 // without), unsafe (records with the class), initiator (entries without) -- exists when one
 // is nonzero and takes the rule's value (initiator_value), as merge_kernel<K, V, true> does.
-template <class K, class V, bool INIT, int IPT>
+template <bool OWN> struct BucketStartsOf { using type = const int64_t* __restrict__; };
+template <> struct BucketStartsOf<true> { using type = int64_t*; };
+template <bool OWN> using BucketStarts = typename BucketStartsOf<OWN>::type;
+template <class K, class V, bool INIT, int IPT, bool OWN>
 __global__ __launch_bounds__(BK_NT, 2 * BkShape<IPT>::wgs(sizeof(K))) void bucket_merge_kernel(
     StepArgs a, const K* __restrict__ ak, const V* __restrict__ av, const K* __restrict__ bk,
-    const V* __restrict__ bv, const V* __restrict__ bo, int64_t* rstart, int64_t* vstart, int64_t nbk,
+    const V* __restrict__ bv, const V* __restrict__ bo, BucketStarts<OWN> rstart, BucketStarts<OWN> vstart, int64_t nbk,
     OwnBounds own, int lowbits, K* __restrict__ slot_k, V* __restrict__ slot_v, int64_t* __restrict__ bucket_cnt,
     double* __restrict__ partials, int* flags) {
     constexpr int NW = BK_NT / WAVE;
@@ -191,7 +196,7 @@ __global__ __launch_bounds__(BK_NT, 2 * BkShape<IPT>::wgs(sizeof(K))) void bucke
     __shared__ BucketLds<K, V, INIT, IPT> sm;
     // no sorted list to merge (raised by earlier kernels, or by every workgroup's own look at the
     // count: every wave takes the same branch)
-    const bool spec_miss = own.on && count_value(own.S) > own.S.cap;
+    const bool spec_miss = OWN && count_value(own.S) > own.S.cap;
     if (spec_miss && blockIdx.x == 0 && threadIdx.x == 0) atomicOr(flags, FLAG_SPEC);
     if (spec_miss || (*flags & (FLAG_LOOKBACK | FLAG_SPEC))) {
         for (int64_t b = blockIdx.x; b < nbk; b += gridDim.x) {
@@ -254,7 +259,7 @@ __global__ __launch_bounds__(BK_NT, 2 * BkShape<IPT>::wgs(sizeof(K))) void bucke
             }
         }
     };
-    if (own.on) {
+    if constexpr (OWN) {
         // one bucket per workgroup: wavefronts 0..3 find the bounds of its records and entries
         // (neighbours write the same values)
         const int w = threadIdx.x / WAVE;

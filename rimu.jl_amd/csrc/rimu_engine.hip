@@ -667,8 +667,9 @@ int bucket_merge_shape(rimu_engine* e, const StepArgs& a, const K* ak, const V* 
         if (e->n_cu <= 0) e->n_cu = 1;
     }
     const int64_t grid = std::min(nbk, (int64_t)e->n_cu * BkShape<IPT>::wgs(sizeof(K)));
-    const OwnBounds own{grid == nbk, Count{S, S_dev, S}, L};
-    if (!own.on) {
+    const bool own_bounds = grid == nbk;
+    const OwnBounds own{Count{S, S_dev, S}, L};
+    if (!own_bounds) {
         const K kmask = a.init_rule != 0 ? (K)~class_bit<K>() : (K)~(K)0;
         e->timer.begin("bucket_bounds", e->stream, &ev);
         bucket_bounds_kernel<K><<<ceil_div(2 * nbk + 2, NT), NT, 0, e->stream>>>(
@@ -676,14 +677,15 @@ int bucket_merge_shape(rimu_engine* e, const StepArgs& a, const K* ak, const V* 
         e->timer.end(e->stream);
     }
     e->timer.begin("bucket_merge", e->stream, &ev);
-    if (a.init_rule != 0)
-        bucket_merge_kernel<K, V, true, IPT><<<grid, BK_NT, 0, e->stream>>>(
-            a, ak, av, bk, bv, bo, e->bk_rstart.p, e->bk_vstart.p, nbk, own, B - T, (K*)e->slot_k.p, (V*)e->slot_v.p,
-            e->tile_cnt.p, e->merge_p.p, &dm->flags);
-    else
-        bucket_merge_kernel<K, V, false, IPT><<<grid, BK_NT, 0, e->stream>>>(
-            a, ak, av, bk, bv, nullptr, e->bk_rstart.p, e->bk_vstart.p, nbk, own, B - T, (K*)e->slot_k.p, (V*)e->slot_v.p,
-            e->tile_cnt.p, e->merge_p.p, &dm->flags);
+    auto merge = [&](auto kernel) {
+        kernel<<<grid, BK_NT, 0, e->stream>>>(a, ak, av, bk, bv, a.init_rule != 0 ? bo : nullptr, e->bk_rstart.p,
+                                              e->bk_vstart.p, nbk, own, B - T, (K*)e->slot_k.p, (V*)e->slot_v.p,
+                                              e->tile_cnt.p, e->merge_p.p, &dm->flags);
+    };
+    if (a.init_rule != 0 && own_bounds) merge(bucket_merge_kernel<K, V, true, IPT, true>);
+    else if (a.init_rule != 0) merge(bucket_merge_kernel<K, V, true, IPT, false>);
+    else if (own_bounds) merge(bucket_merge_kernel<K, V, false, IPT, true>);
+    else merge(bucket_merge_kernel<K, V, false, IPT, false>);
     e->timer.end(e->stream);
     HIP_TRY(hipGetLastError());
     e->timer.begin("compact", e->stream, &ev);
