@@ -235,9 +235,11 @@ int rimu_overlaps(rimu_engine* left, rimu_engine* right, const rimu_operator* op
 int rimu_engine_set_sort_bits(rimu_engine* e, int32_t bits);
 
 /* (No counterpart in the reference; for tests and tuning.)  Sort and merge of the spawn
- * records.  2 (default): where eligible (one-word keys of more than 20 bits, at least 4096
- * records), sort on the top bits of the stored keys only and merge bucket by bucket, each
- * bucket's records and vector entries sorted and folded in LDS; other steps as 1.  1: one histogram
+ * records.  2 (default): sort on the top bits of the stored keys only and merge bucket by
+ * bucket, each bucket's records and vector entries sorted and folded in LDS; a step that fits
+ * one bucket is not sorted at all.  Keys of at most 20 bits are not mixed, so larger steps on
+ * them go as 1, as does a step whose key bits below the buckets do not fit a bucket's words
+ * or whose spread overfilled a bucket.  1: one histogram
  * pass for every digit and scatters that find their offsets by a look-back over the tiles
  * before them, then the merge path.  0: as 1 with counts per pass and a scan between passes.
  * All give the same step results. */

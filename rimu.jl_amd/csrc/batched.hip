@@ -407,7 +407,7 @@ __device__ void sort_phase(RunState* __restrict__ runs, const Pools& P, int run,
         // counters of its own, 64 records a round and no barrier between rounds, then one scan
         // of the counts places them: five barriers a pass whatever S is.  (Passing through in
         // chunks of one record per thread took two barriers a chunk: the sort of 64 runs of up to
-        // 1e5 walkers 27.7 us then, 20 us now, tile boundaries
+        // 1e5 walkers 27.7 us then, 20.7 us now, tile boundaries
         // included.)
         constexpr int RND = SORT_LDS_CAP / NT;
         const int per = ((int)S + NW * WAVE - 1) / (NW * WAVE) * WAVE;

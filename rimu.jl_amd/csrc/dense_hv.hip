@@ -91,10 +91,10 @@ __device__ inline int64_t dense_tile(int64_t b, int64_t n) {
 // sum over hops of -sqrt * v[neighbour][i]; returns sum n(n - 1) / 2 of the address.
 // One pass over the M - 1 bonds and the boundary, both directions of a bond from the same
 // occupations, the same instructions in every lane: a hop that the address does not have loads
-// the row itself and adds zero.  Bound by instruction issue: per bond two table reads, two
-// gathers of 8R bytes and 2R fused multiply-adds.  (Walking each lane's own occupied modes
-// with popcounts, clz and an f64 sqrt per hop took 106 us per product at dimension 1,352,078,
-// R = 4; see the figures at dense_apply_kernel.)
+// the row itself and adds zero.  Per bond two table reads, two gathers of 8R bytes and 2R fused
+// multiply-adds.  Bound by the gathers that miss the L2: at dimension 1,352,078, R = 4 they
+// bring in 265 MB a product (v alone is 43 MB) at 4.8 TB/s.  (Walking each lane's own occupied
+// modes with popcounts, clz and an f64 sqrt per hop took 106 us a product there.)
 template <int R>
 __device__ inline int hop_sum(uint64_t bits, int64_t r, int M, int row_len, uint2 rot,
                               const double* s_root, const uint32_t* s_delta,
