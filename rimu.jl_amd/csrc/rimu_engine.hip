@@ -582,8 +582,10 @@ int reorder_on_device(rimu_engine* e, int64_t n, int forward, int* result, Fill&
 // keys 52 of them there and the rest in the low word
 constexpr int BK_MAX_LOWBITS = 48, BK_MAX_LOWBITS_WIDE = 116;
 constexpr int BK_IPT_MAX_WIDE = 4;   // two-word buckets of five items per thread leave one workgroup a CU
-constexpr int BK_COOLDOWN = 16;      // steps on the merge path after a bucket overflowed
-constexpr int BK_ROOMY = 256;        // steps with the largest shape after that
+constexpr int BK_COOLDOWN = 16;      // steps on the merge path after a bucket overflowed the largest shape
+constexpr int BK_ROOMY = 256;        // steps with the largest shape after a bucket overflowed any
+
+int max_bucket_ipt(int B) { return B > 64 ? BK_IPT_MAX_WIDE : BK_IPT_MAX; }
 
 // How a step's records are cut into buckets: the top T stored-key bits, and the kernel shape
 // (items per thread) that holds a bucket.  T = 0: one bucket, no radix pass.
@@ -610,7 +612,7 @@ double bucket_mean_max(int ipt) {
 // the merge path, 66 us so); more buckets need mixed keys, whose top bits are spread evenly.
 BucketCut bucket_cut(int64_t S, int64_t L, int B, bool mixed, int min_ipt) {
     const double items = (double)S + (double)L;
-    const int max_ipt = B > 64 ? BK_IPT_MAX_WIDE : BK_IPT_MAX;
+    const int max_ipt = max_bucket_ipt(B);
     const int max_low = B > 64 ? BK_MAX_LOWBITS_WIDE : BK_MAX_LOWBITS;
     BucketCut cut;
     cut.T = B > 64 ? std::max(B - max_low, 0) : 0;  // at most 2^12 buckets more than the items need
@@ -902,12 +904,14 @@ int step_impl(rimu_engine* e, int64_t step, double shift, double dtau, double bo
                                 (const V*)e->dvals.p, L, (K*)e->vkeys[nxt].p, (V*)e->vvals[nxt].p,
                                 e->max_entries, dm, &merge_tiles, vv, merge_S_dev);
     };
+    auto bucket_merge = [&]() -> int {
+        return bucket_merge_into<K, V>(e, a, (const K*)e->skeys[sorted].p, (const V*)e->svals[sorted].p, S, vk,
+                                       (const V*)e->dvals.p, vv, L, cut, (K*)e->vkeys[nxt].p, (V*)e->vvals[nxt].p,
+                                       e->max_entries, dm, &merge_tiles, S_dev);
+    };
     if (cut.T >= 0) {
         if (int rc = radix_sort<K, V>(e, S, nbits, kor ^ kand, 0, &sorted, nbits - cut.T, S_dev)) return rc;
-        if (int rc = bucket_merge_into<K, V>(e, a, (const K*)e->skeys[sorted].p, (const V*)e->svals[sorted].p,
-                                             S, vk, (const V*)e->dvals.p, vv, L, cut,
-                                             (K*)e->vkeys[nxt].p, (V*)e->vvals[nxt].p, e->max_entries, dm,
-                                             &merge_tiles, S_dev)) return rc;
+        if (int rc = bucket_merge()) return rc;
     } else {
         if (S > 1 || S_dev) {
             if (!e->mix.on || nbits <= e->sort_bits) {
@@ -998,6 +1002,16 @@ int step_impl(rimu_engine* e, int64_t step, double shift, double dtau, double bo
         return rc;
     }
     if (e->h_misc->flags & FLAG_LOOKBACK) return fail(RIMU_ERR_INTERNAL, "radix look-back did not complete");
+    if ((e->h_misc->flags & FLAG_BUCKET_OVERFLOW) && cut.ipt < max_bucket_ipt(nbits)) {
+        // the same buckets fit the largest shape more often than not: merge them again
+        e->bucket_roomy = BK_ROOMY;
+        e->timer.begin("bucket_retry", e->stream, &ev);
+        e->timer.end(e->stream);
+        HIP_TRY(hipMemsetAsync(&dm->flags, 0, sizeof(int), e->stream));
+        cut.ipt = max_bucket_ipt(nbits);
+        if (int rc = bucket_merge()) return rc;
+        if (int rc = finish()) return rc;
+    }
     if (e->h_misc->flags & FLAG_BUCKET_OVERFLOW) {
         // sort the bucketed records on every bit (stable passes keep their list order within
         // an address) and merge along the merge path
