@@ -87,6 +87,19 @@ __device__ inline int64_t dense_tile(int64_t b, int64_t n) {
     return b < per * 8 ? (b & 7) * per + (b >> 3) : b;
 }
 
+// acc[i] += -s_root[x] * v[k][i], or zero where the row r has no such hop (it loads itself).
+template <int R>
+__device__ inline void add_hop(bool has, int64_t r, int64_t k, int x, const double* s_root,
+                               const double* __restrict__ v, double (&acc)[R]) {
+    const double* vk = v + (has ? k : r) * R;
+    const double amp = -s_root[has ? x : 0];
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+        const double y = vk[i];
+        acc[i] = fma(amp, has ? y : 0.0, acc[i]);
+    }
+}
+
 // K v at row r (K: the hopping with unit amplitude, elements -sqrt(n (n' + 1))): acc[i] =
 // sum over hops of -sqrt * v[neighbour][i]; returns sum n(n - 1) / 2 of the address.
 // One pass over the M - 1 bonds and the boundary, both directions of a bond from the same
@@ -96,22 +109,13 @@ __device__ inline int64_t dense_tile(int64_t b, int64_t n) {
 // bring in 265 MB a product (v alone is 43 MB) at 4.8 TB/s.  (Walking each lane's own occupied
 // modes with popcounts, clz and an f64 sqrt per hop took 106 us a product there.)
 template <int R>
-__device__ inline int hop_sum(uint64_t bits, int64_t r, int M, int row_len, uint2 rot,
-                              const double* s_root, const uint32_t* s_delta,
-                              const double* __restrict__ v, double (&acc)[R]) {
+__device__ inline int hop_sum_bonds(uint64_t bits, int64_t r, int M, int row_len, uint2 rot,
+                                    const double* s_root, const uint32_t* s_delta,
+                                    const double* __restrict__ v, double (&acc)[R]) {
 #pragma unroll
     for (int i = 0; i < R; ++i) acc[i] = 0.0;
-    auto add = [&](bool has, int64_t k, int x) {
-        const double* vk = v + (has ? k : r) * R;
-        const double amp = -s_root[has ? x : 0];
-#pragma unroll
-        for (int i = 0; i < R; ++i) {
-            const double y = vk[i];
-            acc[i] = fma(amp, has ? y : 0.0, acc[i]);
-        }
-    };
     uint64_t x = bits;
-    const int n1 = __builtin_ctzll(~x);  // B < 64 or a full lowest mode: ~x has a bit (see below)
+    const int n1 = __builtin_ctzll(~x);  // M >= 2: an address has a zero bit
     x = shr(x, n1 + 1);
     int nc = n1, s = n1;
     int pairs = n1 * (n1 - 1) / 2;
@@ -120,19 +124,66 @@ __device__ inline int hop_sum(uint64_t bits, int64_t r, int M, int row_len, uint
     for (int m = 1; m < M; ++m, dl += row_len) {
         const int nn = ctz64(~x);
         x = shr(x, nn + 1);
-        add(nc > 0, r + dl[s], nc * (nn + 1));
-        add(nn > 0, r - (int64_t)dl[s + 1], nn * (nc + 1));
+        add_hop<R>(nc > 0, r, r + dl[s], nc * (nn + 1), s_root, v, acc);
+        add_hop<R>(nn > 0, r, r - (int64_t)dl[s + 1], nn * (nc + 1), s_root, v, acc);
         s += nn;
         nc = nn;
         pairs += nn * (nn - 1) / 2;
     }
-    add(nc > 0, rot.x, nc * (n1 + 1));
-    add(n1 > 0, rot.y, n1 * (nc + 1));
+    add_hop<R>(nc > 0, r, rot.x, nc * (n1 + 1), s_root, v, acc);
+    add_hop<R>(n1 > 0, r, rot.y, n1 * (nc + 1), s_root, v, acc);
     return pairs;
 }
 
+// The same sum over the occupied modes only, left hop then right hop, modes ascending: the
+// hops in the order of their bonds, so the same additions and the same bits as hop_sum_bonds.
+template <int R>
+__device__ inline int hop_sum_occupied(uint64_t bits, int64_t r, int M, int row_len, uint2 rot,
+                                       const double* s_root, const uint32_t* s_delta,
+                                       const double* __restrict__ v, double (&acc)[R]) {
+#pragma unroll
+    for (int i = 0; i < R; ++i) acc[i] = 0.0;
+    const int n1 = __builtin_ctzll(~bits);
+    uint64_t x = bits;
+    int m = 1, n = 0, s = 0, pairs = 0;  // the last run's mode and bosons, the bosons so far
+    while (x) {
+        const int z = __builtin_ctzll(x);  // modes further on
+        const int before = z == 1 ? n : 0;
+        m += z;
+        x >>= z;
+        n = ctz64(~x);
+        x = shr(x, n);
+        const int after = __builtin_ctzll(~(x >> 1));
+        add_hop<R>(m > 1, r, r - (int64_t)s_delta[(m - 1) * row_len + s + 1], n * (before + 1), s_root, v, acc);
+        s += n;
+        add_hop<R>(m < M, r, r + s_delta[(m < M ? m : 0) * row_len + s], n * (after + 1), s_root, v, acc);
+        pairs += n * (n - 1) / 2;
+    }
+    const int nM = m == M ? n : 0;
+    add_hop<R>(nM > 0, r, rot.x, nM * (n1 + 1), s_root, v, acc);
+    add_hop<R>(n1 > 0, r, rot.y, n1 * (nM + 1), s_root, v, acc);
+    return pairs;
+}
+
+template <int R, bool OCC>
+__device__ inline int hop_sum(uint64_t bits, int64_t r, int M, int row_len, uint2 rot, const double* s_root,
+                              const uint32_t* s_delta, const double* __restrict__ v, double (&acc)[R]) {
+    return OCC ? hop_sum_occupied<R>(bits, r, M, row_len, rot, s_root, s_delta, v, acc)
+               : hop_sum_bonds<R>(bits, r, M, row_len, rot, s_root, s_delta, v, acc);
+}
+
+// Whether a product walks the occupied modes instead of all bonds.  A wavefront takes as many turns
+// as its fullest row has occupied modes, up to N, against M: but a turn that finds a run costs more
+// than a bond, and a bond that holds no boson only loads its own row (8R bytes, from the caches).
+// Where the line lies, in ms for 200 projector steps with their adjoint, walk against bonds:
+//   R = 4: N/M = 0.07 (60 modes) 14.5 : 48.2, 0.25 (24) 14.6 : 22.0, 0.42 (12) 4.1 : 4.2,
+//          0.50 (12) 4.4 : 4.2, 0.64 (14) 17.5 : 17.5, 1 (12) 43.4 : 38.8
+//   R = 1: 0.42 3.35 : 3.35, 0.50 3.6 : 3.4, 0.64 8.0 : 7.9, 1 17.2 : 15.0
+//   R = 8: 0.50 (16) 40.0 : 47.9, 0.67 (12) 10.3 : 12.0, 0.83 (12) 32.6 : 31.2 (5 and 6 alike)
+bool walk_occupied(int M, int N, int R) { return R > 4 ? 3 * N <= 2 * M : 2 * N < M; }
+
 // w = (a + b H) v, one thread per row.  DOT: also per-block partials[i][block] of <v|w>.
-template <int R, bool DOT>
+template <int R, bool DOT, bool OCC>
 __global__ __launch_bounds__(DT) void dense_apply_kernel(const uint64_t* __restrict__ basis,
                                                          const uint2* __restrict__ rot, int64_t D,
                                                          DenseParams p, HopTables t,
@@ -148,7 +199,7 @@ __global__ __launch_bounds__(DT) void dense_apply_kernel(const uint64_t* __restr
     for (int i = 0; i < R; ++i) dt[i] = 0.0;
     if (r < D) {
         double acc[R];
-        const double dr = (double)hop_sum<R>(basis[r], r, p.M, p.N + 2, rot[r], s_tab, s_delta, v, acc);
+        const double dr = (double)hop_sum<R, OCC>(basis[r], r, p.M, p.N + 2, rot[r], s_tab, s_delta, v, acc);
 #pragma unroll
         for (int i = 0; i < R; ++i) {
             const double vr = v[r * R + i];
@@ -169,7 +220,7 @@ __global__ __launch_bounds__(DT) void dense_apply_kernel(const uint64_t* __restr
 // Pullback: vbar = (a + b H) ybar; per-block partial sums of b <ybar|D|v> and b <ybar|K|v>
 // written to partials[2R][blocks].  K is real symmetric, so <ybar|K|v> = sum_r v_r (K ybar)_r
 // and only ybar is gathered at the neighbours.
-template <int R>
+template <int R, bool OCC>
 __global__ __launch_bounds__(DT) void dense_pullback_kernel(const uint64_t* __restrict__ basis,
                                                             const uint2* __restrict__ rot, int64_t D,
                                                             DenseParams p, HopTables t,
@@ -188,7 +239,7 @@ __global__ __launch_bounds__(DT) void dense_pullback_kernel(const uint64_t* __re
     for (int i = 0; i < 2 * R; ++i) ps[i] = 0.0;
     if (r < D) {
         double ky[R];
-        const double dr = (double)hop_sum<R>(basis[r], r, p.M, p.N + 2, rot[r], s_tab, s_delta, ybar, ky);
+        const double dr = (double)hop_sum<R, OCC>(basis[r], r, p.M, p.N + 2, rot[r], s_tab, s_delta, ybar, ky);
 #pragma unroll
         for (int i = 0; i < R; ++i) {
             const double yr = ybar[r * R + i];
@@ -357,14 +408,15 @@ template <int R>
 int launch_apply(rimu_dense* d, const DenseParams& p, const double* v, double* w, double* out) {
     const HopTables t = tables(d);
     const int64_t blocks = ceil_div(d->D, DT);
+    const bool occ = walk_occupied(d->M, d->N, R);
     if (out) {
         HIP_TRY(d->partials.alloc((size_t)blocks * R));
-        dense_apply_kernel<R, true><<<blocks, DT, table_bytes(t), d->stream>>>(d->basis.p, d->rot.p, d->D, p, t, v, w,
-                                                                               d->partials.p);
+        const auto product = occ ? dense_apply_kernel<R, true, true> : dense_apply_kernel<R, true, false>;
+        product<<<blocks, DT, table_bytes(t), d->stream>>>(d->basis.p, d->rot.p, d->D, p, t, v, w, d->partials.p);
         reduce_rows_kernel<<<R, RED_NT, 0, d->stream>>>(d->partials.p, blocks, out, 0);
     } else {
-        dense_apply_kernel<R, false><<<blocks, DT, table_bytes(t), d->stream>>>(d->basis.p, d->rot.p, d->D, p, t, v, w,
-                                                                                nullptr);
+        const auto product = occ ? dense_apply_kernel<R, false, true> : dense_apply_kernel<R, false, false>;
+        product<<<blocks, DT, table_bytes(t), d->stream>>>(d->basis.p, d->rot.p, d->D, p, t, v, w, nullptr);
     }
     HIP_TRY(hipGetLastError());
     return RIMU_OK;
@@ -390,8 +442,8 @@ int launch_pullback(rimu_dense* d, const DenseParams& p, const double* v, const 
     const HopTables t = tables(d);
     const int64_t blocks = ceil_div(d->D, DT);
     HIP_TRY(d->partials.alloc((size_t)blocks * 2 * R));
-    dense_pullback_kernel<R><<<blocks, DT, table_bytes(t), d->stream>>>(d->basis.p, d->rot.p, d->D, p, t, v, ybar,
-                                                                        vbar, d->partials.p);
+    const auto product = walk_occupied(d->M, d->N, R) ? dense_pullback_kernel<R, true> : dense_pullback_kernel<R, false>;
+    product<<<blocks, DT, table_bytes(t), d->stream>>>(d->basis.p, d->rot.p, d->D, p, t, v, ybar, vbar, d->partials.p);
     reduce_rows_kernel<<<2 * R, RED_NT, 0, d->stream>>>(d->partials.p, blocks, cot, accumulate);
     HIP_TRY(hipGetLastError());
     return RIMU_OK;
