@@ -533,14 +533,16 @@ __global__ __launch_bounds__(NT) void mix_keys_kernel(K* __restrict__ keys, int6
     keys[i] = forward ? mix_bits<K>(m, keys[i]) : unmix_bits<K>(m, keys[i]);
 }
 
-// Vectors of this many entries or more are reordered between address order and stored-key
-// order on the device, when the spawn buffers can hold them.  Reading out 50,000 two-word
-// entries takes 5.2 ms with the host's sort and 0.9 ms with the device's, 5e6 take 650 and 8 ms;
-// a few hundred entries cost the host less than the launches of a sort.
-constexpr int64_t DEVICE_REORDER_MIN = 1024;
+// Vectors are reordered between address order and stored-key order on the device from this many
+// entries on, when the spawn buffers can hold them.  The device's sort costs its launches, so
+// key bits; the host's its comparisons.  Upload in us, host : device, on new vectors each time:
+//   21 bits: 1500 entries 81 : 102, 3000 148 : 123      39 bits: 2000 108 : 136, 4000 207 : 169
+//   65 bits: 4000 209 : 243, 6000 313 : 283             127 bits: 6000 315 : 408, 9000 478 : 434
+// (download alike; 200,000 entries of 65 bits: 13.9 and 1.4 ms).
+constexpr int64_t reorder_min(int bits) { return 1024 + 56 * bits; }
 
 bool device_reorder(const rimu_engine* e, int64_t n) {
-    return e->mix.on && n >= DEVICE_REORDER_MIN && n <= e->max_spawns;
+    return e->mix.on && n >= reorder_min(e->hdev.B) && n <= e->max_spawns;
 }
 
 // n (key, value) pairs that fill() puts into spawn buffer 0: turn the keys into stored keys
