@@ -1177,6 +1177,7 @@ int rimu_vector_upload(rimu_engine* e, const uint64_t* keys, const void* vals, i
     std::vector<u128> stored;  // mix(address) of the kept entries
     const bool on_device = device_reorder(e, n);  // mix and sort on the device
     k.reserve((size_t)n * kw);
+    if (e->int_vals) vi.reserve((size_t)n); else vd.reserve((size_t)n);
     u128 prev = 0;
     for (int64_t i = 0; i < n; ++i) {
         const u128 key = key_at(i);
