@@ -245,6 +245,11 @@ int rimu_engine_set_sort_bits(rimu_engine* e, int32_t bits);
  * All give the same step results. */
 int rimu_engine_set_radix_mode(rimu_engine* e, int32_t mode);
 
+/* (No counterpart in the reference; for tests and tuning.)  How the last step's records were
+ * merged: the top `bits` key bits cut them into 2^bits buckets, each merged by a workgroup with
+ * `items` items per thread (512 threads); bits = -1, items = 0: along the merge path. */
+int rimu_engine_last_cut(rimu_engine* e, int32_t* bits, int32_t* items);
+
 /* (No counterpart in the reference; for tests.)  Every look-back wait of the step kernels
  * (the plan's attempt offsets, the radix scatters' digit offsets) is bounded by spin_limit
  * rounds (default 2^25).  A radix wait that gives up makes the engine repeat the step with

@@ -28,8 +28,8 @@ EXPORTS = (
     "rimu_engine_reserve", "rimu_vector_upload", "rimu_vector_length", "rimu_vector_download",
     "rimu_set_projector", "rimu_step", "rimu_engine_set_shift_update", "rimu_engine_get_shift",
     "rimu_engine_set_initiator", "rimu_overlaps",
-    "rimu_engine_set_sort_bits", "rimu_engine_set_radix_mode", "rimu_engine_set_lookback",
-    "rimu_engine_set_timing",
+    "rimu_engine_set_sort_bits", "rimu_engine_set_radix_mode", "rimu_engine_last_cut",
+    "rimu_engine_set_lookback", "rimu_engine_set_timing",
     "rimu_engine_kernel_times",
     "rimu_engine_last_traffic", "rimu_annihilate", "rimu_annihilate_noalloc", "rimu_hamiltonian_eval",
     "rimu_basis_size", "rimu_dense_create", "rimu_dense_destroy", "rimu_dense_dim",
@@ -113,6 +113,7 @@ def lib():
         L.rimu_engine_set_initiator.argtypes = [vp, i32, dbl]
         L.rimu_engine_set_sort_bits.argtypes = [vp, i32]
         L.rimu_engine_set_radix_mode.argtypes = [vp, i32]
+        L.rimu_engine_last_cut.argtypes = [vp, P(i32), P(i32)]
         L.rimu_engine_set_lookback.argtypes = [vp, ctypes.c_uint32, i32]
         L.rimu_overlaps.argtypes = [vp, vp, P(Operator), i32, P(dbl)]
         L.rimu_engine_set_timing.argtypes = [vp, i32]
@@ -334,6 +335,13 @@ class Engine:
         and bucket merge where eligible (default), 1 look-back scatters over every bit and the
         merge path, 0 per-pass counts and the merge path."""
         check(lib().rimu_engine_set_radix_mode(self._h, int(mode)))
+
+    def last_cut(self):
+        """(bits, items per thread) of the last step's bucket merge, (-1, 0) for the merge path
+        (``rimu_engine_last_cut``)."""
+        bits, items = ctypes.c_int32(0), ctypes.c_int32(0)
+        check(lib().rimu_engine_last_cut(self._h, ctypes.byref(bits), ctypes.byref(items)))
+        return bits.value, items.value
 
     def set_lookback(self, spin_limit: int, withhold_first: bool = False):
         """Bound of the look-back waits and the host-forced give-up test

@@ -126,6 +126,7 @@ struct rimu_engine {
     DevBuf<uint64_t> lb_status;     // look-back radix: status words [pass][tile][digit]
     uint32_t lb_epoch = 0;          // sort calls since lb_status was last cleared
     int bucket_cooldown = 0;        // steps left on the merge path after a bucket overflow
+    int cut_bits = -1, cut_items = 0;  // the last step's buckets (rimu_engine_last_cut)
     int bucket_roomy = 0;           // steps left that take the roomiest buckets, after an overflow
     bool spec_ok = false;           // the grids of the next step may be sized from W_prev, S_prev
     int64_t W_prev = 0, S_prev = 0; // spawn attempts and records of the last step
@@ -1029,6 +1030,7 @@ int step_impl(rimu_engine* e, int64_t step, double shift, double dtau, double bo
         int full = sorted;
         if (int rc = radix_sort<K, V>(e, S, nbits, kor ^ kand, sorted, &full)) return rc;
         sorted = full;
+        cut = BucketCut{};
         if (int rc = merge_path()) return rc;
         if (int rc = finish()) return rc;
         if (e->h_misc->flags & FLAG_LOOKBACK) return fail(RIMU_ERR_INTERNAL, "radix look-back did not complete");
@@ -1058,6 +1060,8 @@ int step_impl(rimu_engine* e, int64_t step, double shift, double dtau, double bo
         e->h_shift = s[NSTAT];
         e->h_pnorm = s[NSTAT + 1];
     }
+    e->cut_bits = cut.T;
+    e->cut_items = cut.T >= 0 ? cut.ipt : 0;
     // the counts that size the next step's grids
     e->W_prev = e->h_misc->W;
     e->S_prev = dense ? e->h_misc->W : e->h_misc->S;
@@ -1502,6 +1506,13 @@ int rimu_engine_set_radix_mode(rimu_engine* e, int32_t mode) {
     if (!e) return fail(RIMU_ERR_ARG, "engine is null");
     if (mode < 0 || mode > 2) return fail(RIMU_ERR_ARG, "radix mode must be 0, 1 or 2");
     e->radix_mode = mode;
+    return RIMU_OK;
+}
+
+int rimu_engine_last_cut(rimu_engine* e, int32_t* bits, int32_t* items) {
+    if (!e || !bits || !items) return fail(RIMU_ERR_ARG, "null argument");
+    *bits = e->cut_bits;
+    *items = e->cut_items;
     return RIMU_OK;
 }
 
