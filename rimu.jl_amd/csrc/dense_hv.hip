@@ -317,6 +317,17 @@ __global__ __launch_bounds__(DT) void rq_gradient_kernel(const double* __restric
 // Krylov space is exhausted goes on with zero vectors.
 __device__ inline double lanczos_scale(double n2, double floor2) { return n2 > floor2 ? 1.0 / sqrt(n2) : 0.0; }
 
+// The start vector over its norm, n2 = |x|^2, and one for the squared norm that the first update
+// takes: <x|Hx> of a vector as it was given may overflow or underflow where |x|^2 does not.
+__global__ __launch_bounds__(DT) void lanczos_start_kernel(double* __restrict__ x, int64_t D, int R,
+                                                           const double* __restrict__ n2, double* __restrict__ x2) {
+    const int64_t r = (int64_t)blockIdx.x * DT + threadIdx.x;
+    for (int i = 0; i < R; ++i) {
+        if (r < D) x[r * R + i] = n2[i] > 0.0 ? x[r * R + i] / sqrt(n2[i]) : 0.0;
+        if (r == 0) x2[i] = 1.0;
+    }
+}
+
 // One three-term Lanczos update per right-hand side.  The vectors are kept unnormalised with
 // their squared norms in device memory: v_j = x / sqrt(x2), v_{j-1} = y / sqrt(y2), and w = H x,
 // so H v_j = w / sqrt(x2) and alpha_j = <v_j|H v_j> = xw / x2.  Writes
@@ -811,17 +822,20 @@ int rimu_dense_ground_state(rimu_dense* d, const double* v0, int64_t max_iters, 
     const DenseParams pH = params(d, a_h, b_h);
     DevBuf<double>&x = d->x, &y = d->y, &w = d->z, &hist = d->hist;  // kept with the handle
     // hist: alpha [cap][R], then beta^2 [cap + 1][R] (beta^2[0] = 0 in the tridiagonal matrix, its
-    // place holds |v0|^2 = x2 of the first iteration on the device), then <x|Hx> [R]
+    // place holds one, x2 of the first iteration), then <x|Hx> [R], then |v0|^2 [R]
     auto run = [&]() -> int {
         HIP_TRY(x.alloc(n));
         HIP_TRY(y.alloc(n));
         HIP_TRY(w.alloc(n));
-        HIP_TRY(hist.alloc((size_t)(2 * cap + 2) * R));
+        HIP_TRY(hist.alloc((size_t)(2 * cap + 3) * R));
         double* alpha = hist.p;
         double* beta2 = hist.p + cap * R;
         double* xw = hist.p + (2 * cap + 1) * R;
+        double* n0 = xw + R;
         HIP_TRY(hipMemcpyAsync(x.p, v0, n * 8, hipMemcpyHostToDevice, d->stream));
-        if (int rc = dot(d, x.p, x.p, beta2)) return rc;
+        if (int rc = dot(d, x.p, x.p, n0)) return rc;
+        lanczos_start_kernel<<<ceil_div(d->D, DT), DT, 0, d->stream>>>(x.p, d->D, R, n0, beta2);
+        HIP_TRY(hipGetLastError());
         std::vector<double> h_a, h_b2, h_n0(R), last(R, INFINITY), cur(R);
         std::vector<int64_t> m_eff(R, -1);
         int64_t j = 0;
@@ -840,8 +854,8 @@ int rimu_dense_ground_state(rimu_dense* d, const double* v0, int64_t max_iters, 
             h_b2.resize((size_t)(m + 1) * R);
             HIP_TRY(hipMemcpyAsync(h_a.data(), alpha, (size_t)m * R * 8, hipMemcpyDeviceToHost, d->stream));
             HIP_TRY(hipMemcpyAsync(h_b2.data(), beta2, (size_t)(m + 1) * R * 8, hipMemcpyDeviceToHost, d->stream));
+            HIP_TRY(hipMemcpyAsync(h_n0.data(), n0, R * 8, hipMemcpyDeviceToHost, d->stream));
             HIP_TRY(hipStreamSynchronize(d->stream));
-            for (int i = 0; i < R; ++i) h_n0[i] = h_b2[i];
             bool done = true;
             std::vector<double> a(m), b2(m + 1);
             for (int i = 0; i < R; ++i) {
