@@ -1021,7 +1021,7 @@ __global__ __launch_bounds__(1 << RB) void radix_scatter_lb_kernel(const K* __re
     static_assert(TILE % NTS == 0 && TILE <= UINT16_MAX, "whole rounds per thread, 16-bit counts");
     __shared__ K s_k[TILE];
     __shared__ V s_v[TILE];
-    __shared__ uint16_t s_wcnt[NW][NDIG];
+    __shared__ alignas(4) uint16_t s_wcnt[NW][NDIG];
     __shared__ uint32_t s_start[NDIG];
     __shared__ uint32_t s_run[NDIG];
     __shared__ uint32_t s_goff[NDIG];
@@ -1041,7 +1041,8 @@ __global__ __launch_bounds__(1 << RB) void radix_scatter_lb_kernel(const K* __re
     const int64_t base = (int64_t)tile * TILE;
     const int64_t wbase = base + (int64_t)wid * IPT * WAVE;
 
-    for (int j = threadIdx.x; j < NW * NDIG / 2; j += NTS) ((uint32_t*)&s_wcnt[0][0])[j] = 0;
+    typedef uint32_t __attribute__((may_alias)) two_counts;
+    for (int j = threadIdx.x; j < NW * NDIG / 2; j += NTS) ((two_counts*)&s_wcnt[0][0])[j] = 0;
     __syncthreads();
 
     uint32_t digit_total = 0;  // of digit threadIdx.x over the whole list
