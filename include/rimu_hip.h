@@ -239,7 +239,7 @@ int rimu_engine_set_sort_bits(rimu_engine* e, int32_t bits);
  * bucket, each bucket's records and vector entries sorted and folded in LDS; a step that fits
  * one bucket is not sorted at all.  Keys of at most 20 bits are not mixed, so larger steps on
  * them go as 1, as does a step whose key bits below the buckets do not fit a bucket's words
- * or whose spread overfilled a bucket.  1: one histogram
+ * or whose spread overfilled a bucket of the largest kernel.  1: one histogram
  * pass for every digit and scatters that find their offsets by a look-back over the tiles
  * before them, then the merge path.  0: as 1 with counts per pass and a scan between passes.
  * All give the same step results. */

@@ -25,7 +25,8 @@
 // The result is that of the full sort and merge: same addresses, same fold order, same
 // draws; with an initiator rule each address folds three components instead of one, as on
 // the merge path.  A bucket larger than its LDS arrays raises FLAG_BUCKET_OVERFLOW and writes
-// nothing; the host then sorts on every bit and merges along the merge path.
+// nothing; the host then merges the same buckets in the largest shape, or, where that was the
+// one, sorts on every bit and merges along the merge path.
 //
 // Two-word keys have more bits below the bucket bits than a packed word holds: the word takes
 // the upper 52 of them and the key's low word is kept in LDS by item index.  Addresses are told
