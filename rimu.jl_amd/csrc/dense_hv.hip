@@ -821,22 +821,22 @@ int rimu_dense_ground_state(rimu_dense* d, const double* v0, int64_t max_iters, 
     for (int i = 0; i < R; ++i) { a_h[i] = 0; b_h[i] = 1; }
     const DenseParams pH = params(d, a_h, b_h);
     DevBuf<double>&x = d->x, &y = d->y, &w = d->z, &hist = d->hist;  // kept with the handle
-    // hist: alpha [cap][R], then beta^2 [cap + 1][R] (beta^2[0] = 0 in the tridiagonal matrix, its
-    // place holds one, x2 of the first iteration), then <x|Hx> [R], then |v0|^2 [R]
+    // hist: alpha [cap][R], then |v0|^2 [R], then beta^2 [cap + 1][R] (beta^2[0] = 0 in the
+    // tridiagonal matrix, its place holds one, x2 of the first iteration), then <x|Hx> [R]
     auto run = [&]() -> int {
         HIP_TRY(x.alloc(n));
         HIP_TRY(y.alloc(n));
         HIP_TRY(w.alloc(n));
         HIP_TRY(hist.alloc((size_t)(2 * cap + 3) * R));
         double* alpha = hist.p;
-        double* beta2 = hist.p + cap * R;
-        double* xw = hist.p + (2 * cap + 1) * R;
-        double* n0 = xw + R;
+        double* n0 = hist.p + cap * R;
+        double* beta2 = n0 + R;
+        double* xw = beta2 + (cap + 1) * R;
         HIP_TRY(hipMemcpyAsync(x.p, v0, n * 8, hipMemcpyHostToDevice, d->stream));
         if (int rc = dot(d, x.p, x.p, n0)) return rc;
         lanczos_start_kernel<<<ceil_div(d->D, DT), DT, 0, d->stream>>>(x.p, d->D, R, n0, beta2);
         HIP_TRY(hipGetLastError());
-        std::vector<double> h_a, h_b2, h_n0(R), last(R, INFINITY), cur(R);
+        std::vector<double> h_a, h_n, last(R, INFINITY), cur(R);
         std::vector<int64_t> m_eff(R, -1);
         int64_t j = 0;
         for (; j < cap; ++j) {
@@ -851,15 +851,15 @@ int rimu_dense_ground_state(rimu_dense* d, const double* v0, int64_t max_iters, 
             if ((j + 1) % CHECK != 0 && !last_iter) continue;
             const int64_t m = j + 1;
             h_a.resize((size_t)m * R);
-            h_b2.resize((size_t)(m + 1) * R);
+            h_n.resize((size_t)(m + 2) * R);  // |v0|^2, then beta^2
             HIP_TRY(hipMemcpyAsync(h_a.data(), alpha, (size_t)m * R * 8, hipMemcpyDeviceToHost, d->stream));
-            HIP_TRY(hipMemcpyAsync(h_b2.data(), beta2, (size_t)(m + 1) * R * 8, hipMemcpyDeviceToHost, d->stream));
-            HIP_TRY(hipMemcpyAsync(h_n0.data(), n0, R * 8, hipMemcpyDeviceToHost, d->stream));
+            HIP_TRY(hipMemcpyAsync(h_n.data(), n0, (size_t)(m + 2) * R * 8, hipMemcpyDeviceToHost, d->stream));
             HIP_TRY(hipStreamSynchronize(d->stream));
+            const double* h_b2 = h_n.data() + R;
             bool done = true;
             std::vector<double> a(m), b2(m + 1);
             for (int i = 0; i < R; ++i) {
-                if (!(h_n0[i] > 0)) return fail(RIMU_ERR_ARG, "start vector is zero");
+                if (!(h_n[i] > 0)) return fail(RIMU_ERR_ARG, "start vector is zero");
                 int64_t mi = m;
                 for (int64_t k = 1; k <= m; ++k) {
                     if (!(h_b2[k * R + i] > FLOOR2)) { mi = k; break; }  // exhausted after k vectors
