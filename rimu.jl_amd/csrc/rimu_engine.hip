@@ -128,7 +128,8 @@ struct rimu_engine {
     int bucket_cooldown = 0;        // steps left on the merge path after a bucket overflow
     int cut_bits = -1, cut_items = 0;  // the last step's buckets (rimu_engine_last_cut)
     int bucket_roomy = 0;           // steps left that take the roomiest buckets, after an overflow
-    int bucket_spread = 0;          // steps left that take twice the buckets, after one of the largest shape
+    int bucket_wary = 0;            // steps left with a lower mean of the buckets, after one overflowed the largest shape
+    double bucket_mean = 0;         // that mean
     bool spec_ok = false;           // the grids of the next step may be sized from W_prev, S_prev
     int64_t W_prev = 0, S_prev = 0; // spawn attempts and records of the last step
     uint32_t lb_spin_limit = LB_SPIN_LIMIT;  // bound of every look-back wait
@@ -590,9 +591,12 @@ constexpr int BK_COOLDOWN = 16;      // steps on the merge path after a bucket o
 // Steps with the largest shape after a bucket overflowed any: they cost 0.47 ms each more than the
 // smallest shape at 1.5e8 items, the overflow itself 2.3 ms.
 constexpr int BK_ROOMY = 256;
-// Steps with twice the buckets after one overflowed the largest shape.  An overflow costs about
-// nine steps' time (the full sort and 17 merge paths), twice the buckets up to 4 % of a step.
-constexpr int BK_SPREAD = 256;
+// An overflow of the largest shape costs five to nine steps' time (the full sort and 17 merge paths)
+// and comes again where an address collects records by the hundred (runs that grow, momentum
+// space).  For BK_WARY steps the buckets' mean then stays an eighth below the one that overflowed:
+// where that makes more buckets it costs 2 to 4 % of a step.
+constexpr int BK_WARY = 256;
+constexpr double BK_WARY_MIN = 1000;  // below it more buckets cost more than the merge path
 
 int max_bucket_ipt(int B) { return B > 64 ? BK_IPT_MAX_WIDE : BK_IPT_MAX; }
 
@@ -603,42 +607,42 @@ struct BucketCut {
     int ipt = 0;
 };
 
-// The largest mean of a shape: `sd` standard deviations of a bucket's count below its capacity.
-// Records come to addresses in groups, so counts vary more than independent ones: with 1e8 walkers
-// on 20 sites, 1 bucket of 3.5e7 exceeds 1536 items where the mean is 1144, and 1 of 5e5 exceeds
-// 2048 where it is 1640 -- a variance of 4.7 times the mean both times.
-constexpr double BK_VARIANCE = 4.7;
-double bucket_mean_max(int ipt, double sd) {
-    const double cap = (double)BK_NT * ipt, q = sd * sd * BK_VARIANCE / 4;
+// The largest mean of a shape: 4.57 standard deviations of a bucket's count below its capacity.
+// Records come to addresses in groups, so counts vary more than independent ones, a run that grows
+// more than one that has spread out.  With 1e8 walkers on 20 sites 1 bucket of 5e5 exceeded 2048
+// items where the mean was 1640, and at another time 1 of 3.5e7 1536 where it was 1144: a variance
+// of 4.7 times the mean, one overflow in 6 steps of 2^16 full buckets; later on 150 steps whose mean
+// was 2030 to 2100 met none.  So the line stays where more buckets would cost 12 % of every step
+// (2^17 instead of 2^16, sorted in nine-bit digits: 6.95 and 6.2 ms at 1.33e8 items) and a run
+// that does overflow moves it (BK_ROOMY, BK_WARY).
+constexpr double BK_VARIANCE = 4.7, BK_SD = 4.57;
+double bucket_mean_max(int ipt) {
+    const double cap = (double)BK_NT * ipt, q = BK_SD * BK_SD * BK_VARIANCE / 4;
     const double x = std::sqrt(cap + q) - std::sqrt(q);
     return x * x;
 }
-// Overflows of a small shape cost a second merge (2.3 of 7.2 ms at 1e8 walkers), those of the
-// largest the full sort and the merge path: 5.4 deviations leave one overflow in 230 steps of 2^17
-// buckets (in 3700 of 2^13), which costs about as much as smaller buckets would below that mean.
-constexpr double BK_SD = 4.57, BK_SD_LARGEST = 5.4;
 
 // S records and L entries: the fewest buckets, in the smallest shape (at least `min_ipt` items
-// per thread) that holds them; with `spread`, twice as many buckets.  A bucket costs its workgroup
-// seven microseconds or more whatever it holds, so more and smaller buckets lose: 1.6e7 items in 2^13, 2^14, 2^15, 2^16
-// buckets take 158, 183, 226, 412 us (the last two with two items per thread and four
-// workgroups on a CU, a shape no step takes now); 1.5e8 items in 2^17 buckets take 2.75 ms with
-// three items per thread (three workgroups on a CU) and 3.22 ms with five (two).
+// per thread) that holds them, several with no more than `mean` items on average (if not zero).
+// A bucket costs its workgroup seven microseconds or more whatever it holds, so more and smaller
+// buckets lose: 1.6e7 items in 2^13, 2^14, 2^15, 2^16 buckets take 158, 183, 226, 412 us (the last
+// two with two items per thread and four workgroups on a CU, a shape no step takes now); 1.5e8
+// items in 2^17 buckets take 2.75 ms with three items per thread (three workgroups on a CU) and
+// 3.22 ms with five (two).
 // A step of up to 2105 items (two-word keys 1645) is one bucket, sorted without a radix pass,
 // whether its keys are mixed or not (1000 integer walkers on 19-bit keys: 99 us a step with three
-// radix passes and the merge path, 66 us so); its count only varies from step to step.  More
-// buckets need mixed keys, whose top bits are spread evenly: up to 2032 items (1581) on average.
-BucketCut bucket_cut(int64_t S, int64_t L, int B, bool mixed, int min_ipt, bool spread) {
+// radix passes and the merge path, 66 us so); more buckets need mixed keys, whose top bits are
+// spread evenly.
+BucketCut bucket_cut(int64_t S, int64_t L, int B, bool mixed, int min_ipt, double mean) {
     const double items = (double)S + (double)L;
     const int max_ipt = max_bucket_ipt(B), max_bits = std::min(B, 24);
     const int max_low = B > 64 ? BK_MAX_LOWBITS_WIDE : BK_MAX_LOWBITS;
     BucketCut cut;
     cut.T = B > 64 ? std::max(B - max_low, 0) : 0;  // at most 2^12 buckets more than the items need
-    if (items > bucket_mean_max(max_ipt, BK_SD)) cut.T = std::max(cut.T, 1);
-    while (cut.T > 0 && cut.T < max_bits && std::ldexp(items, -cut.T) > bucket_mean_max(max_ipt, BK_SD_LARGEST)) ++cut.T;
-    if (spread && cut.T > 0) cut.T = std::min(cut.T + 1, max_bits);
+    const double most = bucket_mean_max(max_ipt);
+    while (cut.T < max_bits && std::ldexp(items, -cut.T) > (cut.T > 0 && mean > 0 ? std::min(mean, most) : most)) ++cut.T;
     cut.ipt = std::min(min_ipt, max_ipt);
-    while (cut.ipt < max_ipt && std::ldexp(items, -cut.T) > bucket_mean_max(cut.ipt, BK_SD)) ++cut.ipt;
+    while (cut.ipt < max_ipt && std::ldexp(items, -cut.T) > bucket_mean_max(cut.ipt)) ++cut.ipt;
     if (B - cut.T > max_low || (cut.T > 0 && !mixed)) cut.T = -1;
     return cut;
 }
@@ -779,7 +783,7 @@ int step_impl(rimu_engine* e, int64_t step, double shift, double dtau, double bo
     // the path the counts of the last step choose; sorts with a host check stay synchronous
     auto cut_for = [&](int64_t records) {
         return e->style.kind == 2 ? exact_cut(records, L, nbits, e->mix.on)
-                                   : bucket_cut(records, L, nbits, e->mix.on, min_ipt, e->bucket_spread > 0);
+                                   : bucket_cut(records, L, nbits, e->mix.on, min_ipt, e->bucket_wary > 0 ? e->bucket_mean : 0.0);
     };
     if (spec && bucket_ok) cut = cut_for(e->S_prev);
     const int64_t W_cap = spec ? e->W_prev + e->W_prev / 4 + 16 * spawn_tile(SPAWN_ITEMS) : 0;
@@ -922,7 +926,7 @@ int step_impl(rimu_engine* e, int64_t step, double shift, double dtau, double bo
         --e->bucket_cooldown;
     } else {
         if (e->bucket_roomy > 0) --e->bucket_roomy;
-        if (e->bucket_spread > 0) --e->bucket_spread;
+        if (e->bucket_wary > 0) --e->bucket_wary;
     }
     const int64_t* merge_S_dev = S_dev;  // the merge path after the fallback sort reads S from the host
     auto merge_path = [&]() -> int {
@@ -1042,8 +1046,6 @@ int step_impl(rimu_engine* e, int64_t step, double shift, double dtau, double bo
         // sort the bucketed records on every bit (stable passes keep their list order within
         // an address) and merge along the merge path
         e->bucket_cooldown = BK_COOLDOWN;
-        e->bucket_roomy = BK_ROOMY;  // uneven counts: the roomiest buckets, and twice as many, for a while
-        e->bucket_spread = BK_SPREAD;
         e->timer.begin("bucket_fallback", e->stream, &ev);
         e->timer.end(e->stream);
         HIP_TRY(hipMemsetAsync(&dm->flags, 0, sizeof(int), e->stream));
@@ -1051,6 +1053,9 @@ int step_impl(rimu_engine* e, int64_t step, double shift, double dtau, double bo
             S = dense ? e->h_misc->W : e->h_misc->S;
             merge_S_dev = nullptr;
         }
+        e->bucket_roomy = 0;  // the shape that a lower mean asks for
+        e->bucket_wary = BK_WARY;
+        e->bucket_mean = std::max(std::ldexp((double)S + (double)L, -cut.T) * 7 / 8, BK_WARY_MIN);
         int full = sorted;
         if (int rc = radix_sort<K, V>(e, S, nbits, kor ^ kand, sorted, &full)) return rc;
         sorted = full;

@@ -1,6 +1,5 @@
 """Steps whose buckets vary more in size than the rule expects: after one that overfilled the
-largest shape, more and smaller buckets hold the same records; and where the largest shape's
-mean lies."""
+largest shape, smaller buckets hold the same records; and where the largest shape's mean lies."""
 import numpy as np
 import pytest
 
@@ -42,13 +41,13 @@ def test_more_buckets_after_an_overflow(gpu):
         assert x[:2] == y[:2]
         assert np.array_equal(x[2], y[2]) and np.array_equal(x[3].view(np.uint64), y[3].view(np.uint64))
     assert cuts[:17] == [(-1, 0)] * 17          # the overflow, and 16 steps along the merge path
-    assert cuts[17:] == [(6, 5)] * 23           # one bit more, in the roomiest shape
+    assert cuts[17:] == [(6, 5)] * 23           # a mean of 999 instead of 1999; the smallest shape was overfilled once
     assert overflows == 1
 
 
-# 39 bits: buckets of 2032 on average are the largest that several may have (5.4 deviations of a
-# bucket's count below the 2560 items it holds); 99 bits: 1581 of 2048
-@pytest.mark.parametrize("M,items,cut", [(20, 2028 * 16, (4, 5)), (20, 2036 * 16, (5, 3)), (20, 2100, (0, 5)),
-                                         (50, 1577 * 4, (2, 4)), (50, 1585 * 4, (3, 3)), (50, 1640, (0, 4))])
+# 39 bits: buckets of 2105 on average are the largest, 4.57 deviations of their count below the 2560
+# items they hold; 99 bits: 1645 of 2048
+@pytest.mark.parametrize("M,items,cut", [(20, 2101 * 16, (4, 5)), (20, 2109 * 16, (5, 3)),
+                                         (50, 1642 * 4, (2, 4)), (50, 1649 * 4, (3, 3))])
 def test_largest_mean(gpu, M, items, cut):
     assert _first_cut(gpu, M, M, items) == cut
