@@ -588,9 +588,9 @@ int reorder_on_device(rimu_engine* e, int64_t n, int forward, int* result, Fill&
 constexpr int BK_MAX_LOWBITS = 48, BK_MAX_LOWBITS_WIDE = 116;
 constexpr int BK_IPT_MAX_WIDE = 4;   // two-word buckets of five items per thread leave one workgroup a CU
 constexpr int BK_COOLDOWN = 16;      // steps on the merge path after a bucket overflowed the largest shape
-// Steps with the largest shape after a bucket overflowed any: they cost 0.47 ms each more than the
-// smallest shape at 1.5e8 items, the overflow itself 2.3 ms.
-constexpr int BK_ROOMY = 256;
+// Steps with the largest shape after a bucket overflowed any: the second merge costs as much as
+// five of them do (2.3 ms and 0.47 ms a step at 1.5e8 items, 0.16 and 0.04 ms at 1.6e7).
+constexpr int BK_ROOMY = 8;
 // An overflow of the largest shape costs five to nine steps' time (the full sort and 17 merge paths)
 // and comes again where an address collects records by the hundred (runs that grow, momentum
 // space).  For BK_WARY steps the buckets' mean then stays an eighth below the one that overflowed:
