@@ -128,6 +128,7 @@ struct rimu_engine {
     int bucket_cooldown = 0;        // steps left on the merge path after a bucket overflow
     int cut_bits = -1, cut_items = 0;  // the last step's buckets (rimu_engine_last_cut)
     int bucket_roomy = 0;           // steps left that take the roomiest buckets, after an overflow
+    int roomy_len = 0, roomy_since = 0;  // how many those were, and steps since then
     int bucket_wary = 0;            // steps left with a lower mean of the buckets, after one overflowed the largest shape
     double bucket_mean = 0;         // that mean
     bool spec_ok = false;           // the grids of the next step may be sized from W_prev, S_prev
@@ -588,9 +589,12 @@ int reorder_on_device(rimu_engine* e, int64_t n, int forward, int* result, Fill&
 constexpr int BK_MAX_LOWBITS = 48, BK_MAX_LOWBITS_WIDE = 116;
 constexpr int BK_IPT_MAX_WIDE = 4;   // two-word buckets of five items per thread leave one workgroup a CU
 constexpr int BK_COOLDOWN = 16;      // steps on the merge path after a bucket overflowed the largest shape
-// Steps with the largest shape after a bucket overflowed any: the second merge costs as much as
-// five of them do (2.3 ms and 0.47 ms a step at 1.5e8 items, 0.16 and 0.04 ms at 1.6e7).
-constexpr int BK_ROOMY = 8;
+// Steps with the largest shape after a bucket overflowed a smaller one.  The second merge costs as
+// much as five of them where the smallest shape does (2.3 ms and 0.47 ms a step at 1.5e8 items), as
+// much as eighteen where the middle one does (2.3 and 0.13 at 1.07e8): sixteen, and four times as
+// many each time that the next overflow comes soon after them.
+constexpr int BK_ROOMY = 16, BK_ROOMY_MAX = 256;
+
 // An overflow of the largest shape costs five to nine steps' time (the full sort and 17 merge paths)
 // and comes again where an address collects records by the hundred (runs that grow, momentum
 // space).  For BK_WARY steps the buckets' mean then stays an eighth below the one that overflowed:
@@ -926,6 +930,7 @@ int step_impl(rimu_engine* e, int64_t step, double shift, double dtau, double bo
         --e->bucket_cooldown;
     } else {
         if (e->bucket_roomy > 0) --e->bucket_roomy;
+        else if (e->roomy_since < 4 * BK_ROOMY_MAX) ++e->roomy_since;
         if (e->bucket_wary > 0) --e->bucket_wary;
     }
     const int64_t* merge_S_dev = S_dev;  // the merge path after the fallback sort reads S from the host
@@ -1034,7 +1039,9 @@ int step_impl(rimu_engine* e, int64_t step, double shift, double dtau, double bo
     if (e->h_misc->flags & FLAG_LOOKBACK) return fail(RIMU_ERR_INTERNAL, "radix look-back did not complete");
     if ((e->h_misc->flags & FLAG_BUCKET_OVERFLOW) && cut.ipt < max_bucket_ipt(nbits)) {
         // the same buckets fit the largest shape more often than not: merge them again
-        e->bucket_roomy = BK_ROOMY;
+        const bool again = e->roomy_len > 0 && e->roomy_since < 4 * e->roomy_len;
+        e->bucket_roomy = e->roomy_len = again ? std::min(4 * e->roomy_len, BK_ROOMY_MAX) : BK_ROOMY;
+        e->roomy_since = 0;
         e->timer.begin("bucket_retry", e->stream, &ev);
         e->timer.end(e->stream);
         HIP_TRY(hipMemsetAsync(&dm->flags, 0, sizeof(int), e->stream));

@@ -10,6 +10,8 @@ pytestmark = pytest.mark.gpu
 
 
 def test_shape_after_an_overflow(gpu):
+    """Sixteen steps after the first overflow; 64 after one that comes soon after those; sixteen
+    after one that does not."""
     M = N = 20
     rng = np.random.default_rng(4)
     small, _ = _chain_vector(M, N, 250, rng)
@@ -17,16 +19,35 @@ def test_shape_after_an_overflow(gpu):
     h = device_model(gpu, "real", M, N, 0.0, 1.0)
     e = gpu._native.Engine(h.descriptor(), gpu.IsDynamicSemistochastic().descriptor(), 5, 1 << 18, 1 << 18)
     e.set_timing(True)
-    e.upload(small, np.full(250, 1.5))              # the second step has five times the first's attempts
-    e.step(1, 4000.0, 1e-3)
-    e.step(2, 0.0, 1e-3)
-    assert set(e.kernel_times()) & {"bucket_retry", "bucket_fallback"} == {"bucket_retry"}
-    assert e.last_cut() == (0, 5)
-    cuts = []
-    for s in range(3, 16):
-        e.upload(keys, vals)
-        e.step(s, 0.0, 1e-3)
-        cuts.append(e.last_cut()[1])
+    step = 0
+
+    def overflow():
+        nonlocal step
+        e.upload(small, np.full(250, 1.2))          # two small steps, the second sized by the first
+        e.step(step + 1, 0.0, 1e-3)
+        e.upload(small, np.full(250, 1.2))
+        e.step(step + 2, 0.0, 1e-3)
+        e.upload(small, np.full(250, 6.5))          # five times their attempts
+        e.step(step + 3, 0.0, 1e-3)
+        step += 3
+        return e.kernel_times().get("bucket_retry", (0, 0))[1], e.last_cut()
+
+    def shapes(n):
+        nonlocal step
+        out = []
+        for _ in range(n):
+            step += 1
+            e.upload(keys, vals)
+            e.step(step, 0.0, 1e-3)
+            out.append(e.last_cut()[1])
+        return out
+
+    assert overflow() == (1, (0, 5))
+    assert shapes(21) == [5] * 16 + [3] * 5
+    assert overflow() == (2, (0, 5))
+    assert shapes(69) == [5] * 64 + [3] * 5
+    assert shapes(256) == [3] * 256
+    assert overflow() == (3, (0, 5))
+    assert shapes(21) == [5] * 16 + [3] * 5
+    assert "bucket_fallback" not in e.kernel_times()
     e.close()
-    print(cuts, flush=True)
-    assert cuts[:8] == [5] * 8 and cuts[8:] == [3] * 5
