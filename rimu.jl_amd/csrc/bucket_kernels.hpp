@@ -403,8 +403,10 @@ __global__ __launch_bounds__(BK_NT, 2 * BkShape<IPT>::wgs(sizeof(K))) void bucke
                     }
                 }
             }
-            const uint64_t wprev = p0 > 0 && p0 < n ? sm.sk[p0 - 1] : NOKEY;
-            const uint64_t kprev = WIDE || p0 == 0 || p0 >= n ? wprev : wprev >> BK_IDX_BITS;
+            // (read and shifted in one select: with the shift in another the kernel of five items needs
+            // more than its 128 registers, spills one of the values it has just asked for and waits
+            // for it: 2.30 ms at 1.07e8 items, 2.25 so)
+            const uint64_t kprev = p0 > 0 && p0 < n ? (WIDE ? sm.sk[p0 - 1] : sm.sk[p0 - 1] >> BK_IDX_BITS) : NOKEY;
             // whether position p0 + k holds another address than the one before it
             auto differ = [&](int k, uint64_t x, uint64_t before) {
                 if constexpr (WIDE) return p0 + k == 0 || ((x ^ before) >> BK_IDX_BITS) != 0;
