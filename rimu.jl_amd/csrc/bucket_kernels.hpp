@@ -292,22 +292,22 @@ __global__ __launch_bounds__(BK_NT, 2 * BkShape<IPT>::wgs(sizeof(K))) void bucke
 
         const int n = na + nb;
         const bool fits = n <= BK_CAP;  // uniform over the workgroup
-        // the key of a survivor: one-word keys from its bits below the bucket bits, two-word keys
-        // from its packed word (the low word by the item index in it)
+        // the key of a survivor from okey: one-word keys lie there whole, two-word keys as their packed
+        // word (the low word by the item index in it)
         auto key_of = [&](uint64_t x) -> K {
-            const K top = shlA((K)b, lowbits);
             if constexpr (WIDE) {
-                const K k = top | shlA((K)(x >> BK_IDX_BITS), drop);
+                const K k = shlA((K)b, lowbits) | shlA((K)(x >> BK_IDX_BITS), drop);
                 return (K)(k >> 64) << 64 | (K)sm.klo[(int)(x & IDX_MASK)];
             } else {
-                return top | x;
+                return x;
             }
         };
-        uint64_t okey[BK_IPT];  // key_of's argument
+        uint64_t okey[BK_IPT];
         V oval[BK_IPT];
         uint32_t cvalid = 0;
         int n_before = 0;  // len_before: folded values that are not zero
         if (fits) {
+            const uint64_t bucket_key = WIDE || lowbits >= 64 ? 0ull : (uint64_t)b << lowbits;
             // ---- 1. pack (key bits below the bucket bits, item index), values by item
             // index, drop every word into its sub-bucket (arrival order is arbitrary) ---------
             uint64_t w[BK_IPT];
@@ -391,7 +391,7 @@ __global__ __launch_bounds__(BK_NT, 2 * BkShape<IPT>::wgs(sizeof(K))) void bucke
             for (int k = 0; k <= NWIN; ++k) {
                 const int p = p0 + k;
                 const uint64_t wd = p < n ? sm.sk[p] : NOKEY;
-                kk[k] = WIDE || p >= n ? wd : wd >> BK_IDX_BITS;
+                kk[k] = WIDE ? wd : p < n ? wd >> BK_IDX_BITS : NOKEY;
                 if (k < NWIN) {
                     const int idx = (int)(wd & IDX_MASK);
                     vv[k] = p < n ? sm.vin[idx] : (V)0;
@@ -405,7 +405,7 @@ __global__ __launch_bounds__(BK_NT, 2 * BkShape<IPT>::wgs(sizeof(K))) void bucke
             }
             // (read and shifted in one select: with the shift in another the kernel of five items needs
             // more than its 128 registers, spills one of the values it has just asked for and waits
-            // for it: 2.30 ms at 1.07e8 items, 2.25 so)
+            // for it: 2.30 ms at 1.07e8 items against 2.25)
             const uint64_t kprev = p0 > 0 && p0 < n ? (WIDE ? sm.sk[p0 - 1] : sm.sk[p0 - 1] >> BK_IDX_BITS) : NOKEY;
             // whether position p0 + k holds another address than the one before it
             auto differ = [&](int k, uint64_t x, uint64_t before) {
@@ -435,7 +435,7 @@ __global__ __launch_bounds__(BK_NT, 2 * BkShape<IPT>::wgs(sizeof(K))) void bucke
                     const bool end = valid && ((WIDE && p0 + k + 1 >= n) || differ(k + 1, kk[k + 1], kk[k]));
                     const int slot_k = k < BK_IPT - 1 ? k : BK_IPT - 1;
                     if (own && end) {
-                        okey[slot_k] = kk[k];
+                        okey[slot_k] = bucket_key | kk[k];
                         oval[slot_k] = acc;
                         if (acc != (V)0) cvalid |= 1u << slot_k;
                         own = false;
@@ -448,7 +448,7 @@ __global__ __launch_bounds__(BK_NT, 2 * BkShape<IPT>::wgs(sizeof(K))) void bucke
                         if ((wd >> BK_IDX_BITS) != (WIDE ? key >> BK_IDX_BITS : key)) break;
                         acc = acc + sm.vin[(int)(wd & IDX_MASK)];
                     }
-                    okey[BK_IPT - 1] = key;
+                    okey[BK_IPT - 1] = bucket_key | key;
                     oval[BK_IPT - 1] = acc;
                     if (acc != (V)0) cvalid |= 1u << (BK_IPT - 1);
                 }
@@ -472,7 +472,7 @@ __global__ __launch_bounds__(BK_NT, 2 * BkShape<IPT>::wgs(sizeof(K))) void bucke
                         cpres |= 1u << slot_k;
                         const V val = initiator_value<V>(a, cs, cu, ci);
                         if (val != (V)0 || keep_zero) {
-                            okey[slot_k] = key;
+                            okey[slot_k] = bucket_key | key;
                             oval[slot_k] = val;
                             cvalid |= 1u << slot_k;
                         }
