@@ -591,9 +591,9 @@ constexpr int BK_IPT_MAX_WIDE = 4;   // two-word buckets of five items per threa
 constexpr int BK_COOLDOWN = 16;      // steps on the merge path after a bucket overflowed the largest shape
 // Steps with the largest shape after a bucket overflowed a smaller one.  The second merge costs as
 // much as five of them where the smallest shape does (2.3 ms and 0.47 ms a step at 1.5e8 items), as
-// much as eighteen where the middle one does (2.3 and 0.13 at 1.07e8): sixteen, and four times as
-// many each time that the next overflow comes soon after them.
-constexpr int BK_ROOMY = 16, BK_ROOMY_MAX = 256;
+// much as forty where the middle one does (2.2 and 0.05 at 1.07e8): sixteen and 64, and four times
+// as many as last time when the next overflow comes soon after them.
+constexpr int BK_ROOMY = 16, BK_ROOMY_MIDDLE = 64, BK_ROOMY_MAX = 256;
 
 // An overflow of the largest shape costs five to nine steps' time (the full sort and 17 merge paths)
 // and comes again where an address collects records by the hundred (runs that grow, momentum
@@ -1040,7 +1040,8 @@ int step_impl(rimu_engine* e, int64_t step, double shift, double dtau, double bo
     if ((e->h_misc->flags & FLAG_BUCKET_OVERFLOW) && cut.ipt < max_bucket_ipt(nbits)) {
         // the same buckets fit the largest shape more often than not: merge them again
         const bool again = e->roomy_len > 0 && e->roomy_since < 4 * e->roomy_len;
-        e->bucket_roomy = e->roomy_len = again ? std::min(4 * e->roomy_len, BK_ROOMY_MAX) : BK_ROOMY;
+        const int steps = std::max(cut.ipt > BK_IPT_MIN ? BK_ROOMY_MIDDLE : BK_ROOMY, again ? 4 * e->roomy_len : 0);
+        e->bucket_roomy = e->roomy_len = std::min(steps, BK_ROOMY_MAX);
         e->roomy_since = 0;
         e->timer.begin("bucket_retry", e->stream, &ev);
         e->timer.end(e->stream);
